@@ -33,7 +33,6 @@ namespace tdx {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 struct KArgs {
     const void *X;
@@ -379,46 +378,6 @@ __global__ __launch_bounds__(256, (ST != 0 && NB >= 3) ? 1 : 2) void k_mttkrp(KA
     }
 }
 
-// Generic fallback for shapes the register-tile kernel does not cover (odd leading
-// extent, rank > 64): one workgroup per (output row, split), one lane per column.
-template <int ST>
-__global__ __launch_bounds__(64) void k_mttkrp_generic(KArgs a, long kelems) {
-    if (a.skip && *a.skip) return;
-    const long row = blockIdx.x % a.In;
-    const long split = blockIdx.x / a.In;
-    const long k0 = split * a.kper, k1 = min(k0 + a.kper, kelems);
-    const int Rp = a.Rp;
-    for (int c0 = 0; c0 < Rp; c0 += 64) {
-        const int r = c0 + threadIdx.x;
-        double accd = 0.0;
-        for (long e = k0; e < k1; ++e) {
-            long rem = e, off = row * a.stride[a.mode];
-            float kr = 1.0f;
-            for (int m = 0; m < a.order; ++m) {
-                if (m == a.mode) continue;
-                const long idx = rem % a.dims[m];
-                rem /= a.dims[m];
-                off += idx * a.stride[m];
-                if (r < Rp) kr *= a.panel[m][((idx >> 3) * Rp + r) * 8 + (idx & 7)];
-            }
-            float x;
-            if constexpr (ST == 0) x = reinterpret_cast<const float *>(a.X)[off];
-            else if constexpr (ST == 1) x = __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(a.X)[off] << 16);
-            else {
-                const uint8_t q = reinterpret_cast<const uint8_t *>(a.X)[off];
-                f32x2 d = __builtin_amdgcn_cvt_pk_f32_fp8((int)q, false);
-                x = d.x;
-            }
-            accd += (double)x * (double)kr;
-        }
-        if (r < Rp) {
-            float v = (float)accd;
-            if (ST == 2 && a.mode == 0) v *= a.row_scale[row];
-            a.partial[(split * a.rows_pad + row) * Rp + r] = v;
-        }
-    }
-}
-
 __global__ void k_pack_panel(const float *__restrict__ U, long I, long R, int Rp, const float *__restrict__ scale,
                              float *__restrict__ panel, long Ipad) {
     const long n = Ipad * Rp;
@@ -550,19 +509,7 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
         if (p.ksteps_per_split > kmax) p.ksteps_per_split = kmax;
         p.nsplit = (int)ceil_div(p.ksteps, p.ksteps_per_split);
     } else {
-        long kelems = 1;
-        for (int m = 0; m < order; ++m)
-            if (m != mode) kelems *= dims[m];
-        p.rows_per_wg = 1;
-        p.rowtiles = (int)In;
-        p.rows_pad = In;
-        p.ksteps = kelems;
-        long want = ceil_div(4096, In);
-        long maxs = ceil_div(kelems, 64);
-        long ns = want < maxs ? want : maxs;
-        if (ns < 1) ns = 1;
-        p.ksteps_per_split = ceil_div(kelems, ns);
-        p.nsplit = (int)ceil_div(kelems, p.ksteps_per_split);
+        mttkrp_any_plan(p);
     }
     return TDX_OK;
 }
@@ -627,11 +574,7 @@ int mttkrp_launch(const MttkrpPlan &p, const void *X, const float *const *panels
         else if (stt == 1) { if (ca) launch_fast<1, true>(p, a, s); else launch_fast<1, false>(p, a, s); }
         else { if (ca) launch_fast<2, true>(p, a, s); else launch_fast<2, false>(p, a, s); }
     } else {
-        a.FB = 1;
-        const int grid = (int)(a.In * p.nsplit);
-        if (stt == 0) k_mttkrp_generic<0><<<grid, 64, 0, s>>>(a, p.ksteps);
-        else if (stt == 1) k_mttkrp_generic<1><<<grid, 64, 0, s>>>(a, p.ksteps);
-        else k_mttkrp_generic<2><<<grid, 64, 0, s>>>(a, p.ksteps);
+        return mttkrp_any_launch(p, X, panels, row_scale, partial, s, skip);
     }
     TDX_LAUNCH_CHECK();
     return TDX_OK;

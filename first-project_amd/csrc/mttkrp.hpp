@@ -49,6 +49,12 @@ bool mttkrp_lds_covers(int order, int mode, long rank, long In, int dtype);
 int mttkrp_lds_launch(const MttkrpPlan &p, const void *X, const float *const *panels, const float *row_scale,
                       float *partial, hipStream_t s, const int *skip);
 
+// the kernel for the remaining shapes and alignments (mttkrp_any.hip): completes a plan whose
+// order, extents, mode, storage and rank are set; partial rows are exactly the output rows
+void mttkrp_any_plan(MttkrpPlan &p);
+int mttkrp_any_launch(const MttkrpPlan &p, const void *X, const float *const *panels, const float *row_scale,
+                      float *partial, hipStream_t s, const int *skip);
+
 // the shared pass of an order-3 CP-ALS sweep (dtree.hip): T = X x_0 A^T with the mode-1
 // partials in the same pass over X, then the mode-2 partials from T
 struct DtreePlan {
