@@ -857,10 +857,9 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
 static int refresh_factors(CpPlan &P, const Storage &S, hipStream_t s) {
     // partials of a previous storage phase are never reused across a storage change
     if (P.ls_mode) k_set_int<<<1, 1, 0, s>>>(&P.ls->skip, 0);
+    int st = pack_panels(P.order, P.dims, -1, P.U, P.R, P.Rp, S.dtype == TDX_FP8_E4M3 ? S.scales : nullptr, P.panel, s);
+    if (st) return st;
     for (int m = 0; m < P.order; ++m) {
-        const float *sc = (S.dtype == TDX_FP8_E4M3 && m == 0) ? S.scales : nullptr;
-        int st = pack_panel(P.U[m], P.dims[m], P.R, P.Rp, sc, P.panel[m], s);
-        if (st) return st;
         st = gram_of(P.U[m], P.dims[m], (int)P.R, P.gram_part, P.G[m], s);
         if (st) return st;
     }

@@ -590,11 +590,10 @@ int tdx_mttkrp_dtree(const void *X, int dtype, const float *scales, const long *
         void *ws = nullptr;
         st = workspace(WS_PANEL0 + m, sizeof(float) * panel_floats(dims[m], d.Rp), &ws);
         if (st) return st;
-        st = pack_panel(factors[m], dims[m], rank, d.Rp, (dtype == TDX_FP8_E4M3 && m == 0) ? scales : nullptr,
-                        (float *)ws, s);
-        if (st) return record(st);
         panel[m] = (float *)ws;
     }
+    st = pack_panels(2, dims, -1, factors, rank, d.Rp, dtype == TDX_FP8_E4M3 ? scales : nullptr, panel, s);
+    if (st) return record(st);
     void *T = nullptr, *part = nullptr;
     st = workspace(WS_MISC0, d.t_bytes(), &T);
     if (st) return st;
@@ -640,11 +639,10 @@ int tdx_bench_mttkrp_dtree(const void *X, int dtype, const float *scales, const 
         void *ws = nullptr;
         st = workspace(WS_PANEL0 + m, sizeof(float) * panel_floats(dims[m], d.Rp), &ws);
         if (st) return st;
-        st = pack_panel(factors[m], dims[m], rank, d.Rp, (dtype == TDX_FP8_E4M3 && m == 0) ? scales : nullptr,
-                        (float *)ws, s);
-        if (st) return record(st);
         panel[m] = (float *)ws;
     }
+    st = pack_panels(2, dims, -1, factors, rank, d.Rp, dtype == TDX_FP8_E4M3 ? scales : nullptr, panel, s);
+    if (st) return record(st);
     void *T = nullptr, *part = nullptr;
     st = workspace(WS_MISC0, d.t_bytes(), &T);
     if (st) return st;

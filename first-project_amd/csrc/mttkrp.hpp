@@ -94,8 +94,10 @@ int dtree_m2_vinv_launch(const DtreePlan &d, const uint16_t *T, const float *pan
                          const double *G0, const double *G1, int R, double *Vinv, int *status, double *fb_ws,
                          hipStream_t s);
 
-// panel packing (optionally scaling row i by scale[i])
-int pack_panel(const float *U, long I, long R, int Rp, const float *scale, float *panel, hipStream_t s);
+// packs the panels of every factor but `skip` (-1: all) in one launch; scale0 (or null): row i
+// of the mode-0 factor is multiplied by scale0[i]
+int pack_panels(int order, const long *dims, int skip, const float *const *U, long R, int Rp, const float *scale0,
+                float *const *panels, hipStream_t s);
 
 // sums the split partials into out (I_mode x rank, column-major FP32)
 int mttkrp_reduce(const MttkrpPlan &p, const float *partial, float *out, hipStream_t s);
