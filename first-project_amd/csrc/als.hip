@@ -68,7 +68,9 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
 }
 
 // U_n rows = M V^{-1} for kSolveRows rows per workgroup (256 threads), M summed here from
-// the MTTKRP's split partials in FP64 in split order (the order of k_split_sum).  Also
+// the MTTKRP's split partials in FP64 in a fixed order.  Bound by latency (8 workgroups at 128
+// rows): the split sum used 64 of the 256 threads at 16 columns, 10.2 us for 64 splits and 15.0
+// for 128 (128^3, rank 16); its four groups now take 7.9 and 9.3.  Also
 // writes the panel layout (optionally row-scaled for FP8 storage), the per-block inner
 // product <M, U> (fit) and the per-block Gram partial U_blk^T U_blk.  Register blocks:
 // 1 x 4 outputs of U per thread (V^{-1} is symmetric, so its rows are read contiguously),
@@ -94,26 +96,27 @@ __global__ __launch_bounds__(256) void k_solve(const float *__restrict__ partial
         const int e = tid + 256 * k;
         vreg[k] = e < RR ? Vinv[e] : 0.0;
     }
-    // thread (row r, columns b .. b + 3): one 16-byte load per split (Rp % 16 == 0, so
-    // kSolveRows Rp / 4 <= 256 threads cover the block), 16 splits in flight
-    const int q4 = Rp / 4;
-    if (tid < kSolveRows * q4) {
-        const int r = tid / q4, b = 4 * (tid % q4);
+    // thread (split group g, row r, columns b .. b + 3): one 16-byte load per split, 16 splits in
+    // flight; the 256 threads hold 256 / (4 Rp) groups (4 at Rp 16, 2 at Rp 32, else 1), group g
+    // the splits g, g + groups, ...; the groups are added in order
+    const int q4 = Rp / 4, per = kSolveRows * q4, ng = 256 / per;
+    {
+        const int g = tid / per, t = tid - g * per, r = t / q4, b = 4 * (t % q4);
         const long i = row0 + r;
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        if (i < In) {
+        if (i < In && g < ng) {
             const float4 *pp = reinterpret_cast<const float4 *>(partial + i * Rp + b);
             const long ps4 = rows_pad * Rp / 4;
-            for (int sp = 0; sp < nsplit; sp += 16) {
+            for (int sp = g; sp < nsplit; sp += 16 * ng) {
                 float4 v[16];
 #pragma unroll
                 for (int u = 0; u < 16; ++u) {
-                    const int sq = sp + u < nsplit ? sp + u : nsplit - 1;  // valid; not summed
+                    const int sq = sp + u * ng < nsplit ? sp + u * ng : nsplit - 1;  // valid; not summed
                     v[u] = pp[(long)sq * ps4];
                 }
 #pragma unroll
                 for (int u = 0; u < 16; ++u)
-                    if (sp + u < nsplit) {  // split order, as k_split_sum
+                    if (sp + u * ng < nsplit) {
                         acc[0] += (double)v[u].x;
                         acc[1] += (double)v[u].y;
                         acc[2] += (double)v[u].z;
@@ -121,8 +124,22 @@ __global__ __launch_bounds__(256) void k_solve(const float *__restrict__ partial
                     }
             }
         }
+        if (ng > 1) {
+            // (V^{-1} has not been written yet: its array, R^2 <= 1024 doubles of 4096, is free
+            // above 1024 for the groups past the first)
+            double *gs = Vs + 1024;
+            if (g > 0 && g < ng)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) Ms[r * kMaxR + b + q] = acc[q];
+                for (int q = 0; q < 4; ++q) gs[((g - 1) * per + t) * 4 + q] = acc[q];
+            __syncthreads();
+            if (g == 0)
+                for (int k = 1; k < ng; ++k)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[q] += gs[((k - 1) * per + t) * 4 + q];
+        }
+        if (g == 0)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) Ms[r * kMaxR + b + q] = acc[q];
     }
 #pragma unroll
     for (int k = 0; k < kVPer; ++k) {
@@ -837,7 +854,7 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     S.dtype = dtype;
     S.scales = scales;
     for (int m = 0; m < P.order; ++m) {
-        int st = mttkrp_plan(S.mp[m], P.order, P.dims, m, dtype, P.R, X, 0, split);
+        int st = mttkrp_plan(S.mp[m], P.order, P.dims, m, dtype, P.R, X, true, split);
         if (st) return st;
         if (split) {
             if (dtype != TDX_BF16 || !S.mp[m].lds) {

@@ -470,7 +470,7 @@ static int storage_type(int dtype) {
 }
 
 int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype, long rank,
-                const void *X, int target_wgs, bool split) {
+                const void *X, bool for_solve, bool split) {
     if (order < 2 || order > 4 || mode < 0 || mode >= order || rank <= 0) return record(TDX_ERR_ARG);
     const int st = storage_type(dtype);
     if (st < 0) return record(TDX_ERR_UNSUPPORTED);
@@ -489,7 +489,6 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
     const int vec = (st == 0) ? 4 : 8;
     const size_t align = (st == 2) ? 8 : 16;
     p.fast = rank <= 64 && (dims[0] % vec == 0) && (((uintptr_t)X) % align == 0);
-    if (target_wgs <= 0) target_wgs = 512;
     // the LDS-staged kernel: for output modes > 0 when mode 0 holds whole 16-byte vectors,
     // for mode 0 when it holds whole row groups
     const long lvec = (st == 0) ? 4 : (st == 1) ? 8 : 16;
@@ -519,11 +518,22 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
         if (ns < 1) ns = 1;
         long cps = 1, nss = 1;
         if (ns >= nfc) {
-            // at least 8 slow indices per split: small tensors otherwise produce many tiny
-            // splits whose partials cost more to sum than they save
-            nss = ns / nfc;
-            const long cap = ceil_div(S, 8L);
-            if (nss > cap) nss = cap;
+            // A small tensor is latency: its steps of ~1.2 us each run in turn, so it wants few of
+            // them per workgroup (64 x 48 x 40 rank 6: 15 us with 8 slow indices a split, 7.4 with
+            // 2), as long as the sum over the splits stays short.  The split sum of a standalone
+            // call spreads over the splits (2 slow indices a split); k_solve's has four groups of
+            // 16 loads in flight at 16 columns, which holds 128 splits (20 sweeps of 128^3 rank 16
+            // at 32 / 64 / 128 splits: 2.09 / 1.90 / 1.85 ms; of 256^3 at 128 / 256: 2.35 / 2.67),
+            // and above 16 columns gains nothing past 8 slow indices (128^3 rank 32: 2.87 ms with
+            // 8, 3.04 with 4).  Never more partials than the fixed scratch of the no-allocation
+            // call holds, unless 8 slow indices a split needed them too.
+            const long fit = ns / nfc, base = std::min(fit, ceil_div(S, 8L));
+            const long most = !for_solve ? ceil_div(S, 2L) : p.Rp == 16 ? std::min(ceil_div(S, 2L), 128 / nfc) : 0;
+            nss = std::max(base, std::min(fit, most));
+            size_t need = sizeof(float) * (size_t)(nss * nfc) * p.rows_pad * p.Rp;
+            for (int m = 0; m < order; ++m)
+                if (m != mode) need += (sizeof(float) * (size_t)panel_floats(dims[m], p.Rp) + 255) & ~size_t(255);
+            if (need > kNoAllocScratchBytes) nss = base;
             if (nss < 1) nss = 1;
         } else {
             cps = ceil_div(nfc, ns);
@@ -544,7 +554,7 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
         for (int m = 0; m < order; ++m)
             if (m != mode && m != fmode) S *= dims[m];
         p.ksteps = ceil_div(dims[fmode], KS) * S;
-        long want = ceil_div(target_wgs, p.rowtiles);
+        long want = ceil_div(512L, (long)p.rowtiles);
         long maxs = ceil_div(p.ksteps, 16);  // at least 4 K steps per wave
         long ns = want < maxs ? want : maxs;
         if (ns < 1) ns = 1;
