@@ -13,7 +13,7 @@
 //   relerr from the fast-fit identity, appended to the tensor's history.
 // Every tensor element is read from HBM once per mode, exactly like the single-tensor path.
 // Tunables (block size, slab capacity) are template parameters picked by the autotuner.
-#include "common.hpp"
+#include "batched.hpp"
 #include "linalg.hpp"
 #include <algorithm>
 #include <map>
@@ -23,38 +23,6 @@
 #include <vector>
 
 namespace tdx {
-
-static constexpr int kBMaxDim = 128;
-static constexpr int kBMaxR = 16;
-static constexpr int kSlabCols = 128;  // columns per slab (per-column scratch Ys)
-
-struct BDesc {
-    long xoff;
-    long uoff[3];
-    int I, J, K, R;
-    long toff;  // split design with T: X x_0 A^T of the tensor (J K x R floats) at toff
-};
-
-typedef float bf32x4 __attribute__((ext_vector_type(4)));
-
-// sum over the workgroup: wave shuffles, then one value per wave through LDS (sh >= BS/64
-// doubles); every thread returns the total
-template <int BS>
-__device__ inline double bsum(double v, double *sh) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const int tid = threadIdx.x;
-    __syncthreads();
-    if ((tid & 63) == 0) sh[tid >> 6] = v;
-    __syncthreads();
-    double r = 0.0;
-#pragma unroll
-    for (int w = 0; w < BS / 64; ++w) r += sh[w];
-    return r;
-}
-
-__device__ inline int sel3(int m, int a, int b, int c) { return m == 0 ? a : (m == 1 ? b : c); }
-__device__ inline long sel3l(int m, long a, long b, long c) { return m == 0 ? a : (m == 1 ? b : c); }
 
 // The solve-phase arrays live in the slab (idle between the MTTKRP streams): V, L, W, V^{-1}
 // (R^2 doubles each), the Jacobi fallback's rotation table and the reduction scratch.
@@ -678,6 +646,7 @@ __global__ __launch_bounds__(256) void k_bm_solve(float *__restrict__ U, const f
 }
 
 __global__ void k_batched_prologue(int *queue) { *queue = 0; }
+__global__ void k_batched_set(int *p, int v) { *p = v; }
 __global__ void k_bm_prologue(int *queues) {
     queues[0] = 0;
     queues[1] = 0;
@@ -755,7 +724,10 @@ static const Variant kVariants[] = {
      {k_bm_mttkrp<0, 256, 4096, 3>, k_bm_mttkrp<1, 256, 4096, 3>, k_bm_mode2_t<256, 4096, 3>}},
     {256, 6144, nullptr, "split_t_bs256_slab6k",
      {k_bm_mttkrp<0, 256, 6144, 2>, k_bm_mttkrp<1, 256, 6144, 2>, k_bm_mode2_t<256, 6144, 2>}},
+    // work items of equal size (batched_items.hip), the default
+    {256, 0, nullptr, "items", {nullptr, nullptr, nullptr}},
 };
+static constexpr int kItemsVariant = sizeof(kVariants) / sizeof(kVariants[0]) - 1;
 static bool variant_uses_t(int v) { return v >= 0 && kVariants[v].m[2] != nullptr && strncmp(kVariants[v].name, "split_t_", 8) == 0; }
 static constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -806,8 +778,7 @@ const char *tdx_cp_batched_variant_name(int v) {
 // CP-ALS of `ntensors` 3rd-order tensors packed in X (tensor t at xoff[t], column-major
 // dims[3t..3t+2]) with ranks[t] <= 16 and extents <= 128; factors packed in U (mode m of
 // tensor t at uoff[3t+m], I_m x R column-major).  init = 0 draws U(0,1) from Philox stream
-// (seed + t, m); 1 uses the caller's U.  variant < 0 picks variant 9 (split_t_bs256_slab4k,
-// the autotuner's choice on the 4096-tensor benchmark batch).  fit_hist (host, may
+// (seed + t, m); 1 uses the caller's U.  variant < 0 picks the item design ("items").  fit_hist (host, may
 // be NULL) receives ntensors x sweeps relative errors; sweep_ms (host, may be NULL) the
 // device time of every sweep.  The per-sweep launches are captured once in a hipGraph.
 int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *ranks, const long *xoff,
@@ -815,7 +786,7 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
                        double *fit_hist, float *sweep_ms) {
     if (!X || !U || !dims || !ranks || !xoff || !uoff || ntensors <= 0 || sweeps < 0) return record(TDX_ERR_ARG);
     if (variant >= kNumVariants) return record(TDX_ERR_ARG);
-    if (variant < 0) variant = 9;
+    if (variant < 0) variant = kItemsVariant;
     std::vector<BDesc> h(ntensors);
     std::vector<std::pair<long, int>> order(ntensors);
     for (long t = 0; t < ntensors; ++t) {
@@ -847,14 +818,14 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
     double *d_nx = nullptr, *d_fit = nullptr;
     struct Guard {
         hipStream_t st;
-        void *p[8];
+        void *p[11];
         ~Guard() {
             if (st) (void)hipStreamSynchronize(st);
             for (void *q : p)
                 if (q) (void)hipFree(q);
             if (st) (void)hipStreamDestroy(st);
         }
-    } guard{owned, {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}};
+    } guard{owned, {nullptr}};
     TDX_HIP(hipMalloc(&d_desc, sizeof(BDesc) * ntensors));
     guard.p[0] = d_desc;
     TDX_HIP(hipMalloc(&d_sched, sizeof(int) * ntensors));
@@ -872,10 +843,34 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
     k_batched_prologue<<<1, 1, 0, s>>>(sweep_ctr);
     k_batched_prologue<<<1, 1, 0, s>>>(status);
     if (init == 0) k_batched_init<<<1024, 256, 0, s>>>(U, d_desc, (int)ntensors, seed);
-    k_batched_norm2<<<1024, 256, 0, s>>>(X, d_desc, (int)ntensors, d_nx);
     TDX_LAUNCH_CHECK();
     BmBuffers bm;
-    if (!kVariants[variant].fn) {
+    ItemPlan ip;
+    ItemBuffers ib{};
+    const bool items = variant == kItemsVariant;
+    if (items) {
+        items_plan(ip, h.data(), ntensors);
+        void **dst[6] = {(void **)&ib.desc, (void **)&ib.items, (void **)&ib.part, (void **)&ib.T, (void **)&ib.G,
+                         (void **)&ib.npart};
+        const size_t bytes[6] = {sizeof(IDesc) * ntensors, sizeof(IItem) * ip.items.size(),
+                                 sizeof(float) * ip.part_floats, sizeof(float) * ip.t_floats,
+                                 sizeof(double) * ntensors * 3 * kBMaxR * kBMaxR, sizeof(double) * ip.items.size()};
+        for (int k = 0; k < 6; ++k) {
+            TDX_HIP(hipMalloc(dst[k], bytes[k]));
+            guard.p[5 + k] = *dst[k];
+        }
+        ib.ntensors = (int)ntensors;
+        ib.nitems = (int)ip.items.size();
+        TDX_HIP(hipMemcpyAsync((void *)ib.desc, ip.desc.data(), bytes[0], hipMemcpyHostToDevice, s));
+        TDX_HIP(hipMemcpyAsync((void *)ib.items, ip.items.data(), bytes[1], hipMemcpyHostToDevice, s));
+        k_batched_set<<<1, 1, 0, s>>>(sweep_ctr, -1);
+        const int st = items_prologue(ib, X, U, d_nx, s);
+        if (st) return st;
+    } else {
+        k_batched_norm2<<<1024, 256, 0, s>>>(X, d_desc, (int)ntensors, d_nx);
+        TDX_LAUNCH_CHECK();
+    }
+    if (!items && !kVariants[variant].fn) {
         long mf = 0;  // M is laid out like the factors
         for (long t = 0; t < ntensors; ++t)
             for (int m = 0; m < 3; ++m) mf = std::max(mf, h[t].uoff[m] + (long)dims[3 * t + m] * h[t].R);
@@ -901,8 +896,9 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
     TDX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int st = launch_variant(variant, s, X, U, d_desc, d_sched, (int)ntensors, queue, d_nx, d_fit, S, sweep_ctr,
-                            status, bm);
+    int st = items ? items_sweep(ib, X, U, d_nx, d_fit, S, sweep_ctr, status, s)
+                   : launch_variant(variant, s, X, U, d_desc, d_sched, (int)ntensors, queue, d_nx, d_fit, S, sweep_ctr,
+                                    status, bm);
     hipError_t e = hipStreamEndCapture(s, &g);
     if (st) {
         if (g) (void)hipGraphDestroy(g);

@@ -282,9 +282,10 @@ int tdx_cp_tensorcore(const float *X, float *A, float *B, float *C, long a, long
  *      call, src/cp_als.cu:3) ---- */
 /* CP-ALS of `ntensors` 3rd-order tensors packed in X (tensor t at element offset xoff[t],
  * column-major, extents dims[3t..3t+2] <= 128) with ranks[t] <= 16; factors packed in U (mode
- * m of tensor t at uoff[3t+m], I_m x R column-major).  Workgroups pull tensors from a
- * size-sorted queue: one persistent kernel per sweep, or (the split variants, the default)
- * one MTTKRP and one solve kernel per mode; the sweep is captured in a hipGraph.  init = 0 draws
+ * m of tensor t at uoff[3t+m], I_m x R column-major).  By default the batch is cut into work items
+ * of equal size (runs of slices of a tensor); the older variants (a persistent kernel per sweep, or
+ * one MTTKRP and one solve kernel per mode over a queue of whole tensors) are kept for the
+ * autotuner.  A sweep is captured in a hipGraph.  init = 0 draws
  * U(0,1) from Philox stream (seed + t, m), 1 uses the caller's U.  variant: kernel variant
  * (see tdx_cp_batched_autotune), < 0 for the default.  fit_hist (host, ntensors x sweeps,
  * may be NULL) receives the fast-fit relative errors; sweep_ms (host, may be NULL) the device
