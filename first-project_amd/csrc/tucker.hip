@@ -9,8 +9,8 @@
 //
 // The Gram never forms an unfolded copy (the reference materialises X2 with t2m and, for
 // order 4, X2 and X3 by identity-matrix GEMMs, src/tucker4_hosvd.cu:23-37): a workgroup
-// stages 32 fibres of the (P, In, Q) view in LDS and accumulates an In x In FP32 tile,
-// partial tiles are summed in FP64 in a fixed order.  The eigensolve is the FP64
+// accumulates an In x In FP32 tile over a range of the (P, In, Q) view's fibres (gram_any.hip,
+// gram.hip), partial tiles are summed in FP64 in a fixed order.  The eigensolve is the FP64
 // tridiagonal solver in one workgroup (subspace iteration first where the top eigenvalues
 // stand clear of the rest, warm-started from the previous factor in HOOI); eigenvector signs
 // are fixed so that the entry of largest magnitude is positive (syevdx leaves the sign
@@ -25,66 +25,12 @@ namespace tdx {
 
 int ttm_generic(const float *X, int order, const long *dims, int mode, const float *U, long lda, long ldi, long Ra,
                 float *Y, hipStream_t s);
-int gram_mfma_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
+int gram_mfma_launch(const void *X, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
+int gram_any_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
 int ttm_generic_t(const void *X, int xtype, int order, const long *dims, int mode, const float *U, long lda, long ldi,
                   long Ra, float *Y, hipStream_t s);
 
 static constexpr int kGramMaxN = 128;
-static constexpr int kGramChunk = 32;
-
-// partial Gram of the (P, In, Q) view over fibre chunks: thread (ty, tx) owns an 8x8 block
-// of the In x In tile (In <= 128).  Fibre k of a chunk is (p, q) with p fastest.
-__device__ __forceinline__ float ldx(const float *p, long i) { return p[i]; }
-__device__ __forceinline__ float ldx(const uint16_t *p, long i) { return __uint_as_float((uint32_t)p[i] << 16); }
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_gram_partial(const T *__restrict__ X, long P, long In, long Q,
-                                                      long kper, float *__restrict__ part) {
-    __shared__ float xs[kGramChunk][kGramMaxN + 1];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const long K = P * Q;
-    const long k0 = blockIdx.x * kper, k1 = min(k0 + kper, K);
-    float acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0f;
-    for (long kb = k0; kb < k1; kb += kGramChunk) {
-        // stage X[fibre kb+kk][a] for kk < 32, a < In
-        for (int e = tid; e < kGramChunk * kGramMaxN; e += 256) {
-            int kk, a;
-            if (P == 1) { a = e % kGramMaxN; kk = e / kGramMaxN; }   // contiguous along a
-            else { kk = e % kGramChunk; a = e / kGramChunk; }      // contiguous along p
-            const long k = kb + kk;
-            float v = 0.0f;
-            if (k < k1 && a < In) {
-                const long p = k % P, q = k / P;
-                v = ldx(X, p + a * P + q * P * In);
-            }
-            xs[kk][a] = v;
-        }
-        __syncthreads();
-        for (int kk = 0; kk < kGramChunk; ++kk) {
-            float av[8], bv[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                av[i] = xs[kk][ty * 8 + i];
-                bv[i] = xs[kk][tx * 8 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-    float *dst = part + (long)blockIdx.x * kGramMaxN * kGramMaxN;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dst[(ty * 8 + i) * kGramMaxN + tx * 8 + j] = acc[i][j];
-}
 
 // G = the sum of the nblk FP32 partial Grams (pitch kGramMaxN), in FP64: a workgroup takes 64
 // consecutive entries (a, b) of the upper triangle (b fastest: contiguous reads) and its four
@@ -193,28 +139,13 @@ static int unfold_gram(const void *X, int xtype, int order, const long *dims, in
     for (int m = mode + 1; m < order; ++m) Q *= dims[m];
     const long In = dims[mode];
     if (In > kGramMaxN) return record(TDX_ERR_UNSUPPORTED);
-    const long K = P * Q;
-    // MFMA path for the shapes it covers (16-byte vectors along the contiguous index)
-    {
-        const int mb = W.gram_blocks < 512 ? W.gram_blocks : 512;
-        const int nb = gram_mfma_launch(X, xtype, P, In, Q, W.gram_part, mb, s);
-        if (nb < 0) return record(TDX_ERR_HIP);
-        if (nb > 0) {
-            k_gram_sum<<<(int)ceil_div(In * In, 64L), 256, 0, s>>>(W.gram_part, nb, In, G);
-            TDX_LAUNCH_CHECK();
-            return TDX_OK;
-        }
-    }
-    long nblk = ceil_div(K, 2048);
-    if (nblk > W.gram_blocks) nblk = W.gram_blocks;
-    if (nblk < 1) nblk = 1;
-    long kper = ceil_div(ceil_div(K, nblk), kGramChunk) * kGramChunk;
-    nblk = ceil_div(K, kper);
+    // the BF16 kernel for whole vectors (gram.hip), the LDS kernel otherwise
+    int nb = 0;
     if (xtype == TDX_BF16)
-        k_gram_partial<uint16_t><<<(int)nblk, 256, 0, s>>>((const uint16_t *)X, P, In, Q, kper, W.gram_part);
-    else
-        k_gram_partial<float><<<(int)nblk, 256, 0, s>>>((const float *)X, P, In, Q, kper, W.gram_part);
-    k_gram_sum<<<(int)ceil_div(In * In, 64L), 256, 0, s>>>(W.gram_part, (int)nblk, In, G);
+        nb = gram_mfma_launch(X, P, In, Q, W.gram_part, W.gram_blocks < 512 ? W.gram_blocks : 512, s);
+    if (nb == 0) nb = gram_any_launch(X, xtype, P, In, Q, W.gram_part, W.gram_blocks, s);
+    if (nb < 0) return record(TDX_ERR_HIP);
+    k_gram_sum<<<(int)ceil_div(In * In, 64L), 256, 0, s>>>(W.gram_part, nb, In, G);
     TDX_LAUNCH_CHECK();
     return TDX_OK;
 }
