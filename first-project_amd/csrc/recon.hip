@@ -1,6 +1,7 @@
 // recon.hip -- reconstruction, residual norms, synthetic CP tensors and the generic
 // mode-n product used by the Tucker path.
 #include "common.hpp"
+#include <algorithm>
 #include <math.h>
 
 namespace tdx {
@@ -25,14 +26,197 @@ struct FacArgs {
     int R;
 };
 
-// For each fibre along mode 0 (fixed i_1..i_{d-1}): w[r] = prod_{m>=1} U_m[i_m, r] in
-// LDS, then x_hat[i] = sum_r U_0[i, r] w[r].
-//  MODE 0: write x_hat (gencp / gencp4, src/rse.cu:17-30,53-73)
-//  MODE 1: accumulate (x - x_hat)^2 and x^2 in FP64 (compensated CP residual)
-//  MODE 2: write x_hat and accumulate x_hat^2 and e^2 for E ~ N(0,1) (synthetic tensors)
-template <int MODE>
-__global__ __launch_bounds__(256) void k_cp_fibres(FacArgs f, float *__restrict__ out, const float *__restrict__ X,
-                                                   double *__restrict__ part, uint64_t seed, uint32_t strm) {
+// The CP model and its residual, x_hat[i, c] = sum_r U_0[i, r] w[c, r] over the fibres c =
+// (i_1, .., i_{d-1}) with w[c, r] = U_1[i_1, r] (U_2[i_2, r] U_3[i_3, r]), on FP32 MFMA.
+//  RES = false: writes x_hat (gencp / gencp4, src/rse.cu:17-30,53-73)
+//  RES = true: sums (x - x_hat)^2 and x^2 in FP64 (compensated CP residual)
+// A workgroup walks a range of fibres 64 at a time: its threads form w for them in LDS (a lane a
+// fibre, whose digits advance by a mixed-radix addition; the next 64's factor entries are in
+// flight meanwhile), RW of its waves take a block of 64 rows each and the other 4 / RW share the
+// four blocks of 16 fibres.  A wave's U_0 rows stay in registers as the A operand (KS k-steps of 4
+// columns; BIG, ranks above 64, reloads them per block of 64 columns).  Lane (lm, lg) holds rows
+// 16 t + 4 lg .. + 3 of fibre lm: 16-byte loads and stores of whole 64-byte runs, 4-byte aligned.
+// Bound by HBM (512 x 384 x 320: 252 MB, 55 us at the 4.6 TB/s of a large copy).  One thread per
+// entry, with a load of U_0 for every multiply-add, took 496 us (model) and 828 us (residual) at
+// rank 32; these take 68 and 90 us (each wave loading its own w: 157 and 215).
+typedef float rc_f4 __attribute__((ext_vector_type(4)));
+typedef float rc_f4u __attribute__((ext_vector_type(4), aligned(4)));
+static constexpr int kModelLd = 80;  // W row pitch: 4 rows of 16 fibres in distinct banks
+
+template <bool RES, int KS, int RW, bool BIG>
+__global__ __launch_bounds__(256, 2) void k_cp_model(FacArgs f, float *__restrict__ out, const float *__restrict__ X,
+                                                     long ntile, long tper, int nrg, double *__restrict__ part) {
+    extern __shared__ float W[];  // [max(4 KS, R rounded up to 64)][kModelLd]
+    __shared__ double sh[RES ? 256 : 1];
+    constexpr int FW = 4 / RW;
+    const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave % RW, fw = wave / RW;
+    const long I = f.dims[0], D1 = f.dims[1], D2 = f.dims[2], D3 = f.dims[3];
+    const long nfib = D1 * D2 * D3;
+    const int R = f.R;
+    const long row0 = ((long)(blockIdx.x % nrg) * RW + rw) * 64;
+    const long t0 = (blockIdx.x / nrg) * tper, t1 = min(t0 + tper, ntile);
+    const float *U0 = f.U[0], *U1 = f.U[1], *U2 = f.order > 2 ? f.U[2] : nullptr,
+                *U3 = f.order > 3 ? f.U[3] : nullptr;
+    double s1 = 0.0, c1 = 0.0, s2 = 0.0, c2 = 0.0;
+
+    float aop[4][KS];
+    auto load_a = [&](int r0) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float *p = U0 + min(row0 + 16 * t + lm, I - 1);
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const int r = r0 + 4 * k + lg;
+                aop[t][k] = p[(r < R ? r : 0) * I];
+            }
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+                if (r0 + 4 * k + lg >= R) aop[t][k] = 0.0f;
+        }
+    };
+    if (!BIG) load_a(0);
+    // this lane's fibre of the 64 and its digits
+    long c = 64 * t0 + lane;
+    long i1 = c % D1, i2 = (c / D1) % D2, i3 = c / D1 / D2;
+    const long A1 = 64 % D1, A2 = (64 / D1) % D2, A3 = 64 / D1 / D2;
+    float w1[KS], w2[KS], w3[KS];  // columns r0 + wave + 4 k of the fibre's factor rows
+    auto load_w = [&](int r0) {
+        const bool on = c < nfib;
+        const float *p1 = U1 + (on ? i1 : 0), *p2 = U2 ? U2 + (on ? i2 : 0) : U1, *p3 = U3 ? U3 + (on ? i3 : 0) : U1;
+        int rb = r0 + wave;
+        asm volatile("" : "+s"(rb));  // (hoisted out of the loop the column offsets fill the scalar registers)
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const long r = rb + 4 * k < R ? rb + 4 * k : 0;
+            w1[k] = p1[r * D1];
+            if (U2) w2[k] = p2[r * D2];
+            if (U3) w3[k] = p3[r * D3];
+        }
+    };
+    auto store_w = [&](int r0) {
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            // reference order: the KR of the later modes is formed first (src/rse.cu:65-66)
+            float q = 1.0f, v = w1[k];
+            if (U2) q = w2[k];
+            if (U3) q *= w3[k];
+            if (U2) v *= q;
+            W[(r0 + wave + 4 * k) * kModelLd + lane] = r0 + wave + 4 * k < R ? v : 0.0f;
+        }
+    };
+    auto advance = [&]() {
+        c += 64;
+        i1 += A1;
+        i2 += A2;
+        i3 += A3;
+        if (i1 >= D1) {
+            i1 -= D1;
+            ++i2;
+        }
+        if (i2 >= D2) {
+            i2 -= D2;
+            ++i3;
+        }
+    };
+    const bool rows = row0 + 64 <= I;  // uniform
+    if (!BIG && t0 < t1) load_w(0);
+    for (long tl = t0; tl < t1; ++tl) {
+        __syncthreads();  // every wave is done with the previous W
+        if constexpr (BIG) {
+            for (int r0 = 0; r0 < R; r0 += 4 * KS) {
+                load_w(r0);
+                store_w(r0);
+            }
+            advance();
+        } else {
+            store_w(0);
+        }
+        __syncthreads();
+        if constexpr (!BIG) {
+            advance();
+            load_w(0);  // past the last tile: valid addresses, never consumed
+        }
+        if (row0 >= I) continue;  // (a row block past the extent: this wave only forms w)
+        for (int fb = fw; fb < 4; fb += FW) {
+            const long cf = 64 * tl + 16 * fb + lm;  // this lane's fibre of the block
+            const bool on = cf < nfib, full = rows && 64 * tl + 16 * fb + 16 <= nfib;
+            rc_f4 x[4];
+            if constexpr (RES) {
+                const float *p = X + (on ? cf : 0) * I + row0 + 4 * lg;
+                if (full) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) x[t] = *reinterpret_cast<const rc_f4u *>(p + 16 * t);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) x[t][v] = p[min(16L * t + v, I - 1 - row0 - 4 * lg)];
+                }
+            }
+            rc_f4 acc[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = rc_f4{0.f, 0.f, 0.f, 0.f};
+            for (int r0 = 0; r0 < (BIG ? R : 1); r0 += 4 * KS) {
+                if (BIG) load_a(r0);
+                const float *wp = W + (r0 + lg) * kModelLd + 16 * fb + lm;
+#pragma unroll
+                for (int k = 0; k < KS; ++k) {
+                    const float w = wp[4 * k * kModelLd];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (row0 + 16 * t < I)
+                            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(aop[t][k], w, acc[t], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const long i = row0 + 16 * t + 4 * lg;
+                if constexpr (RES) {
+                    // four squares added, then compensated
+                    double d2 = 0.0, x2 = 0.0;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        double xv = (double)x[t][v], d = xv - (double)acc[t][v];
+                        if (!full && !(on && i + v < I)) xv = d = 0.0;
+                        d2 = fma(d, d, d2);
+                        x2 = fma(xv, xv, x2);
+                    }
+                    double y = d2 - c1, s = s1 + y;
+                    c1 = (s - s1) - y;
+                    s1 = s;
+                    y = x2 - c2;
+                    s = s2 + y;
+                    c2 = (s - s2) - y;
+                    s2 = s;
+                } else {
+                    float *p = out + (on ? cf : 0) * I + i;
+                    if (full) {
+                        *reinterpret_cast<rc_f4u *>(p) = acc[t];
+                    } else if (on) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (i + v < I) p[v] = acc[t][v];
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (RES) {
+        s1 = block_sum_d(s1, sh);
+        s2 = block_sum_d(s2, sh);
+        if (tid == 0) {
+            part[2 * blockIdx.x] = s1;
+            part[2 * blockIdx.x + 1] = s2;
+        }
+    }
+}
+
+// Synthetic tensors: for each fibre along mode 0 (fixed i_1..i_{d-1}) w[r] = prod_{m>=1}
+// U_m[i_m, r] in LDS, then x_hat[i] = sum_r U_0[i, r] w[r]; writes x_hat and accumulates x_hat^2
+// and e^2 for E ~ N(0,1).
+__global__ __launch_bounds__(256) void k_cp_fibres(FacArgs f, float *__restrict__ out, double *__restrict__ part,
+                                                   uint64_t seed, uint32_t strm) {
     __shared__ float w[64 * 4];
     __shared__ double sh[256];
     const long I0 = f.dims[0];
@@ -59,38 +243,25 @@ __global__ __launch_bounds__(256) void k_cp_fibres(FacArgs f, float *__restrict_
             float acc = 0.0f;
             for (int r = 0; r < f.R; ++r) acc = fmaf(f.U[0][i + r * I0], w[r], acc);
             const long e = fib * I0 + i;
-            if (MODE == 0) out[e] = acc;
-            if (MODE == 1) {
-                double d = (double)X[e] - (double)acc;
-                double y = d * d - c1, t = s1 + y;
-                c1 = (t - s1) - y; s1 = t;
-                double x2 = (double)X[e] * (double)X[e];
-                y = x2 - c2; t = s2 + y;
-                c2 = (t - s2) - y; s2 = t;
-            }
-            if (MODE == 2) {
-                out[e] = acc;
-                uint64_t n = (uint64_t)e;
-                uint64_t blk = (2 * n) >> 2;
-                uint32_t c[4] = {(uint32_t)blk, (uint32_t)(blk >> 32), strm, 0u};
-                philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-                int wd = (int)((2 * n) & 3);
-                double u1 = (double)word_to_uniform(c[wd]), u2 = (double)word_to_uniform(c[wd + 1]);
-                double g = (double)(float)(sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2));
-                double y = (double)acc * (double)acc - c1, t = s1 + y;
-                c1 = (t - s1) - y; s1 = t;
-                y = g * g - c2; t = s2 + y;
-                c2 = (t - s2) - y; s2 = t;
-            }
+            out[e] = acc;
+            uint64_t n = (uint64_t)e;
+            uint64_t blk = (2 * n) >> 2;
+            uint32_t c[4] = {(uint32_t)blk, (uint32_t)(blk >> 32), strm, 0u};
+            philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+            int wd = (int)((2 * n) & 3);
+            double u1 = (double)word_to_uniform(c[wd]), u2 = (double)word_to_uniform(c[wd + 1]);
+            double g = (double)(float)(sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2));
+            double y = (double)acc * (double)acc - c1, t = s1 + y;
+            c1 = (t - s1) - y; s1 = t;
+            y = g * g - c2; t = s2 + y;
+            c2 = (t - s2) - y; s2 = t;
         }
     }
-    if (MODE != 0) {
-        s1 = block_sum_d(s1, sh);
-        s2 = block_sum_d(s2, sh);
-        if (threadIdx.x == 0) {
-            part[2 * blockIdx.x] = s1;
-            part[2 * blockIdx.x + 1] = s2;
-        }
+    s1 = block_sum_d(s1, sh);
+    s2 = block_sum_d(s2, sh);
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = s1;
+        part[2 * blockIdx.x + 1] = s2;
     }
 }
 
@@ -121,18 +292,54 @@ __global__ void k_add_noise(float *__restrict__ X, long n, const double *__restr
     }
 }
 
-// ||X - X1||^2 and ||X||^2 (FP64, compensated) partials (src/rse.cu:4-15 without clobbering X1)
+// ||X - X1||^2 and ||X||^2 (FP64, compensated) partials (src/rse.cu:4-15 without clobbering X1).
+// Bound by HBM: 4 elements of each per load (VEC) and four loads in flight; the squares of a
+// load are added before the compensated sum.  63 M elements (512 x 384 x 320): 151 us with one
+// element a load and one load in flight, 80 us here.
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_rse_partial(const float *__restrict__ X, const float *__restrict__ X1, long n,
                                                      double *__restrict__ part) {
     __shared__ double sh[256];
+    constexpr int W = VEC ? 4 : 1;
+    typedef float vec __attribute__((ext_vector_type(4)));
     double s1 = 0.0, c1 = 0.0, s2 = 0.0, c2 = 0.0;
-    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-        double x = X[e];
-        double d = x - (double)X1[e];
-        double y = d * d - c1, t = s1 + y;
+    const long n4 = n / W, st = (long)gridDim.x * 256;
+    auto take = [&](double d2, double x2) {
+        double y = d2 - c1, t = s1 + y;
         c1 = (t - s1) - y; s1 = t;
-        y = x * x - c2; t = s2 + y;
+        y = x2 - c2; t = s2 + y;
         c2 = (t - s2) - y; s2 = t;
+    };
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n4; e += 4 * st) {
+        float a[4][W], b[4][W];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const long i = e + u * st < n4 ? e + u * st : e;
+            if constexpr (VEC) {
+                const vec va = __builtin_nontemporal_load(reinterpret_cast<const vec *>(X) + i);
+                const vec vb = __builtin_nontemporal_load(reinterpret_cast<const vec *>(X1) + i);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) a[u][q] = va[q], b[u][q] = vb[q];
+            } else {
+                a[u][0] = X[i];
+                b[u][0] = X1[i];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            double d2 = 0.0, x2 = 0.0;
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                const double x = a[u][q], d = x - (double)b[u][q];
+                d2 = fma(d, d, d2);
+                x2 = fma(x, x, x2);
+            }
+            if (e + u * st < n4) take(d2, x2);
+        }
+    }
+    if (VEC && blockIdx.x == 0 && threadIdx.x < n - 4 * n4) {
+        const double x = X[4 * n4 + threadIdx.x], d = x - (double)X1[4 * n4 + threadIdx.x];
+        take(d * d, x * x);
     }
     s1 = block_sum_d(s1, sh);
     s2 = block_sum_d(s2, sh);
@@ -181,19 +388,65 @@ int ttm_generic(const float *X, int order, const long *dims, int mode, const flo
     return ttm_generic_t(X, TDX_F32, order, dims, mode, U, lda, ldi, Ra, Y, s);
 }
 
-static int cp_fibres_launch(int mode, int order, const long *dims, const float *const *U, long R, float *out,
-                            const float *X, double *part, int blocks, uint64_t seed, uint32_t strm, hipStream_t s) {
+static constexpr long kModelBlocks = 2048;
+// row groups of a k_cp_model launch: the most row blocks a workgroup can take (4, 2 or 1) with at
+// most a sixth of them past the extent
+static long model_row_waves(long I0) {
+    const long nrc = ceil_div(I0, 64L);
+    for (long rw = 4; rw > 1; rw /= 2)
+        if (6 * (ceil_div(nrc, rw) * rw - nrc) <= nrc) return rw;
+    return 1;
+}
+// the most workgroups such a launch has
+static long model_blocks(long I0) { return kModelBlocks + ceil_div(ceil_div(I0, 64L), model_row_waves(I0)); }
+
+static int fac_args(FacArgs &f, int order, const long *dims, const float *const *U, long R) {
     if (R > 256) return record(TDX_ERR_UNSUPPORTED);
-    FacArgs f{};
     f.order = order;
     f.R = (int)R;
     for (int m = 0; m < 4; ++m) {
         f.U[m] = m < order ? U[m] : nullptr;
         f.dims[m] = m < order ? dims[m] : 1;
     }
-    if (mode == 0) k_cp_fibres<0><<<blocks, 256, 0, s>>>(f, out, X, part, seed, strm);
-    else if (mode == 1) k_cp_fibres<1><<<blocks, 256, 0, s>>>(f, out, X, part, seed, strm);
-    else k_cp_fibres<2><<<blocks, 256, 0, s>>>(f, out, X, part, seed, strm);
+    return TDX_OK;
+}
+
+// the model into out, or (X) its residual partials into part, one pair per block of *blocks
+static int cp_model_launch(int order, const long *dims, const float *const *U, long R, float *out, const float *X,
+                           double *part, int *blocks, hipStream_t s) {
+    FacArgs f{};
+    int st = fac_args(f, order, dims, U, R);
+    if (st) return st;
+    // about kModelBlocks workgroups, of at least two tiles of 64 fibres
+    const long rw = model_row_waves(dims[0]), nrg = ceil_div(ceil_div(dims[0], 64L), rw);
+    const long ntile = ceil_div(f.dims[1] * f.dims[2] * f.dims[3], 64L);
+    const long tper = std::max(2L, ceil_div(nrg * ntile, kModelBlocks));
+    const int grid = (int)(nrg * ceil_div(ntile, tper));
+    if (blocks) *blocks = grid;
+    const int ks = R <= 16 ? 4 : R <= 32 ? 8 : R <= 48 ? 12 : 16;
+    const size_t lds = sizeof(float) * kModelLd * (size_t)std::max(4L * ks, ceil_div(R, 64L) * 64L * (R > 64));
+#define TDX_MODEL2(KS_, RW_, BIG_)                                                                                  \
+    do {                                                                                                            \
+        if (BIG_ && lds > 65536)                                                                                    \
+            TDX_HIP(hipFuncSetAttribute(X ? (const void *)k_cp_model<true, KS_, RW_, BIG_>                          \
+                                          : (const void *)k_cp_model<false, KS_, RW_, BIG_>,                        \
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                     \
+        if (X) k_cp_model<true, KS_, RW_, BIG_><<<grid, 256, lds, s>>>(f, out, X, ntile, tper, (int)nrg, part);     \
+        else k_cp_model<false, KS_, RW_, BIG_><<<grid, 256, lds, s>>>(f, out, X, ntile, tper, (int)nrg, part);      \
+    } while (0)
+#define TDX_MODEL(KS_, BIG_)                         \
+    do {                                             \
+        if (rw == 4) TDX_MODEL2(KS_, 4, BIG_);       \
+        else if (rw == 2) TDX_MODEL2(KS_, 2, BIG_);  \
+        else TDX_MODEL2(KS_, 1, BIG_);               \
+    } while (0)
+    if (R > 64) TDX_MODEL(16, true);
+    else if (ks == 4) TDX_MODEL(4, false);
+    else if (ks == 8) TDX_MODEL(8, false);
+    else if (ks == 12) TDX_MODEL(12, false);
+    else TDX_MODEL(16, false);
+#undef TDX_MODEL
+#undef TDX_MODEL2
     TDX_LAUNCH_CHECK();
     return TDX_OK;
 }
@@ -208,7 +461,7 @@ int tdx_gencp(float *rec, const float *A, const float *B, const float *C, long a
     TDX_CHECK_ARG(rec && A && B && C && a > 0 && b > 0 && c > 0 && r > 0);
     const long dims[3] = {a, b, c};
     const float *U[3] = {A, B, C};
-    return record(cp_fibres_launch(0, 3, dims, U, r, rec, nullptr, nullptr, 2048, 0, 0, stream()));
+    return record(cp_model_launch(3, dims, U, r, rec, nullptr, nullptr, nullptr, stream()));
 }
 
 int tdx_gencp4(float *rec, const float *A, const float *B, const float *C, const float *D, long a, long b, long c,
@@ -216,7 +469,7 @@ int tdx_gencp4(float *rec, const float *A, const float *B, const float *C, const
     TDX_CHECK_ARG(rec && A && B && C && D && a > 0 && b > 0 && c > 0 && d > 0 && r > 0);
     const long dims[4] = {a, b, c, d};
     const float *U[4] = {A, B, C, D};
-    return record(cp_fibres_launch(0, 4, dims, U, r, rec, nullptr, nullptr, 2048, 0, 0, stream()));
+    return record(cp_model_launch(4, dims, U, r, rec, nullptr, nullptr, nullptr, stream()));
 }
 
 int tdx_cp_relerr(const void *X, int dtype, const float *scales, int order, const long *dims,
@@ -224,15 +477,16 @@ int tdx_cp_relerr(const void *X, int dtype, const float *scales, int order, cons
     TDX_CHECK_ARG(X && dims && factors && relerr && order >= 2 && order <= 4 && rank > 0);
     if (dtype != TDX_F32) return record(TDX_ERR_UNSUPPORTED);
     (void)scales;
-    const int blocks = 2048;
+    const long blocks = model_blocks(dims[0]);
     void *ws = nullptr;
     int st = workspace(WS_MISC0, sizeof(double) * (2 * blocks + 1), &ws);
     if (st) return st;
     double *part = (double *)ws;
     hipStream_t s = stream();
-    st = cp_fibres_launch(1, order, dims, factors, rank, nullptr, (const float *)X, part, blocks, 0, 0, s);
+    int used = 0;
+    st = cp_model_launch(order, dims, factors, rank, nullptr, (const float *)X, part, &used, s);
     if (st) return record(st);
-    k_ratio<<<1, 256, 0, s>>>(part, blocks, part + 2 * blocks);
+    k_ratio<<<1, 256, 0, s>>>(part, used, part + 2 * blocks);
     TDX_LAUNCH_CHECK();
     TDX_HIP(hipMemcpyAsync(relerr, part + 2 * blocks, sizeof(double), hipMemcpyDeviceToHost, s));
     TDX_HIP(hipStreamSynchronize(s));
@@ -250,8 +504,11 @@ int tdx_gen_cp_tensor(float *X, int order, const long *dims, const float *const 
     hipStream_t s = stream();
     long N = 1;
     for (int m = 0; m < order; ++m) N *= dims[m];
-    st = cp_fibres_launch(2, order, dims, factors, rank, X, nullptr, part, blocks, seed, strm, s);
-    if (st) return record(st);
+    FacArgs f{};
+    st = fac_args(f, order, dims, factors, rank);
+    if (st) return st;
+    k_cp_fibres<<<blocks, 256, 0, s>>>(f, X, part, seed, strm);
+    TDX_LAUNCH_CHECK();
     long g = ceil_div(N, 256);
     if (g > 65536) g = 65536;
     k_add_noise<<<(int)g, 256, 0, s>>>(X, N, part, blocks, eta, seed, strm);
@@ -261,13 +518,14 @@ int tdx_gen_cp_tensor(float *X, int order, const long *dims, const float *const 
 
 int tdx_rse(const float *X, const float *X1, long m, float *error) {
     TDX_CHECK_ARG(X && X1 && error && m > 0);
-    const int blocks = 1024;
+    const int blocks = (int)std::min(2048L, ceil_div(m, 1024L));
     void *ws = nullptr;
     int st = workspace(WS_MISC0, sizeof(double) * (2 * blocks + 1), &ws);
     if (st) return st;
     double *part = (double *)ws;
     hipStream_t s = stream();
-    k_rse_partial<<<blocks, 256, 0, s>>>(X, X1, m, part);
+    if (((((uintptr_t)X) | ((uintptr_t)X1)) & 15) == 0) k_rse_partial<true><<<blocks, 256, 0, s>>>(X, X1, m, part);
+    else k_rse_partial<false><<<blocks, 256, 0, s>>>(X, X1, m, part);
     k_ratio<<<1, 256, 0, s>>>(part, blocks, part + 2 * blocks);
     TDX_LAUNCH_CHECK();
     double r = 0.0;
