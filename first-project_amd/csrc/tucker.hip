@@ -67,43 +67,56 @@ __global__ __launch_bounds__(256) void k_gram_sum(const float *__restrict__ part
     }
 }
 
-// Top-r eigenvectors of the symmetric n x n G (FP64), one workgroup: U (n x r, col-major
+// Top-r eigenvectors of a symmetric n x n G (FP64), one workgroup each: U (n x r, col-major
 // FP32) receives the eigenvectors of the r largest eigenvalues in ascending order.  With
 // try_sub the subspace-iteration path runs first (start block U0, or a built-in one when U0
 // is null; U0 may alias U) and the tridiagonal solver only when it declines.  method (optional,
 // device) receives 1 for the subspace path, 0 for the tridiagonal one.
-__global__ __launch_bounds__(kEigThreads) void k_top_eigvecs(const double *__restrict__ G, int n, int r,
-                                                             const float *U0, int try_sub, float *U, double *w,
-                                                             double *__restrict__ scratch, int *method, int rotate) {
+// A solve is one workgroup's chain of ~200 us whatever the size of the tensor, so the independent
+// ones of an HOSVD (a mode each) share one launch: three modes of 125 x 101 x 77 took 164 + 187 +
+// 249 us one after the other.
+struct EigJob {
+    const double *G;
+    int n, r;
+    const float *U0;
+    float *U;
+    double *w, *scratch;
+    int *method;
+};
+struct EigJobs {
+    EigJob j[4];
+};
+__global__ __launch_bounds__(kEigThreads) void k_top_eigvecs(EigJobs jobs, int try_sub, int rotate) {
     extern __shared__ double smem[];
-    if (try_sub && r <= kSubMaxR) {
-        if (sym_top_eigvecs_subspace(G, n, r, U0, U, w, smem, rotate != 0)) {
-            if (method && threadIdx.x == 0) *method = 1;
+    const EigJob q = jobs.j[blockIdx.x];
+    if (try_sub && q.r <= kSubMaxR) {
+        if (sym_top_eigvecs_subspace(q.G, q.n, q.r, q.U0, q.U, q.w, smem, rotate != 0)) {
+            if (q.method && threadIdx.x == 0) *q.method = 1;
             return;
         }
         __syncthreads();  // the LDS is reused below
     }
-    sym_top_eigvecs_block(G, n, r, U, w, scratch, scratch + (long)n * n, smem);
-    if (method && threadIdx.x == 0) *method = 0;
+    sym_top_eigvecs_block(q.G, q.n, q.r, q.U, q.w, q.scratch, q.scratch + (long)q.n * q.n, smem);
+    if (q.method && threadIdx.x == 0) *q.method = 0;
 }
 
-__global__ void k_sumsq(const float *__restrict__ X, long n, double *__restrict__ out) {
-    __shared__ double sh[256];
-    double s = 0.0;
-    for (long e = threadIdx.x; e < n; e += 256) s += (double)X[e] * (double)X[e];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) *out = s;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_norm2_blocks(const T *__restrict__ X, long n, double *__restrict__ part) {
+// ||X||^2 in FP64 (Kahan per thread), block partials.  Eight loads in flight: with one, 128^4
+// took 500 us (2.1 TB/s).
+__global__ __launch_bounds__(256) void k_norm2_blocks(const float *__restrict__ X, long n, double *__restrict__ part) {
     __shared__ double sh[256];
     double s = 0.0, c = 0.0;
-    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-        double x = (double)X[e];
-        double y = x * x - c, t = s + y;
-        c = (t - s) - y;
-        s = t;
+    const long st = (long)gridDim.x * 256;
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 8 * st) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = X[e + u * st < n ? e + u * st : e];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const double x = e + u * st < n ? (double)v[u] : 0.0;
+            const double y = x * x - c, t = s + y;
+            c = (t - s) - y;
+            s = t;
+        }
     }
     s = block_sum(s, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
@@ -165,12 +178,19 @@ static long eig_kernel_lds_doubles(int n) {
     return a > b ? a : b;
 }
 
-// scratch: 2 n^2 doubles.  try_sub: try the subspace path first, starting from U0 (or the
-// built-in block when U0 is null).  rotate = 0: an orthonormal basis of the top-r subspace is
-// enough (the subspace path may then skip its Rayleigh-Ritz rotation; w is not written then).
-static int top_eigvecs(const double *G, long n, long r, double *scratch, const float *U0, int try_sub, float *U,
-                       double *w, int *method, hipStream_t s, int rotate = 1) {
-    if (n < 1 || n > kEigMaxN || r < 1 || r > n) return record(TDX_ERR_ARG);
+// njobs <= 4 independent eigensolves in one launch; scratch: 2 n^2 doubles each.  try_sub: try the
+// subspace path first, starting from U0 (or the built-in block when U0 is null).  rotate = 0: an
+// orthonormal basis of the top-r subspace is enough (the subspace path may then skip its
+// Rayleigh-Ritz rotation; w is not written then).
+static int top_eigvecs(const EigJob *jobs, int njobs, int try_sub, hipStream_t s, int rotate = 1) {
+    EigJobs a{};
+    int nmax = 1;
+    for (int k = 0; k < njobs; ++k) {
+        const EigJob &q = jobs[k];
+        if (q.n < 1 || q.n > kEigMaxN || q.r < 1 || q.r > q.n) return record(TDX_ERR_ARG);
+        a.j[k] = q;
+        nmax = q.n > nmax ? q.n : nmax;
+    }
     static bool attr_set = false;
     if (!attr_set) {
         TDX_HIP(hipFuncSetAttribute((const void *)k_top_eigvecs, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -178,8 +198,7 @@ static int top_eigvecs(const double *G, long n, long r, double *scratch, const f
         attr_set = true;
     }
     const int sub = (try_sub && subspace_enabled()) ? 1 : 0;
-    k_top_eigvecs<<<1, kEigThreads, sizeof(double) * eig_kernel_lds_doubles((int)n), s>>>(
-        G, (int)n, (int)r, U0, sub, U, w, scratch, method, rotate);
+    k_top_eigvecs<<<njobs, kEigThreads, sizeof(double) * eig_kernel_lds_doubles(nmax), s>>>(a, sub, rotate);
     TDX_LAUNCH_CHECK();
     return TDX_OK;
 }
@@ -187,8 +206,8 @@ static int top_eigvecs(const double *G, long n, long r, double *scratch, const f
 static int ws_setup(TuckerWs &W, int order, const long *dims, const long *ranks) {
     W.gram_blocks = 1024;
     TDX_HIP(hipMalloc(&W.gram_part, sizeof(float) * (size_t)W.gram_blocks * kGramMaxN * kGramMaxN));
-    TDX_HIP(hipMalloc(&W.G, sizeof(double) * kGramMaxN * kGramMaxN));
-    TDX_HIP(hipMalloc(&W.Q, sizeof(double) * 2 * kGramMaxN * kGramMaxN));
+    TDX_HIP(hipMalloc(&W.G, sizeof(double) * 4 * kGramMaxN * kGramMaxN));
+    TDX_HIP(hipMalloc(&W.Q, sizeof(double) * 8 * kGramMaxN * kGramMaxN));
     TDX_HIP(hipMalloc(&W.scal, sizeof(double) * 2048));
     // largest intermediate of a TTM chain: the first contraction of the biggest mode
     long N = 1;
@@ -266,14 +285,22 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
     }
     // HOSVD init (only the spans matter when HOOI iterations follow: every later product
     // contracts U U^T, so the eigenvector rotation is left to the last iteration)
+    EigJob jobs[4];
     for (int m = 0; m < order; ++m) {
-        st = unfold_gram(Xs, xtype, order, dims, m, W, W.G, s);
-        if (!st) st = top_eigvecs(W.G, dims[m], ranks[m], W.Q, nullptr, 1, U[m], nullptr, nullptr, s, iters == 0);
+        double *G = W.G + (long)m * kGramMaxN * kGramMaxN;
+        st = unfold_gram(Xs, xtype, order, dims, m, W, G, s);
         if (st) return st;
+        jobs[m] = EigJob{G, (int)dims[m], (int)ranks[m], nullptr, U[m], nullptr, W.Q + 2L * m * kGramMaxN * kGramMaxN,
+                         nullptr};
     }
-    k_norm2_blocks<float><<<1024, 256, 0, s>>>(X, N, W.scal);
-    k_sum_to<<<1, 256, 0, s>>>(W.scal, 1024, W.scal + 1024);
-    TDX_LAUNCH_CHECK();
+    st = top_eigvecs(jobs, order, 1, s, iters == 0);
+    if (st) return st;
+    // ||X||^2 serves the error history only: a pass over X that a call without one does not make
+    if (relerr_hist) {
+        k_norm2_blocks<<<1024, 256, 0, s>>>(X, N, W.scal);
+        k_sum_to<<<1, 256, 0, s>>>(W.scal, 1024, W.scal + 1024);
+        TDX_LAUNCH_CHECK();
+    }
     double nx2 = 0.0;
     long nc = 1;
     for (int m = 0; m < order; ++m) nc *= ranks[m];
@@ -305,8 +332,8 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
                 if (!st) st = unfold_gram(Y, TDX_F32, order, ydims, n, W, W.G, s);
                 // warm start: the factor of the previous iteration spans nearly the same subspace;
                 // eigenvectors (ascending, sign convention) only in the last iteration
-                if (!st)
-                    st = top_eigvecs(W.G, dims[n], ranks[n], W.Q, U[n], 1, U[n], nullptr, nullptr, s, it == iters - 1);
+                const EigJob job{W.G, (int)dims[n], (int)ranks[n], U[n], U[n], nullptr, W.Q, nullptr};
+                if (!st) st = top_eigvecs(&job, 1, 1, s, it == iters - 1);
                 if (st) return st;
             }
         }
@@ -320,7 +347,7 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
             {
                 // ||core||^2: block partials (the first 1024 slots are free once ||X||^2 is summed)
                 const int nb = (int)(ceil_div(nc, 1024L) < 1024 ? ceil_div(nc, 1024L) : 1024);
-                k_norm2_blocks<float><<<nb, 256, 0, s>>>(core, nc, W.scal);
+                k_norm2_blocks<<<nb, 256, 0, s>>>(core, nc, W.scal);
                 k_sum_to<<<1, 256, 0, s>>>(W.scal, nb, W.scal + 1025);
             }
             double hv[2];
@@ -366,7 +393,8 @@ int tdx_sym_eig_topr_ex(const double *G, long n, long r, const float *U0, int fl
     int st = workspace(WS_MISC2, sizeof(double) * 2 * n * n + 256, &scr);
     if (st) return st;
     int *dmethod = (int *)((char *)scr + sizeof(double) * 2 * n * n);
-    st = top_eigvecs(G, n, r, (double *)scr, U0, (flags & TDX_EIG_TRY_SUBSPACE) ? 1 : 0, U, w, dmethod, stream());
+    const EigJob job{G, (int)n, (int)r, U0, U, w, (double *)scr, dmethod};
+    st = top_eigvecs(&job, 1, (flags & TDX_EIG_TRY_SUBSPACE) ? 1 : 0, stream());
     int hm = 0;
     if (!st) TDX_HIP(hipMemcpyAsync(&hm, dmethod, sizeof(int), hipMemcpyDeviceToHost, stream()));
     if (!st) TDX_HIP(hipStreamSynchronize(stream()));
