@@ -365,9 +365,9 @@ __global__ void k_ratio(const double *__restrict__ part, int nparts, double *__r
 //   Y[p + a*P + q*P*Ra] = sum_{i < In} U[a*lda + i*ldi] * X[p + i*P + q*P*In]
 // (reference ttm, src/ttm.cu:21,29,37, with lda = 1, ldi = d; transposed factor with
 //  lda = In, ldi = 1; Tucker expansion core -> tensor with lda = 1, ldi = I).
+int ttm_mfma_launch(const void *X, long P, long In, long Q, const float *U, long lda, long ldi, long Ra, float *Y,
+                    hipStream_t s);
 // X is FP32 (xtype TDX_F32) or BF16 bit patterns (TDX_BF16)
-int ttm_mfma_launch(const void *X, int xtype, long P, long In, long Q, const float *U, long lda, long ldi, long Ra,
-                    float *Y, hipStream_t s);
 int ttm_any_launch(const void *X, int xtype, long P, long In, long Q, const float *U, long lda, long ldi, long Ra,
                    float *Y, hipStream_t s);
 
@@ -376,8 +376,8 @@ int ttm_generic_t(const void *X, int xtype, int order, const long *dims, int mod
     long P = 1, Q = 1;
     for (int m = 0; m < mode; ++m) P *= dims[m];
     for (int m = mode + 1; m < order; ++m) Q *= dims[m];
-    // the register kernel for the shapes it covers (ttm.hip), the general one otherwise
-    const int mf = ttm_mfma_launch(X, xtype, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
+    // BF16: the register kernel for the shapes it covers (ttm.hip); the general one otherwise
+    const int mf = xtype != TDX_BF16 ? 0 : ttm_mfma_launch(X, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
     if (mf < 0) return record(TDX_ERR_HIP);
     if (mf > 0) return TDX_OK;
     return ttm_any_launch(X, xtype, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);

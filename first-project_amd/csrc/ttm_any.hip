@@ -1,17 +1,21 @@
-// ttm_any.hip -- mode-n tensor-times-matrix of any shape and alignment on FP32 MFMA:
+// ttm_any.hip -- mode-n tensor-times-matrix through LDS on FP32 MFMA, any shape and alignment:
 //   Y[p, a, q] = sum_i X[p, i, q] U(i, a),  U(i, a) = U[i * ldi + a * lda],
 // X the (P, In, Q) view of an FP32 or BF16 tensor (BF16: U rounded to BF16, as on the other
-// path), Y the (P, Ra, Q) FP32 result.  Modes longer than 128, ranks above 64 (32 in FP32) and
-// extents without whole vectors come here; src/ttm.cu:21,29,37 takes any of them.
+// path), Y the (P, Ra, Q) FP32 result.  All FP32 tensors come here, and BF16 ones whose mode is
+// longer than 128, whose rank is above 64 or whose extents hold no whole vectors
+// (src/ttm.cu:21,29,37 takes any of them).
 //
 // A GEMM of the fibres k = p + P q (rows) with U: a workgroup owns TM fibres x up to 64 columns
 // and walks i in steps of 64.  The TM x 64 tile of X and the 64 x 16 NB block of U are staged in
 // LDS (rows of 68 floats: a lane's 4 consecutive i are one 16-byte operand read, 16 rows in
 // distinct banks) while the next step's elements are in flight in registers; the result leaves
 // through LDS in whole lines.  X is read element by element, 64 lanes on 256 contiguous bytes
-// (along p, or along i when P = 1), so nothing has to be aligned.
-// Bound by HBM: 512 x 384 x 256 FP32 with 48 columns moves 221-252 MB a mode (48-55 us at the
-// 4.6 TB/s of a large copy; the products 32 us).
+// (along p, or along i when P = 1), so nothing has to be aligned; with whole vectors (VEC) a
+// thread loads 16 bytes, along p four fibres of four i transposed in registers.
+// Bound by HBM.  512 x 384 x 256 FP32 with 48 columns (221-252 MB a mode, 48-55 us at the 4.6 TB/s
+// of a large copy): 880-1450 us with a thread per output, 81-89 us element by element, 68-75 us
+// with vectors.  128^4 to 32 columns (1.34 GB, 291 us): 293-315 us, 382 us with U and four steps
+// of X held in one wave's registers; its later, small products 10-84 us against 27-136.
 #include "common.hpp"
 
 namespace tdx {
@@ -33,8 +37,9 @@ __device__ __forceinline__ float ta_f32(uint16_t v) { return __uint_as_float((ui
 __device__ __forceinline__ float ta_coef(float u, float) { return u; }
 __device__ __forceinline__ float ta_coef(float u, uint16_t) { return __uint_as_float((uint32_t)f32_to_bf16_bits(u) << 16); }
 
-// PC: P > 1 (fibres contiguous along p); NB column blocks of 16; RPW row blocks of 16 per wave
-template <typename ET, bool PC, int NB, int RPW>
+// PC: P > 1 (fibres contiguous along p); NB column blocks of 16; RPW row blocks of 16 per wave;
+// VEC (FP32, 16-byte aligned, P % 4 == 0 or, for P = 1, In % 4 == 0): 16-byte loads of X
+template <typename ET, bool PC, int NB, int RPW, bool VEC>
 __global__ __launch_bounds__(256, 2) void k_ttm_any(TaArgs a) {
     constexpr int TM = 64 * RPW, NU = TM / 16, NL = TM / 4, NC = 4 * NB, CW = 16 * NB;
     __shared__ __attribute__((aligned(16))) float xs[TM * kTaLd];
@@ -51,12 +56,15 @@ __global__ __launch_bounds__(256, 2) void k_ttm_any(TaArgs a) {
     // this thread's fibre (PC: row tid % TM of the tile, the same for every load)
     long xrow = 0;
     if constexpr (PC) {
-        const long r = min(row0 + tid % TM, rows - 1), q = r / P;
+        // (VEC: the first of the thread's four fibres, tid % (TM / 4); rows % 4 == 0, and a quad
+        // lies in one run of p)
+        const long r = VEC ? min(row0 + 4 * (tid % (TM / 4)), rows - 4) : min(row0 + tid % TM, rows - 1), q = r / P;
         xrow = (r - q * P) + q * P * In;
     }
     // U: lanes along i where it is contiguous there, else along the columns
     const bool ui = a.ldi == 1;
-    ET xv[NL];
+    ET xv[VEC ? 1 : NL];
+    float4 xq[VEC ? NL / 4 : 1];
     float uv[NC];
     auto load = [&](long i0) {
 #pragma unroll
@@ -68,7 +76,21 @@ __global__ __launch_bounds__(256, 2) void k_ttm_any(TaArgs a) {
                 const long col = min((long)col0 + (ui ? wave * NC + 4 * u + c : e % CW), a.Ra - 1);
                 uv[4 * u + c] = U[min(i, In - 1) * a.ldi + col * a.lda];
             }
-        if constexpr (PC) {
+        if constexpr (VEC && PC) {
+            // 4 fibres x 4 consecutive i a task, RPW tasks a thread
+#pragma unroll
+            for (int u = 0; u < RPW; ++u) {
+                const int kq = (tid + 256 * u) / (TM / 4);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    xq[4 * u + c] = ld_stream(reinterpret_cast<const float4 *>(X + xrow + min(i0 + 4 * kq + c, In - 1) * P));
+            }
+        } else if constexpr (VEC) {
+            const ET *xp = X + min(i0 + 4 * (tid & 15), In - 4);
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                xq[u] = ld_stream(reinterpret_cast<const float4 *>(xp + min(row0 + (tid >> 4) + 16 * u, rows - 1) * In));
+        } else if constexpr (PC) {
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 const int kq = __builtin_amdgcn_readfirstlane((tid + 256 * u) / TM);
@@ -92,7 +114,29 @@ __global__ __launch_bounds__(256, 2) void k_ttm_any(TaArgs a) {
     load(0);
     for (long i0 = 0; i0 < In; i0 += kTaK) {
         __syncthreads();
-        if constexpr (PC) {
+        if constexpr (VEC && PC) {
+#pragma unroll
+            for (int u = 0; u < RPW; ++u) {
+                const int kq = (tid + 256 * u) / (TM / 4);
+                float v[4][4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const bool on = i0 + 4 * kq + c < In;
+                    const float4 w = xq[4 * u + c];
+                    v[0][c] = on ? w.x : 0.f, v[1][c] = on ? w.y : 0.f, v[2][c] = on ? w.z : 0.f, v[3][c] = on ? w.w : 0.f;
+                }
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    *reinterpret_cast<float4 *>(xs + (4 * (tid % (TM / 4)) + t) * kTaLd + 4 * kq) =
+                        float4{v[t][0], v[t][1], v[t][2], v[t][3]};
+            }
+        } else if constexpr (VEC) {
+            const bool on = i0 + 4 * (tid & 15) < In;
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                *reinterpret_cast<float4 *>(xs + ((tid >> 4) + 16 * u) * kTaLd + 4 * (tid & 15)) =
+                    on ? xq[u] : float4{0.f, 0.f, 0.f, 0.f};
+        } else if constexpr (PC) {
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 const int e = tid + 256 * u, kq = e / TM;
@@ -184,13 +228,13 @@ __global__ __launch_bounds__(256, 2) void k_ttm_any(TaArgs a) {
     }
 }
 
-template <typename ET, bool PC, int RPW>
+template <typename ET, bool PC, int RPW, bool VEC>
 static void ta_launch(const TaArgs &a, int nb, unsigned grid, hipStream_t s) {
     switch (nb) {
-        case 1: k_ttm_any<ET, PC, 1, RPW><<<grid, 256, 0, s>>>(a); break;
-        case 2: k_ttm_any<ET, PC, 2, RPW><<<grid, 256, 0, s>>>(a); break;
-        case 3: k_ttm_any<ET, PC, 3, RPW><<<grid, 256, 0, s>>>(a); break;
-        default: k_ttm_any<ET, PC, 4, RPW><<<grid, 256, 0, s>>>(a); break;
+        case 1: k_ttm_any<ET, PC, 1, RPW, VEC><<<grid, 256, 0, s>>>(a); break;
+        case 2: k_ttm_any<ET, PC, 2, RPW, VEC><<<grid, 256, 0, s>>>(a); break;
+        case 3: k_ttm_any<ET, PC, 3, RPW, VEC><<<grid, 256, 0, s>>>(a); break;
+        default: k_ttm_any<ET, PC, 4, RPW, VEC><<<grid, 256, 0, s>>>(a); break;
     }
 }
 
@@ -201,14 +245,16 @@ int ttm_any_launch(const void *X, int xtype, long P, long In, long Q, const floa
     // 128 fibres a workgroup share a U block; 64 where that leaves compute units idle
     const bool wide = ceil_div(a.rows, 128L) * a.ncb >= device_cus();
     const unsigned grid = (unsigned)(ceil_div(a.rows, wide ? 128L : 64L) * a.ncb);
-    const bool pc = P > 1;
-    if (xtype == TDX_BF16) {
-        if (pc) wide ? ta_launch<uint16_t, true, 2>(a, nb, grid, s) : ta_launch<uint16_t, true, 1>(a, nb, grid, s);
-        else wide ? ta_launch<uint16_t, false, 2>(a, nb, grid, s) : ta_launch<uint16_t, false, 1>(a, nb, grid, s);
-    } else {
-        if (pc) wide ? ta_launch<float, true, 2>(a, nb, grid, s) : ta_launch<float, true, 1>(a, nb, grid, s);
-        else wide ? ta_launch<float, false, 2>(a, nb, grid, s) : ta_launch<float, false, 1>(a, nb, grid, s);
-    }
+    const bool pc = P > 1, vec = xtype == TDX_F32 && ((uintptr_t)X & 15) == 0 && (pc ? P : In) % 4 == 0;
+#define TDX_TA(ET_, VEC_)                                                                                             \
+    do {                                                                                                              \
+        if (pc) wide ? ta_launch<ET_, true, 2, VEC_>(a, nb, grid, s) : ta_launch<ET_, true, 1, VEC_>(a, nb, grid, s); \
+        else wide ? ta_launch<ET_, false, 2, VEC_>(a, nb, grid, s) : ta_launch<ET_, false, 1, VEC_>(a, nb, grid, s);  \
+    } while (0)
+    if (xtype == TDX_BF16) TDX_TA(uint16_t, false);
+    else if (vec) TDX_TA(float, true);
+    else TDX_TA(float, false);
+#undef TDX_TA
     TDX_LAUNCH_CHECK();
     return TDX_OK;
 }
