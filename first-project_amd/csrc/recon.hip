@@ -75,7 +75,6 @@ __global__ __launch_bounds__(256, 2) void k_cp_model(FacArgs f, float *__restric
                 if (r0 + 4 * k + lg >= R) aop[t][k] = 0.0f;
         }
     };
-    if (!BIG) load_a(0);
     // this lane's fibre of the 64 and its digits
     long c = 64 * t0 + lane;
     long i1 = c % D1, i2 = (c / D1) % D2, i3 = c / D1 / D2;
@@ -120,7 +119,10 @@ __global__ __launch_bounds__(256, 2) void k_cp_model(FacArgs f, float *__restric
         }
     };
     const bool rows = row0 + 64 <= I;  // uniform
-    if (!BIG && t0 < t1) load_w(0);
+    if (!BIG && t0 < t1) {
+        load_w(0);
+        load_a(0);
+    }
     for (long tl = t0; tl < t1; ++tl) {
         __syncthreads();  // every wave is done with the previous W
         if constexpr (BIG) {
@@ -397,8 +399,8 @@ static long model_row_waves(long I0) {
         if (6 * (ceil_div(nrc, rw) * rw - nrc) <= nrc) return rw;
     return 1;
 }
-// the most workgroups such a launch has
-static long model_blocks(long I0) { return kModelBlocks + ceil_div(ceil_div(I0, 64L), model_row_waves(I0)); }
+// the most workgroups such a launch has (a small one has at most 1024)
+static long model_blocks(long I0) { return kModelBlocks + ceil_div(I0, 64L); }
 
 static int fac_args(FacArgs &f, int order, const long *dims, const float *const *U, long R) {
     if (R > 256) return record(TDX_ERR_UNSUPPORTED);
@@ -417,10 +419,11 @@ static int cp_model_launch(int order, const long *dims, const float *const *U, l
     FacArgs f{};
     int st = fac_args(f, order, dims, U, R);
     if (st) return st;
-    // about kModelBlocks workgroups, of at least two tiles of 64 fibres
-    const long rw = model_row_waves(dims[0]), nrg = ceil_div(ceil_div(dims[0], 64L), rw);
-    const long ntile = ceil_div(f.dims[1] * f.dims[2] * f.dims[3], 64L);
-    const long tper = std::max(2L, ceil_div(nrg * ntile, kModelBlocks));
+    // about kModelBlocks workgroups; one row block each where that leaves compute units idle
+    // (512 x 16 x 8: 9.3 us in 4 workgroups of four row blocks, 6.1 in 16 of one)
+    const long ntile = ceil_div(f.dims[1] * f.dims[2] * f.dims[3], 64L), nrc = ceil_div(dims[0], 64L);
+    const long rw = nrc * ntile <= device_cus() ? 1 : model_row_waves(dims[0]), nrg = ceil_div(nrc, rw);
+    const long tper = std::max(1L, ceil_div(nrg * ntile, kModelBlocks));
     const int grid = (int)(nrg * ceil_div(ntile, tper));
     if (blocks) *blocks = grid;
     const int ks = R <= 16 ? 4 : R <= 32 ? 8 : R <= 48 ? 12 : 16;
