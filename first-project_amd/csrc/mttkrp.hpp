@@ -45,10 +45,14 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
 int mttkrp_launch(const MttkrpPlan &p, const void *X, const float *const *panels,
                   const float *row_scale, float *partial, hipStream_t s, const int *skip = nullptr);
 
-// the LDS-staged kernel (mttkrp_lds.hip)
+// the LDS-staged kernel (mttkrp_lds.hip; BF16 and FP8 storage)
 bool mttkrp_lds_covers(int order, int mode, long rank, long In, int dtype);
 int mttkrp_lds_launch(const MttkrpPlan &p, const void *X, const float *const *panels, const float *row_scale,
                       float *partial, hipStream_t s, const int *skip);
+
+// FP32 storage on the plan of the LDS-staged kernel (mttkrp_f32.hip)
+int mttkrp_f32_launch(const MttkrpPlan &p, const void *X, const float *const *panels, float *partial, hipStream_t s,
+                      const int *skip);
 
 // the kernel for the remaining shapes and alignments (mttkrp_any.hip): completes a plan whose
 // order, extents, mode, storage and rank are set; partial rows are exactly the output rows

@@ -1,18 +1,19 @@
-// mttkrp_lds.hip -- fused MTTKRP with the tensor tile and the Khatri-Rao block staged in
-// LDS.  For an output mode n > 0 the contraction's fast index f is the contiguous mode 0;
-// for n = 0 (TR) it is mode 1 and the tile is transposed on its way into LDS.
+// mttkrp_lds.hip -- fused MTTKRP of a BF16 or FP8 tensor with the tensor tile and the Khatri-Rao
+// block staged in LDS (FP32 storage: mttkrp_f32.hip).  For an output mode n > 0 the contraction's
+// fast index f is the contiguous mode 0; for n = 0 (TR) it is mode 1 and the tile is transposed on
+// its way into LDS.
 //
 // M[i_n, r] = sum_{i_f, slow} X[...] * P_f[i_f, r] * w_slow[r],
 // w_slow[r] = prod over the other contracted modes of their factor rows.
 //
 // Work of a workgroup: 128 consecutive output rows and a range of slow indices; for every
-// chunk of KB consecutive i_f (KB = 128 BF16/FP8, 64 FP32) it walks its slow indices:
+// chunk of KB = 128 consecutive i_f it walks its slow indices:
 //   * n > 0: the (128 x KB) tensor tile is read with 16-byte loads, 16 (FP8: 8) lanes per
 //     row, so each row contributes whole 128-byte lines (256 bytes, FP8 128) per step --
 //     output rows are far apart in memory (the stride of mode n), and half-line accesses
 //     spread over time were re-fetched;
 //   * n = 0 (TR): output rows are contiguous; a thread loads 8 consecutive i_1 of 8 rows
-//     (4 rows for FP32) with 16-byte (FP8 8-byte) loads, 16 threads covering 256 contiguous
+//     with 16-byte (FP8 8-byte) loads, 16 threads covering 256 contiguous
 //     bytes per i_1, and transposes the block in registers so LDS holds [row][k] as above.
 //     Row RL g + t of the tile (row group g) sits in LDS row RG t + g, so the 16-byte stores
 //     of a wave go to consecutive LDS rows (no bank conflicts); the MFMA rows follow the LDS
@@ -25,8 +26,8 @@
 //   * the KB x Rp Khatri-Rao block  P_0[chunk, :] * w_slow  is formed once per step in LDS
 //     for all four waves (each thread keeps its 32 panel values of the chunk in registers
 //     for the whole slow loop);
-//   * each wave multiplies its 32 rows by the block (v_mfma_f32_16x16x32_bf16; FP32
-//     storage v_mfma_f32_16x16x4_f32), accumulating in FP32;
+//   * each wave multiplies its 32 rows by the block (v_mfma_f32_16x16x32_bf16), accumulating in
+//     FP32;
 //   * the tiles of the next two slow indices are in flight in two register buffers while the
 //     current one is multiplied (two steps in flight per workgroup, two workgroups per CU);
 //   * a workgroup's work is one i_0 chunk (rarely a few) times a range of slow indices, so
@@ -40,7 +41,6 @@ namespace tdx {
 
 typedef float lf32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 lbf16x8 __attribute__((ext_vector_type(8)));
-typedef float lf32x2 __attribute__((ext_vector_type(2)));
 
 struct LArgs {
     const void *X;
@@ -74,8 +74,6 @@ __device__ __forceinline__ uint2 lfp8x4_to_bf16(uint32_t q) {
 }
 
 template <int ST> struct LTile;
-// FP32: KB = 64, a row is 256 bytes = 16 lanes x 16 bytes; LDS keeps FP32
-template <> struct LTile<0> { static constexpr int KB = 64, LPR = 16, PAD = 4; typedef float E; };
 // BF16: KB = 128, 256 bytes per row = 16 lanes x 16 bytes; LDS keeps BF16
 template <> struct LTile<1> { static constexpr int KB = 128, LPR = 16, PAD = 8; typedef uint16_t E; };
 // FP8: KB = 128, 128 bytes per row = 8 lanes x 16 bytes; widened to BF16 in LDS
@@ -91,13 +89,9 @@ __device__ __forceinline__ uint32_t lhalf(const uint4 &v, int t) {
     const uint32_t w = (t >> 1) == 0 ? v.x : (t >> 1) == 1 ? v.y : (t >> 1) == 2 ? v.z : v.w;
     return (t & 1) ? (w >> 16) : (w & 0xffffu);
 }
-__device__ __forceinline__ uint32_t lword(const uint4 &v, int t) {
-    return t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
-}
-
 // TR (n = 0) load geometry: a load covers RL rows of one i_1; RG row groups x KG k groups
 template <int ST> struct LTr {
-    static constexpr int RL = (ST == 0) ? 4 : 8;
+    static constexpr int RL = 8;
     static constexpr int RG = 128 / RL;
     static constexpr int KG = 256 / RG;
     typedef typename std::conditional<ST == 2, uint2, uint4>::type V;
@@ -160,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
     // F8T: this thread loads rows 16 (tid % 8) .. + 15 (16 bytes) of fast index tid / 8 + 32 p
     // (8 lanes read one whole 128-byte line per fast index; the planner requires In % 16 == 0).
     const int lrow = F8T ? 16 * (tid % 8) : TR ? LTr<ST>::RL * (tid % LTr<ST>::RG) : tid / LPR;
-    const int lcol = F8T ? tid / 8 : TR ? 8 * (tid / LTr<ST>::RG) : (tid % LPR) * ((ST == 0) ? 4 : (ST == 1) ? 8 : 16);
+    const int lcol = F8T ? tid / 8 : TR ? 8 * (tid / LTr<ST>::RG) : (tid % LPR) * ((ST == 1) ? 8 : 16);
     long roff[NPASS];
     bool rok[NPASS];
 #pragma unroll
@@ -229,8 +223,7 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
             const bool in = rok[p] && fok;
             const long e = off + roff[p] + (fok ? f : 0) * sf;
             const LE *src;
-            if constexpr (ST == 0) src = reinterpret_cast<const LE *>(reinterpret_cast<const float *>(a.X) + e);
-            else if constexpr (ST == 1) src = reinterpret_cast<const LE *>(reinterpret_cast<const uint16_t *>(a.X) + e);
+            if constexpr (ST == 1) src = reinterpret_cast<const LE *>(reinterpret_cast<const uint16_t *>(a.X) + e);
             else src = reinterpret_cast<const LE *>(reinterpret_cast<const uint8_t *>(a.X) + e);
             b.x[p] = ld_stream(reinterpret_cast<const VT *>(src));
             b.ok |= (uint32_t)in << p;
@@ -255,36 +248,23 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
                 *reinterpret_cast<uint4 *>(x8 + k * 128 + 16 * ((lrow >> 4) ^ ((k >> 1) & 7))) = v;
             }
         } else if constexpr (TR) {
-            if constexpr (ST == 0) {
-                // 8 loads of 4 rows -> tile rows lrow + t, 8 fast indices each (two 16-byte stores)
-                uint4 v[8];
+            // 8 loads of 8 rows (BF16, FP8 widened) -> 8x8 transpose of 16-bit elements
+            uint4 v[8];
 #pragma unroll
-                for (int p = 0; p < 8; ++p) v[p] = (!MASKED || ((b.ok >> p) & 1u)) ? b.x[p] : uint4{0u, 0u, 0u, 0u};
+            for (int p = 0; p < 8; ++p) {
+                uint4 u;
+                if constexpr (ST == 2) u = lfp8x8_to_bf16(b.x[p]);
+                else u = b.x[p];
+                v[p] = (!MASKED || ((b.ok >> p) & 1u)) ? u : uint4{0u, 0u, 0u, 0u};
+            }
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    LE *dst = xs + (LTr<ST>::RG * t + tid % LTr<ST>::RG) * XLD + lcol;
-                    *reinterpret_cast<uint4 *>(dst) = uint4{lword(v[0], t), lword(v[1], t), lword(v[2], t), lword(v[3], t)};
-                    *reinterpret_cast<uint4 *>(dst + 4) = uint4{lword(v[4], t), lword(v[5], t), lword(v[6], t), lword(v[7], t)};
-                }
-            } else {
-                // 8 loads of 8 rows (BF16, FP8 widened) -> 8x8 transpose of 16-bit elements
-                uint4 v[8];
-#pragma unroll
-                for (int p = 0; p < 8; ++p) {
-                    uint4 u;
-                    if constexpr (ST == 2) u = lfp8x8_to_bf16(b.x[p]);
-                    else u = b.x[p];
-                    v[p] = (!MASKED || ((b.ok >> p) & 1u)) ? u : uint4{0u, 0u, 0u, 0u};
-                }
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    uint4 o;
-                    o.x = lhalf(v[0], t) | (lhalf(v[1], t) << 16);
-                    o.y = lhalf(v[2], t) | (lhalf(v[3], t) << 16);
-                    o.z = lhalf(v[4], t) | (lhalf(v[5], t) << 16);
-                    o.w = lhalf(v[6], t) | (lhalf(v[7], t) << 16);
-                    *reinterpret_cast<uint4 *>(xs + (LTr<ST>::RG * t + tid % LTr<ST>::RG) * XLD + lcol) = o;
-                }
+            for (int t = 0; t < 8; ++t) {
+                uint4 o;
+                o.x = lhalf(v[0], t) | (lhalf(v[1], t) << 16);
+                o.y = lhalf(v[2], t) | (lhalf(v[3], t) << 16);
+                o.z = lhalf(v[4], t) | (lhalf(v[5], t) << 16);
+                o.w = lhalf(v[6], t) | (lhalf(v[7], t) << 16);
+                *reinterpret_cast<uint4 *>(xs + (LTr<ST>::RG * t + tid % LTr<ST>::RG) * XLD + lcol) = o;
             }
         } else {
 #pragma unroll
@@ -314,12 +294,7 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
         if (kr_on) {
             const float w = (a.nslow > 1) ? b.wa * b.wb : b.wa;
             LE *dst = bs + kr_c * XLD + kr_k0;
-            if constexpr (ST == 0) {
-#pragma unroll
-                for (int q = 0; q < KB / 16; ++q)
-                    *reinterpret_cast<float4 *>(dst + 4 * q) =
-                        float4{pc[4 * q] * w, pc[4 * q + 1] * w, pc[4 * q + 2] * w, pc[4 * q + 3] * w};
-            } else if constexpr (SPLIT) {
+            if constexpr (SPLIT) {
 #pragma unroll
                 for (int q = 0; q < KB / 32; ++q) {
                     uint32_t hi[4], lo[4];
@@ -347,72 +322,49 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
         __builtin_amdgcn_sched_barrier(0);  // the refill's loads stay ahead of the MFMAs
         if (!valid) return;
         // MFMAs: this wave's rows 32 wave + 16 rb + (lane % 16)
-        if constexpr (ST == 0) {
 #pragma unroll
-            for (int q = 0; q < KB / 16; ++q) {
-                float4 av[2], bv[NB];
+        for (int q = 0; q < KB / 32; ++q) {
+            lbf16x8 av[2], bv[NB];
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb)
-                    av[rb] = *reinterpret_cast<const float4 *>(xs + (32 * wave + 16 * rb + lm) * XLD + 16 * q + 4 * lg);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    bv[nb] = *reinterpret_cast<const float4 *>(bs + (16 * nb + lm) * XLD + 16 * q + 4 * lg);
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            const float x = c == 0 ? av[rb].x : c == 1 ? av[rb].y : c == 2 ? av[rb].z : av[rb].w;
-                            const float y = c == 0 ? bv[nb].x : c == 1 ? bv[nb].y : c == 2 ? bv[nb].z : bv[nb].w;
-                            acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc[rb][nb], 0, 0, 0);
-                        }
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < KB / 32; ++q) {
-                lbf16x8 av[2], bv[NB];
-#pragma unroll
-                for (int rb = 0; rb < 2; ++rb) {
-                    if constexpr (F8T) {
-                        // ds_read_b64_tr_b8: in each 16-lane group, lane l receives byte l & 7
-                        // of the 8-byte pieces addressed by lanes 2j + (l >> 3), j = 0..7.  Lane
-                        // 2j + h of group lg addresses fast index k = 32 q + 8 lg + j, rows
-                        // 32 wave + 16 rb + 8 h .. + 7, so lane (lm, lg) gets X(row lm, k =
-                        // 32 q + 8 lg + j) for j = 0..7: the A operand, widened here to BF16.
-                        const int k = 32 * q + 8 * lg + (lm >> 1);
-                        const int gr = 2 * wave + rb;  // 16-row granule
-                        const unsigned char *src = reinterpret_cast<const unsigned char *>(xs) + k * 128 +
-                                                   16 * (gr ^ ((k >> 1) & 7)) + 8 * (lm & 1);
-                        typedef int lv2i __attribute__((ext_vector_type(2)));
-                        const lv2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                            (__attribute__((address_space(3))) lv2i *)(src));
-                        av[rb] = __builtin_bit_cast(lbf16x8, lfp8x8_to_bf16(uint2{(uint32_t)w.x, (uint32_t)w.y}));
-                    } else {
-                        av[rb] = __builtin_bit_cast(
-                            lbf16x8, *reinterpret_cast<const uint4 *>(xs + (32 * wave + 16 * rb + lm) * XLD + 32 * q + 8 * lg));
-                    }
+            for (int rb = 0; rb < 2; ++rb) {
+                if constexpr (F8T) {
+                    // ds_read_b64_tr_b8: in each 16-lane group, lane l receives byte l & 7
+                    // of the 8-byte pieces addressed by lanes 2j + (l >> 3), j = 0..7.  Lane
+                    // 2j + h of group lg addresses fast index k = 32 q + 8 lg + j, rows
+                    // 32 wave + 16 rb + 8 h .. + 7, so lane (lm, lg) gets X(row lm, k =
+                    // 32 q + 8 lg + j) for j = 0..7: the A operand, widened here to BF16.
+                    const int k = 32 * q + 8 * lg + (lm >> 1);
+                    const int gr = 2 * wave + rb;  // 16-row granule
+                    const unsigned char *src = reinterpret_cast<const unsigned char *>(xs) + k * 128 +
+                                               16 * (gr ^ ((k >> 1) & 7)) + 8 * (lm & 1);
+                    typedef int lv2i __attribute__((ext_vector_type(2)));
+                    const lv2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                        (__attribute__((address_space(3))) lv2i *)(src));
+                    av[rb] = __builtin_bit_cast(lbf16x8, lfp8x8_to_bf16(uint2{(uint32_t)w.x, (uint32_t)w.y}));
+                } else {
+                    av[rb] = __builtin_bit_cast(
+                        lbf16x8, *reinterpret_cast<const uint4 *>(xs + (32 * wave + 16 * rb + lm) * XLD + 32 * q + 8 * lg));
                 }
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                bv[nb] = __builtin_bit_cast(
+                    lbf16x8, *reinterpret_cast<const uint4 *>(bs + (16 * nb + lm) * XLD + 32 * q + 8 * lg));
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
-                    bv[nb] = __builtin_bit_cast(
-                        lbf16x8, *reinterpret_cast<const uint4 *>(bs + (16 * nb + lm) * XLD + 32 * q + 8 * lg));
+                    acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rb], bv[nb], acc[rb][nb], 0, 0, 0);
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    bv[nb] = __builtin_bit_cast(lbf16x8, *reinterpret_cast<const uint4 *>(
+                                                             bs + Rp * XLD + (16 * nb + lm) * XLD + 32 * q + 8 * lg));
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
                         acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rb], bv[nb], acc[rb][nb], 0, 0, 0);
-                if constexpr (SPLIT) {
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        bv[nb] = __builtin_bit_cast(lbf16x8, *reinterpret_cast<const uint4 *>(
-                                                                 bs + Rp * XLD + (16 * nb + lm) * XLD + 32 * q + 8 * lg));
-#pragma unroll
-                    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb)
-                            acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rb], bv[nb], acc[rb][nb], 0, 0, 0);
-                }
             }
         }
     };
@@ -460,8 +412,8 @@ __global__ __launch_bounds__(256, 2) void k_mttkrp_lds(LArgs a) {
         }
 }
 
-// covered for rank <= 64 and orders 3 and 4 (at most two slow modes); mode 0 needs whole
-// row groups (In a multiple of 4 rows for FP32, 8 for BF16, 16 for FP8)
+// (and mttkrp_f32.hip) covered for rank <= 64 and orders 3 and 4 (at most two slow modes); mode 0
+// needs whole row groups (In a multiple of 4 rows for FP32, 8 for BF16, 16 for FP8)
 bool mttkrp_lds_covers(int order, int mode, long rank, long In, int dtype) {
     if (rank > 64 || order < 3 || order > 4) return false;
     if (mode == 0) return In % ((dtype == TDX_F32) ? 4 : (dtype == TDX_FP8_E4M3) ? 16 : 8) == 0;
@@ -500,7 +452,7 @@ int mttkrp_lds_launch(const MttkrpPlan &p, const void *X, const float *const *pa
     for (int m = 1; m < p.order; ++m)
         if (m != p.mode && m != fm) a.slow[a.nslow++] = m;
     const int grid = p.rowtiles * p.nsplit;
-    const int stt = (p.dtype == TDX_F32) ? 0 : (p.dtype == TDX_BF16) ? 1 : 2;
+    const int stt = (p.dtype == TDX_BF16) ? 1 : 2;
 #define TDX_LDS_LAUNCH(ST_, TR_, SP_)                                                  \
     switch (p.Rp / 16) {                                                               \
         case 1: k_mttkrp_lds<ST_, 1, TR_, SP_><<<grid, 256, 0, s>>>(a); break;         \
@@ -508,15 +460,13 @@ int mttkrp_lds_launch(const MttkrpPlan &p, const void *X, const float *const *pa
         case 3: k_mttkrp_lds<ST_, 3, TR_, SP_><<<grid, 256, 0, s>>>(a); break;         \
         default: k_mttkrp_lds<ST_, 4, TR_, SP_><<<grid, 256, 0, s>>>(a); break;        \
     }
-    if (p.split && stt != 1) return record(TDX_ERR_UNSUPPORTED);
+    if (p.dtype == TDX_F32 || (p.split && stt != 1)) return record(TDX_ERR_UNSUPPORTED);
     if (p.mode == 0) {
-        if (stt == 0) { TDX_LDS_LAUNCH(0, true, false) }
-        else if (stt == 1 && p.split) { TDX_LDS_LAUNCH(1, true, true) }
+        if (stt == 1 && p.split) { TDX_LDS_LAUNCH(1, true, true) }
         else if (stt == 1) { TDX_LDS_LAUNCH(1, true, false) }
         else { TDX_LDS_LAUNCH(2, true, false) }
     } else {
-        if (stt == 0) { TDX_LDS_LAUNCH(0, false, false) }
-        else if (stt == 1 && p.split) { TDX_LDS_LAUNCH(1, false, true) }
+        if (stt == 1 && p.split) { TDX_LDS_LAUNCH(1, false, true) }
         else if (stt == 1) { TDX_LDS_LAUNCH(1, false, false) }
         else { TDX_LDS_LAUNCH(2, false, false) }
     }
