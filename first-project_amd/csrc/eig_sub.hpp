@@ -13,7 +13,7 @@
 // nearly dependent columns.  Every product (A V, V^T Z, V S, X^T X, X M, V W) runs on FP64
 // MFMA (v_mfma_f64_16x16x4f64: exact products, FP64 accumulation), with A held in registers
 // for the whole call; the Cholesky factorisation and triangular inverse run in one wave's
-// registers; the Jacobi rounds take two barriers each.
+// registers; the Jacobi rounds take one barrier each.
 //
 // The result is accepted only under a certificate that the theta are the r LARGEST
 // eigenvalues, valid for any symmetric A: with orthonormal V and residual bound e = rho +
@@ -30,7 +30,8 @@ namespace tdx {
 
 static constexpr int kSubMaxR = 32;
 static constexpr int kSubRows = kEigMaxN;     // V and Z always hold 128 rows (zero past n)
-static constexpr int kSubLd = kSubMaxR;       // row stride of the n x r blocks V, Z
+// row stride of the n x r blocks V, Z: 16 rows read down a column (sub_xm) hit distinct LDS banks
+static constexpr int kSubLd = kSubMaxR + 4;
 static constexpr int kSubHld = kSubMaxR + 1;  // row stride of the r x r blocks H, W, S, M
 static constexpr int kSubMaxIt = 12;
 
@@ -69,6 +70,41 @@ __device__ inline double sub_blk_sum(double v, double *red) {
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// sums of two values at once (red: 8 doubles)
+__device__ inline void sub_blk_sum2(double &u, double &v, double *red) {
+    u = wave_sum_f64(u);
+    v = wave_sum_f64(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = u;
+        red[4 + (threadIdx.x >> 6)] = v;
+    }
+    __syncthreads();
+    u = (red[0] + red[1]) + (red[2] + red[3]);
+    v = (red[4] + red[5]) + (red[6] + red[7]);
+}
+
+// The Jacobi rotation of the symmetric 2 x 2 block (app, apq; apq, aqq): t = sign(tau) / (|tau| +
+// sqrt(tau^2 + 1)), c = 1 / sqrt(t^2 + 1), s = t c, with the hardware reciprocal / reciprocal-root
+// estimates refined by two Newton steps (full FP64 precision; c^2 + s^2 = 1 to rounding).  The
+// identity for apq = 0 (or too small for 1 / apq); |tau| is held at 1e150, where the angle is far
+// below any rounding.
+struct SubRot {
+    double c, s, t;
+};
+__device__ __forceinline__ SubRot sub_rot(double app, double aqq, double apq) {
+    const bool on = fabs(apq) > 1e-300;
+    const double b = on ? apq : 1.0, d = on ? aqq - app : 1e300;
+    const double tau = d * rcp_f64(b + b), at = fmin(fabs(tau), 1e150);
+    const double a2 = fma(at, at, 1.0);
+    const double t = rcp_f64(fma(a2, rsq_f64(a2), at));
+    SubRot q;
+    q.c = rsq_f64(fma(t, t, 1.0));
+    q.t = on ? copysign(t, tau) : 0.0;
+    q.s = q.t * q.c;
+    return q;
 }
 
 // Out (32 x 32, stride kSubHld) = X^T Y over the 128 rows of X, Y (stride kSubLd); wave w
@@ -122,61 +158,62 @@ __device__ inline void sub_store_rows(const sub_d4 (&acc)[2][2], double *Y, int 
 
 // X (rows < n, columns < r; zero elsewhere) <- orthonormal basis of its column span by
 // Cholesky QR of the column-normalised block: S = X^T X, its normalised Cholesky factor L and
-// L^{-1} in wave 0's registers (lane l holds row l), X <- X diag(1/sqrt(S_jj)) L^{-T}.
+// L^{-1} in wave 0's registers, X <- X diag(1/sqrt(S_jj)) L^{-T}.
 // Returns the smallest Cholesky pivot (1 for orthonormal input; 0 when a column is zero or
 // numerically dependent: the call then leaves X unchanged).
-__device__ inline double sub_orth_pass(double *X, int n, int r, double *S, double *M, double *flag) {
+// Lanes 0 .. 31 hold the rows of the normalised S, lanes 32 .. 63 the columns of the identity:
+// step j of the right-looking factorisation (scale entry j by 1 / L_jj, subtract L_mj times it
+// from entry m) is the same instruction for both and turns the identity into L^{-1}, so L_mj is
+// broadcast once.  The factorisation of 32 columns takes 8.6 us of a pass's 13 us (all of it one
+// wave's work; with a substitution of its own, square roots and divisions the pass took 20 us).
+// Not inlined: one copy of the unrolled code, and its registers are not added to the caller's.
+__device__ __noinline__ double sub_orth_pass(double *X, int n, int r_, double *S, double *M, double *flag) {
+    const int r = __builtin_amdgcn_readfirstlane(r_);  // (uniform also where this is a call)
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     sub_gram(X, X, S);
     __syncthreads();
     if (wv == 0) {
-        const int l = lane;
+        const int l = lane & 31;
+        const bool unit = lane >= 32;
         double a[kSubMaxR];
 #pragma unroll
-        for (int j = 0; j < kSubMaxR; ++j) a[j] = (l < r && j < r) ? S[l * kSubHld + j] : 0.0;
+        for (int j = 0; j < kSubMaxR; ++j) a[j] = S[l * kSubHld + j];
         const double dg = (l < r) ? S[l * kSubHld + l] : 1.0;
         const double cl = (dg > 0.0) ? 1.0 / sqrt(dg) : 0.0;
-        bool bad = false;
+        bool bad = __any(l < r && !(cl > 0.0));
 #pragma unroll
-        for (int j = 0; j < kSubMaxR; ++j) {
-            const double cj = sub_rl(cl, j);
-            bad |= (j < r) && !(cj > 0.0);
-            a[j] *= cl * cj;
-        }
+        for (int j = 0; j < kSubMaxR; ++j)
+            a[j] = unit ? ((j == l) ? 1.0 : 0.0) : (l < r && j < r) ? a[j] * (cl * sub_rl(cl, j)) : 0.0;
         double pmin = 1.0;
-        // right-looking Cholesky of the normalised Gram, whole symmetric matrix kept
 #pragma unroll
         for (int j = 0; j < kSubMaxR; ++j) {
-            if (j < r && !bad) {
+            if (j < r) {
                 const double d = sub_rl(a[j], j);
                 pmin = fmin(pmin, d);
-                if (!(d > 1e-10)) {
-                    bad = true;
-                } else {
-                    const double inv = 1.0 / sqrt(d);
-                    const double lj = a[j] * inv;  // L[l][j] (for l == j: sqrt(d))
-                    a[j] = lj;
+                bad |= !(d > 1e-10);
+                const double lj = a[j] * rsq_f64(bad ? 1.0 : d);  // L[l][j] (for l == j: sqrt(d)); L^{-1}[j][l]
+                a[j] = lj;
 #pragma unroll
-                    for (int m = j + 1; m < kSubMaxR; ++m) a[m] = fma(-lj, sub_rl(lj, m), a[m]);
-                }
+                for (int b = (j + 1) / 8; b < kSubMaxR / 8; ++b)
+                    if (8 * b < r) {
+                        // (all broadcasts before the first use: a scalar register written by a
+                        // vector instruction is not ready at once)
+                        double t[8];
+#pragma unroll
+                        for (int m = 0; m < 8; ++m)
+                            if (8 * b + m > j) t[m] = sub_rl(lj, 8 * b + m);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int m = 0; m < 8; ++m)
+                            if (8 * b + m > j) a[8 * b + m] = fma(-lj, t[m], a[8 * b + m]);
+                    }
             }
         }
-        // lane c < r: column c of L^{-1} by forward substitution, then row c of
-        // M = diag(cl) L^{-T}: M[c][i] = cl_c * Linv[i][c]
-        if (!bad) {
-            double y[kSubMaxR];
+        // row c of M = diag(cl) L^{-T}: M[c][i] = cl_c * Linv[i][c]
+        if (!bad && unit)
 #pragma unroll
-            for (int i = 0; i < kSubMaxR; ++i) {
-                double sacc = (i == l) ? 1.0 : 0.0;
-#pragma unroll
-                for (int j = 0; j < i; ++j) sacc = fma(-sub_rl(a[j], i), y[j], sacc);
-                y[i] = (i < r) ? sacc / sub_rl(a[i], i) : 0.0;
-            }
-            if (l < kSubMaxR)
-#pragma unroll
-                for (int i = 0; i < kSubMaxR; ++i) M[l * kSubHld + i] = (l < r) ? cl * y[i] : 0.0;
-        }
-        if (l == 0) flag[0] = bad ? 0.0 : pmin;
+            for (int i = 0; i < kSubMaxR; ++i) M[l * kSubHld + i] = (l < r && i < r) ? cl * a[i] : 0.0;
+        if (lane == 0) flag[0] = bad ? 0.0 : pmin;
     }
     __syncthreads();
     const double pm = flag[0];
@@ -190,9 +227,11 @@ __device__ inline double sub_orth_pass(double *X, int n, int r, double *S, doubl
 }
 
 __device__ inline bool sub_orth(double *X, int n, int r, double *S, double *M, double *flag) {
-    double p = sub_orth_pass(X, n, r, S, M, flag);
-    if (p <= 0.0) return false;
-    if (p < 1e-2) p = sub_orth_pass(X, n, r, S, M, flag);  // CholQR2
+    double p = 0.0;
+    for (int pass = 0; pass < 2; ++pass) {
+        p = sub_orth_pass(X, n, r, S, M, flag);
+        if (!(p > 0.0) || p >= 1e-2) break;  // (below: CholQR2)
+    }
     return p > 0.0;
 }
 
@@ -266,15 +305,18 @@ __device__ inline bool sym_top_eigvecs_subspace(const double *Ag, int n, int r, 
 #pragma unroll
                 for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = sub_d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int ks = 0; ks < kSubRows / 4; ++ks) {
-                const double *vr = V + (4 * ks + lk) * kSubLd + lr;
-                const double b0 = vr[0], b1 = vr[16];
+            for (int kb = 0; kb < kSubRows / 16; ++kb)
+                if (16 * kb < n)
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-                    acc[rt][0] = sub_mfma(gA[rt][ks], b0, acc[rt][0]);
-                    acc[rt][1] = sub_mfma(gA[rt][ks], b1, acc[rt][1]);
-                }
-            }
+                    for (int ks = 4 * kb; ks < 4 * kb + 4; ++ks) {
+                        const double *vr = V + (4 * ks + lk) * kSubLd + lr;
+                        const double b0 = vr[0], b1 = vr[16];
+#pragma unroll
+                        for (int rt = 0; rt < 2; ++rt) {
+                            acc[rt][0] = sub_mfma(gA[rt][ks], b0, acc[rt][0]);
+                            acc[rt][1] = sub_mfma(gA[rt][ks], b1, acc[rt][1]);
+                        }
+                    }
             sub_store_rows(acc, Z, n);
         }
         __syncthreads();
@@ -299,14 +341,16 @@ __device__ inline bool sym_top_eigvecs_subspace(const double *Ag, int n, int r, 
                         }
                     }
         }
-        for (int e = tid; e < r * r; e += kEigThreads) {
-            const int a = e / r, b = e % r;
+        // (S, and so H, is zero past r)
+        for (int e = tid; e < kSubMaxR * kSubMaxR; e += kEigThreads) {
+            const int a = e / kSubMaxR, b = e % kSubMaxR;
             const double h = 0.5 * (S[a * kSubHld + b] + S[b * kSubHld + a]);
             H[a * kSubHld + b] = h;
             hh = fma(h, h, hh);
         }
-        rho = sqrt(sub_blk_sum(rr, red));
-        hf = sqrt(sub_blk_sum(hh, red + 4));
+        sub_blk_sum2(rr, hh, red);
+        rho = sqrt(rr);
+        hf = sqrt(hh);
         if (rho <= 1e-12 * hf) {
             conv = true;
             break;
@@ -366,111 +410,81 @@ __device__ inline bool sym_top_eigvecs_subspace(const double *Ag, int n, int r, 
     }
 
     // ---- Rayleigh-Ritz: H = W diag(theta) W^T by cyclic Jacobi, round-robin pairs ----
-    // Thread (group g = tid / 32, index j = tid % 32) handles pairs g and g + 8: it computes
-    // their rotations itself (the 32 threads of a group share a wave, so all of them read the
-    // pair's entries before any of them writes), rotates rows p, q of H in column j and
-    // columns p, q of W in row j, then (after a barrier) columns p, q of H in row j.
-    for (int e = tid; e < kSubMaxR * kSubHld; e += kEigThreads) Wm[e] = ((e / kSubHld) == (e % kSubHld)) ? 1.0 : 0.0;
+    // The pairs of a round partition the indices, so H falls into 2 x 2 blocks (pair i, pair j), one
+    // for each thread, which turns its block from both sides and writes it to the other of two
+    // buffers: a round has one barrier.  A thread computes the rotation of its pair j and takes that
+    // of pair i from the lane of its wave that has it.  It also turns columns p, q of pair i of W in
+    // rows j, j + 16.  A round is one chain of latencies (0.50 us at r = 32; 1.15 us with a barrier
+    // between the rows' and the columns' half, two pairs a thread one after the other and branches in
+    // the rotation: the 186 rounds of r = 32 took 213 us, 93 us this way).  An odd r has index r as the partner without entries (row and column r of H are
+    // zero).  The buffers lie in Z; their stride spreads the rows of a wave over the LDS banks.
+    constexpr int ld = 48;
+    double *Hc = Z, *Hn = Z + kSubMaxR * ld;
+    for (int e = tid; e < kSubMaxR * kSubMaxR; e += kEigThreads) {
+        const int a = e / kSubMaxR, b = e % kSubMaxR;
+        Hc[a * ld + b] = H[a * kSubHld + b];
+        Wm[a * kSubHld + b] = a == b ? 1.0 : 0.0;
+    }
     __syncthreads();
     const int re = r + (r & 1), npair = re >> 1, m = re - 1;
-    const int jg = tid >> 5, jj = tid & 31;
+    const int i0 = tid >> 4, j0 = tid & 15;
+    // Round k's pair g: (re - 1, k) for g = 0, (k + g, k - g) modulo m otherwise.  Threads past the
+    // last pair repeat pair 0 (H: the same values twice; W: on a copy in M that nobody reads), so a
+    // round has no branch and its loads stand first.
+    const int gi = i0 < npair ? i0 : 0, gj = j0 < npair ? j0 : 0;
+    const bool dg = gi == gj;
+    double *w0 = (i0 < npair ? Wm : M) + j0 * kSubHld, *w1 = w0 + 16 * kSubHld;
+    auto next = [&](int &p, int &row) {  // p + 1 modulo m and its row's offset
+        const bool wrap = p + 1 == m;
+        p = wrap ? 0 : p + 1;
+        row = wrap ? 0 : row + ld;
+    };
     double off = 0.0;
     bool jconv = (m <= 0);
     for (int sw = 0; sw < 16 && !jconv; ++sw) {
+        int pi = gi ? gi : m, qi = gi ? m - gi : 0, pj = gj ? gj : m, qj = gj ? m - gj : 0;
+        int rpi = pi * ld, rqi = qi * ld, rpj = pj * ld, rqj = qj * ld;
         for (int k = 0; k < m; ++k) {
-            int pp[2], qq[2];
-            double c_[2], s_[2], t_[2], app_[2], aqq_[2], apq_[2];
-            bool on[2];
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-                const int pi = jg + 8 * h2;
-                int p, q;
-                if (pi == 0) {
-                    p = re - 1;
-                    q = k;
-                } else {
-                    p = k + pi;
-                    if (p >= m) p -= m;
-                    q = k - pi + m;
-                    if (q >= m) q -= m;
-                }
-                on[h2] = pi < npair && p < r && q < r;
-                pp[h2] = p;
-                qq[h2] = q;
-                double c = 1.0, s = 0.0, t = 0.0, app = 0.0, aqq = 0.0, apq = 0.0;
-                if (on[h2]) {
-                    app = H[p * kSubHld + p];
-                    aqq = H[q * kSubHld + q];
-                    apq = H[p * kSubHld + q];
-                    if (apq != 0.0) {
-                        // t = sign(tau) / (|tau| + sqrt(tau^2 + 1)), c = 1 / sqrt(t^2 + 1), with
-                        // the hardware reciprocal / reciprocal-root estimates refined by two
-                        // Newton steps (full FP64 precision; c^2 + s^2 = 1 to rounding)
-                        const double tau = (aqq - app) * rcp_f64(2.0 * apq);
-                        if (fabs(tau) > 1e150) {
-                            t = 0.5 * rcp_f64(tau);
-                        } else {
-                            const double a2 = fma(tau, tau, 1.0);
-                            const double y = rsq_f64(a2);
-                            t = copysign(1.0, tau) * rcp_f64(fma(a2, y, fabs(tau)));
-                        }
-                        c = rsq_f64(fma(t, t, 1.0));
-                        s = t * c;
-                    }
-                }
-                c_[h2] = c;
-                s_[h2] = s;
-                t_[h2] = t;
-                app_[h2] = app;
-                aqq_[h2] = aqq;
-                apq_[h2] = apq;
-            }
-            // rows p, q of H (column jj) and columns p, q of W (row jj)
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-                if (!on[h2] || jj >= r) continue;
-                const int p = pp[h2], q = qq[h2];
-                const double c = c_[h2], s = s_[h2];
-                const double hp = H[p * kSubHld + jj], hq = H[q * kSubHld + jj];
-                const double wp = Wm[jj * kSubHld + p], wq = Wm[jj * kSubHld + q];
-                H[p * kSubHld + jj] = c * hp - s * hq;
-                H[q * kSubHld + jj] = s * hp + c * hq;
-                Wm[jj * kSubHld + p] = c * wp - s * wq;
-                Wm[jj * kSubHld + q] = s * wp + c * wq;
-            }
+            const double ajp = Hc[rpj + pj], ajq = Hc[rqj + qj], ajo = Hc[rpj + qj];
+            __builtin_amdgcn_sched_barrier(0);  // (first: the rotation waits for them alone)
+            const double b00 = Hc[rpi + pj], b01 = Hc[rpi + qj], b10 = Hc[rqi + pj], b11 = Hc[rqi + qj];
+            const double w0p = w0[pi], w0q = w0[qi], w1p = w1[pi], w1q = w1[qi];
+            __builtin_amdgcn_sched_barrier(0);
+            const SubRot rj = sub_rot(ajp, ajq, ajo);
+            const double ic = __shfl(rj.c, i0, 64), is = __shfl(rj.s, i0, 64);
+            const double t00 = ic * b00 - is * b10, t01 = ic * b01 - is * b11;
+            const double t10 = is * b00 + ic * b10, t11 = is * b01 + ic * b11;
+            // (the diagonal block is set exactly)
+            Hn[rpi + pj] = dg ? ajp - rj.t * ajo : rj.c * t00 - rj.s * t01;
+            Hn[rpi + qj] = dg ? 0.0 : rj.s * t00 + rj.c * t01;
+            Hn[rqi + pj] = dg ? 0.0 : rj.c * t10 - rj.s * t11;
+            Hn[rqi + qj] = dg ? ajq + rj.t * ajo : rj.s * t10 + rj.c * t11;
+            w0[pi] = ic * w0p - is * w0q;
+            w0[qi] = is * w0p + ic * w0q;
+            w1[pi] = ic * w1p - is * w1q;
+            w1[qi] = is * w1p + ic * w1q;
+            if (gi) next(pi, rpi);
+            next(qi, rqi);
+            if (gj) next(pj, rpj);
+            next(qj, rqj);
             __syncthreads();
-            // columns p, q of H (row jj); the (p, q) block is set exactly
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-                if (!on[h2] || jj >= r) continue;
-                const int p = pp[h2], q = qq[h2];
-                double np_, nq_;
-                if (jj == p) {
-                    np_ = app_[h2] - t_[h2] * apq_[h2];
-                    nq_ = 0.0;
-                } else if (jj == q) {
-                    np_ = 0.0;
-                    nq_ = aqq_[h2] + t_[h2] * apq_[h2];
-                } else {
-                    const double c = c_[h2], s = s_[h2];
-                    const double hp = H[jj * kSubHld + p], hq = H[jj * kSubHld + q];
-                    np_ = c * hp - s * hq;
-                    nq_ = s * hp + c * hq;
-                }
-                H[jj * kSubHld + p] = np_;
-                H[jj * kSubHld + q] = nq_;
-            }
-            __syncthreads();
+            double *t = Hc;
+            Hc = Hn;
+            Hn = t;
         }
         double o = 0.0;
-        for (int e = tid; e < r * r; e += kEigThreads) {
-            const int a = e / r, b = e % r;
-            if (a != b) o = fma(H[a * kSubHld + b], H[a * kSubHld + b], o);
+#pragma unroll
+        for (int u = 0; u < kSubMaxR * kSubMaxR / kEigThreads; ++u) {
+            const int a = (tid + u * kEigThreads) / kSubMaxR, b = (tid + u * kEigThreads) % kSubMaxR;
+            const double h = Hc[a * ld + b];
+            o = fma(h, (a != b && a < r && b < r) ? h : 0.0, o);
         }
         off = sqrt(sub_blk_sum(o, red));
         jconv = off <= 1e-14 * hf;
     }
     if (!jconv) return false;
+    if (tid < r) H[tid * kSubHld + tid] = Hc[tid * ld + tid];
+    __syncthreads();
 
     // ---- certificate that the theta are the r largest eigenvalues ----
     const double eb = rho + off;

@@ -72,9 +72,9 @@ __global__ __launch_bounds__(256) void k_gram_sum(const float *__restrict__ part
 // try_sub the subspace-iteration path runs first (start block U0, or a built-in one when U0
 // is null; U0 may alias U) and the tridiagonal solver only when it declines.  method (optional,
 // device) receives 1 for the subspace path, 0 for the tridiagonal one.
-// A solve is one workgroup's chain of ~200 us whatever the size of the tensor, so the independent
-// ones of an HOSVD (a mode each) share one launch: three modes of 125 x 101 x 77 took 164 + 187 +
-// 249 us one after the other.
+// A solve is one workgroup's chain of 110 to 160 us whatever the size of the tensor, so the independent
+// ones of an HOSVD (a mode each) share one launch: three modes of 125 x 101 x 77 take 115 + 130 +
+// 155 us one after the other.
 struct EigJob {
     const double *G;
     int n, r;
