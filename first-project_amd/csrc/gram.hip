@@ -12,9 +12,9 @@
 //  case A (P == 1): rows are contiguous and K (= q) is strided; a lane loads its 8 consecutive
 //    rows at 8 columns and transposes in registers, so row block t holds rows 8 m + t,
 //    m = lane % 16.
-// BF16 tensors only: FP32 ones, and BF16 ones without whole vectors, go through LDS
-// (gram_any.hip; in FP32 this kernel's one wave per SIMD left the matrix pipe at 404-439 us for
-// 128^4 where that one takes 372-410, and 60 us for 32^3 128 where it takes 14).
+// BF16 tensors only: FP32 ones, and BF16 ones without whole vectors, go through LDS (gram_f32.hip,
+// gram_any.hip; in FP32 this kernel's one wave per SIMD took 404-439 us for 128^4 where the first
+// takes 272-307, and 60 us for 32^3 128 where it takes 14).
 //
 // The 4 waves of a workgroup take contiguous quarters of its K range and are summed in LDS
 // in a fixed order; each workgroup writes one 128 x 128 FP32 partial, and the partials are

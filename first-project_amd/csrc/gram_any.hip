@@ -1,5 +1,5 @@
 // gram_any.hip -- Gram of a mode-n unfolding, G = X(n) X(n)^T, In <= 128, on FP32 MFMA with the
-// tensor tile staged in LDS: FP32 tensors of every shape and BF16 tensors without whole vectors.
+// tensor tile staged in LDS, element by element: FP32 and BF16 tensors without whole vectors.
 //
 // X is read as the (P, In, Q) view, column k = p + P q of the unfolding a fibre.  A workgroup
 // walks its range of columns in steps of 64: the (rows x 64) tile goes to LDS as [row][k]
@@ -9,13 +9,9 @@
 // a pair reading its two operands from LDS.  Each wave keeps two chains of sums (even and odd
 // groups of 16 columns).  Every workgroup writes the FP32 partial of its range; the caller adds
 // them in FP64.
-// With whole vectors (VEC = 4) a thread loads 16 bytes along the contiguous index: along p, or,
-// for P = 1, 4 rows of 4 columns transposed in registers; otherwise element by element.
 //
-// Bound by the FP32 matrix pipe for a large tensor (128^4: 38.7 GFLOP of pairs, 260 us at the
-// 149 TFLOP/s of a large product; 372 us for the modes with P > 1, 410 for mode 0) and by latency
-// for a small one, where it wants many workgroups: 125 x 101 x 77 took 500-730 us a mode with
-// one workgroup per 2048 columns (7 of them) on vector FMAs and takes 13-17 us.
+// Latency bound at the sizes that come here, so it wants many workgroups: 125 x 101 x 77 took
+// 500-730 us a mode with one workgroup per 2048 columns (7 of them) on vector FMAs and takes 13-17 us.
 #include "common.hpp"
 #include <algorithm>
 
@@ -29,10 +25,10 @@ __device__ __forceinline__ float ga_f32(float v) { return v; }
 __device__ __forceinline__ float ga_f32(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 
 // NP: pairs per wave, ceil(nb (nb + 1) / 2 / 4) for nb = ceil(In / 16) row blocks, rounded up
-template <typename ET, bool PC, int VEC, int NP>
+template <typename ET, bool PC, int NP>
 __global__ __launch_bounds__(256, 2) void k_gram_any(const ET *__restrict__ X, long P, long In, long Q, long kper,
                                                      float *__restrict__ part) {
-    constexpr int NL = kGaN * kGaK / 256 / VEC;  // loads per thread and step
+    constexpr int NL = kGaN * kGaK / 256;  // loads per thread and step
     __shared__ __attribute__((aligned(16))) float xs[kGaN * kGaLd];
     const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -41,27 +37,10 @@ __global__ __launch_bounds__(256, 2) void k_gram_any(const ET *__restrict__ X, l
     const int nb = (int)((In + 15) / 16), npair = nb * (nb + 1) / 2;
     const int nrow = 16 * nb;
 
-    // VEC 1: lanes along k (P > 1) or along the rows (P = 1), 32 elements.  VEC 4, P > 1: 16 lanes
-    // a row, 16 rows apart; P = 1: 32 row quads x 8 column quads, 2 of them a thread.
-    float4 xq[VEC == 4 ? NL : 1];
-    ET xe[VEC == 1 ? NL : 1];
+    // lanes along k (P > 1) or along the rows (P = 1), 32 elements
+    ET xe[NL];
     auto load = [&](long k0) {
-        if constexpr (VEC == 4 && PC) {
-            const long k = min(k0 + 4 * (tid & 15), K - 4), q = k / P;  // P % 4 == 0: a quad lies in one run
-            const ET *p = X + (k - q * P) + q * P * In;
-#pragma unroll
-            for (int u = 0; u < NL; ++u)
-                if (16 * u < nrow)
-                    xq[u] = ld_stream(reinterpret_cast<const float4 *>(p + min((long)(tid >> 4) + 16 * u, In - 1) * P));
-        } else if constexpr (VEC == 4) {
-            const long r = min(4L * (tid & 31), In - 4);  // In % 4 == 0
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    xq[4 * u + c] = ld_stream(reinterpret_cast<const float4 *>(
-                        X + r + min(k0 + 4 * ((tid >> 5) + 8 * u) + c, K - 1) * In));
-        } else if constexpr (PC) {
+        if constexpr (PC) {
             const long k = min(k0 + lane, K - 1), q = k / P;
             const ET *p = X + (k - q * P) + q * P * In;
             long r0 = wave;
@@ -78,30 +57,7 @@ __global__ __launch_bounds__(256, 2) void k_gram_any(const ET *__restrict__ X, l
         }
     };
     auto store = [&](long k0) {
-        if constexpr (VEC == 4 && PC) {
-            const bool on = k0 + 4 * (tid & 15) < K;
-#pragma unroll
-            for (int u = 0; u < NL; ++u)
-                if (16 * u < nrow)
-                    *reinterpret_cast<float4 *>(xs + ((tid >> 4) + 16 * u) * kGaLd + 4 * (tid & 15)) =
-                        on ? xq[u] : float4{0.f, 0.f, 0.f, 0.f};
-        } else if constexpr (VEC == 4) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int kq = (tid >> 5) + 8 * u;
-                float v[4][4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const bool on = k0 + 4 * kq + c < K;
-                    const float4 w = xq[4 * u + c];
-                    v[0][c] = on ? w.x : 0.f, v[1][c] = on ? w.y : 0.f, v[2][c] = on ? w.z : 0.f, v[3][c] = on ? w.w : 0.f;
-                }
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    *reinterpret_cast<float4 *>(xs + (4 * (tid & 31) + t) * kGaLd + 4 * kq) =
-                        float4{v[t][0], v[t][1], v[t][2], v[t][3]};
-            }
-        } else if constexpr (PC) {
+        if constexpr (PC) {
             const bool on = k0 + lane < K;
 #pragma unroll
             for (int u = 0; u < NL; ++u)
@@ -163,13 +119,16 @@ __global__ __launch_bounds__(256, 2) void k_gram_any(const ET *__restrict__ X, l
                 dst[(oi[j] + 4 * lg + v) * kGaN + oj[j] + lm] = acc[j][0][v] + acc[j][1][v];
 }
 
-template <typename ET, int VEC>
+int gram_f32_wgs(long In);
+void gram_f32_launch(const float *X, long P, long In, long Q, long kper, float *part, unsigned nblk, hipStream_t s);
+
+template <typename ET>
 static void ga_launch(const ET *X, long P, long In, long Q, long kper, float *part, unsigned g, hipStream_t s) {
     const int nb = (int)ceil_div(In, 16L), np = (int)ceil_div(nb * (nb + 1) / 2, 4L);
 #define TDX_GA(NP_)                                                                                     \
     do {                                                                                                \
-        if (P > 1) k_gram_any<ET, true, VEC, NP_><<<g, 256, 0, s>>>(X, P, In, Q, kper, part);           \
-        else k_gram_any<ET, false, VEC, NP_><<<g, 256, 0, s>>>(X, P, In, Q, kper, part);                \
+        if (P > 1) k_gram_any<ET, true, NP_><<<g, 256, 0, s>>>(X, P, In, Q, kper, part);           \
+        else k_gram_any<ET, false, NP_><<<g, 256, 0, s>>>(X, P, In, Q, kper, part);                \
     } while (0)
     if (np <= 1) TDX_GA(1);
     else if (np <= 3) TDX_GA(3);
@@ -181,16 +140,19 @@ static void ga_launch(const ET *X, long P, long In, long Q, long kper, float *pa
 // Partial Grams (upper triangle of each kGaN^2 block, row-major) in part; returns their number,
 // at most max_parts, or -1 on a launch error.
 int gram_any_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s) {
+    // whole vectors of an FP32 tensor: gram_f32.hip (element by element 64^4 takes 32-38 us a mode
+    // and 128^4 446-487; 21-22 and 277-318 there)
+    const bool vec = xtype == TDX_F32 && ((uintptr_t)X & 15) == 0 && (P > 1 ? P % 4 == 0 : In % 4 == 0);
     const long steps = ceil_div(P * Q, (long)kGaK);
-    // three workgroups per CU; at least two steps each, whose loads overlap, so that a partial
+    // the workgroups that fill the chip; at least two steps each, whose loads overlap, so that a partial
     // (64 KB) is not written for one tile of 32 KB
-    long nblk = std::min<long>(std::min(3L * device_cus(), (long)max_parts), ceil_div(steps, 2L));
+    const int wgs = vec ? gram_f32_wgs(In) : 3;
+    long nblk = std::min<long>(std::min((long)wgs * device_cus(), (long)max_parts), ceil_div(steps, 2L));
     const long kper = ceil_div(steps, nblk) * kGaK;
     nblk = ceil_div(P * Q, kper);
-    const bool vec = xtype == TDX_F32 && ((uintptr_t)X & 15) == 0 && (P > 1 ? P % 4 == 0 : In % 4 == 0);
-    if (xtype == TDX_BF16) ga_launch<uint16_t, 1>((const uint16_t *)X, P, In, Q, kper, part, (unsigned)nblk, s);
-    else if (vec) ga_launch<float, 4>((const float *)X, P, In, Q, kper, part, (unsigned)nblk, s);
-    else ga_launch<float, 1>((const float *)X, P, In, Q, kper, part, (unsigned)nblk, s);
+    if (xtype == TDX_BF16) ga_launch<uint16_t>((const uint16_t *)X, P, In, Q, kper, part, (unsigned)nblk, s);
+    else if (vec) gram_f32_launch((const float *)X, P, In, Q, kper, part, (unsigned)nblk, s);
+    else ga_launch<float>((const float *)X, P, In, Q, kper, part, (unsigned)nblk, s);
     return hipGetLastError() == hipSuccess ? (int)nblk : -1;
 }
 

@@ -1,0 +1,250 @@
+// gram_f32.hip -- Gram of a mode-n unfolding, G = X(n) X(n)^T, In <= 128, of an FP32 tensor with
+// whole 16-byte vectors, its products formed from three BF16 parts per element.
+//
+// X is read as the (P, In, Q) view, column k = p + P q of the unfolding a fibre.  A workgroup
+// walks its range of columns in steps of 64; every element of the (rows x 64) tile is cut once,
+// on its way from registers to LDS, into x = x1 + x2 + x3 exactly, each part what is left rounded
+// to BF16.  v_mfma_f32_16x16x32_bf16 multiplies x1 y1, x1 y2, x2 y1, x1 y3, x2 y2 and x3 y1
+// exactly and adds them in FP32 (the terms left out are below 2^-25 of |x y|, of either sign); the
+// sums of a step enter the FP32 accumulators once, so the chains of roundings stay short.  Every
+// workgroup writes the FP32 partial of its range; the caller adds them in FP64.
+//   * G needs the block pairs bi <= bj of its 16 x 16 blocks only.  Wave w takes the block rows w
+//     and nb - 1 - w: nb + 1 pairs each, whose column operands it reads from LDS once.
+//   * LDS rows are 64 BF16 of a part (128 bytes); chunk c of 8 lies at c ^ (row / 2 ^ row / 16) mod
+//     8, so 16 rows of one chunk hit distinct banks, and so do the rows of a transposing store
+//     but for their parity.
+//   * Loads along the contiguous index: along p, or, for P = 1, 4 rows of 4 columns transposed in
+//     registers.  The next step's are in flight meanwhile.
+//   * A tile with an entry above 2^60 (its products may overflow, an infinity has no parts) or a
+//     loaded vector below 2^-100 throughout (whose last part would lose bits) is read again and
+//     multiplied in FP32.
+//
+// A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
+// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock.  Modes 0 .. 3 on
+// FP32 matrix instructions before: 128^4 420 / 396 / 393 / 395 -> 275 / 272 / 299 / 307 us (1.07 GB:
+// 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 22 / 22 / 22 / 22, 256 x 128 x 128 15 / 13 -> 10 / 10;
+// errors against 64 bits 7e-9 -> 5e-9 (64^4), 2.2e-8 -> 1.1e-8 (124 x 100 x 76), 3.7e-8 -> 1.6e-8
+// (64 x 48 x 40).  Not faster: eight waves a tile (128 registers spill), the pair counts at compile
+// time.
+// A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
+// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock.  Modes 0 .. 3 on
+// FP32 matrix instructions before: 128^4 420 / 396 / 393 / 395 -> 278 / 277 / 306 / 318 us (1.07 GB:
+// 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 21 / 22 / 22 / 21, 256 x 128 x 128 15 -> 12; errors
+// against 64 bits 7e-9 -> 8e-9 (64^4), 2.2e-8 -> 1.8e-8 (124 x 100 x 76), 3.7e-8 -> 2.6e-8 (64 x 48 x
+// 40).  Not faster: eight waves a tile (128 registers spill), the pair counts at compile time.
+#include "common.hpp"
+#include <algorithm>
+
+namespace tdx {
+
+typedef float gf_f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 gf_b8 __attribute__((ext_vector_type(8)));
+
+static constexpr int kGfN = 128, kGfK = 64;
+
+// workgroups per CU (and waves per SIMD): registers allow two of 128 rows
+constexpr int gf_wgs(int nb) { return nb > 4 ? 2 : 3; }
+int gram_f32_wgs(long In) { return gf_wgs((int)ceil_div(In, 16L)); }
+
+// NB: row blocks, at least ceil(In / 16)
+template <bool PC, int NB>
+__global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__restrict__ X, long P, long In, long Q, long kper,
+                                                     float *__restrict__ part) {
+    constexpr int NR = 16 * NB;
+    __shared__ uint4 xs[3 * NR * 8];
+    __shared__ int odd[2];
+    const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const long K = P * Q;
+    const long kbeg = (long)blockIdx.x * kper, kend = min(kbeg + kper, K);
+    const int nb = (int)((In + 15) / 16);
+    const int b1 = wave, b2 = nb - 1 - wave;  // this wave's block rows (none: b2 < b1)
+    if (tid < 2) odd[tid] = 0;
+
+    // P > 1: row tid / 16 + 16 u, columns k .. k + 3, a vector a load; k = p + P q is stepped without
+    // a division.  P = 1: 4 x 4 blocks of rows 4 rq .. and columns k + 4 KQ u .., four vectors a load.
+    constexpr int NT = PC ? NR / 16 : NR / 64, RQ = NR / 4, KQ = 4 * (256 / (4 * RQ));
+    const int rq = (tid >> 2) & (RQ - 1), kq = PC ? tid & 15 : (tid & 3) + 4 * (tid / (4 * RQ));
+    long k = kbeg + 4 * kq;  // of the step to be loaded
+    long q = PC ? k / P : 0, p = PC ? k - q * P : 0;
+    const long qs = kGfK / P, ps = kGfK - qs * P;
+    float4 xq[PC ? NT : 4 * NT];
+    auto load = [&](int u) {
+        if constexpr (PC) {
+            // (P % 4 == 0: a vector lies in one run, and is inside as a whole)
+            xq[u] = ld_stream(reinterpret_cast<const float4 *>(X + (k < K ? p + q * P * In : 0) +
+                                                               min((long)(tid >> 4) + 16 * u, In - 1) * P));
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                xq[4 * u + c] = ld_stream(reinterpret_cast<const float4 *>(
+                    X + min(4L * rq, In - 4) + min(k + 4 * KQ * u + c, K - 1) * In));  // In % 4 == 0
+        }
+    };
+    auto advance = [&]() {
+        k += kGfK;
+        if constexpr (PC) {
+            p += ps;
+            q += qs;
+            const bool wrap = p >= P;
+            p -= wrap ? P : 0;
+            q += wrap;
+        }
+    };
+    // four consecutive columns of a row: their parts to LDS; true where FP32 products are needed
+    auto put = [&](int row, int kq, float4 x) {
+        float m = 0.0f;  // largest magnitude (NaN left out: it stays NaN in its parts)
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x.x), "v"(x.y));
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x.z), "v"(x.w));
+        uint2 *d = reinterpret_cast<uint2 *>(xs + row * 8 + ((kq >> 1) ^ (((row >> 1) ^ (row >> 4)) & 7))) + (kq & 1);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            uint2 w;
+            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w.x) : "v"(x.x), "v"(x.y));
+            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w.y) : "v"(x.z), "v"(x.w));
+            d[k * NR * 16] = w;
+            x.x -= __uint_as_float(w.x << 16), x.y -= __uint_as_float(w.x & 0xffff0000u);
+            x.z -= __uint_as_float(w.y << 16), x.w -= __uint_as_float(w.y & 0xffff0000u);
+        }
+        return m > 0x1p60f || (m < 0x1p-100f && m > 0.0f);
+    };
+    auto store = [&](long k0, int u) {
+        if constexpr (PC) {
+            return put((tid >> 4) + 16 * u, kq, k0 + 4 * kq < K ? xq[u] : float4{0.f, 0.f, 0.f, 0.f});
+        } else {
+            float v[4][4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const bool on = k0 + 4 * (kq + KQ * u) + c < K;
+                const float4 w = xq[4 * u + c];
+                v[0][c] = on ? w.x : 0.f, v[1][c] = on ? w.y : 0.f, v[2][c] = on ? w.z : 0.f, v[3][c] = on ? w.w : 0.f;
+            }
+            bool f = false;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) f |= put(4 * rq + t, kq + KQ * u, float4{v[t][0], v[t][1], v[t][2], v[t][3]});
+            return f;
+        }
+    };
+    auto operand = [&](int b, int ks, int k) {
+        const uint4 v = xs[(k * NR + 16 * b + lm) * 8 + ((4 * ks + lg) ^ ((lm >> 1) ^ (b & 7)))];
+        return __builtin_bit_cast(gf_b8, v);
+    };
+    // acc1[t], acc2[t]: block rows b1, b2 with block column nb - 1 - t
+    gf_f4 acc1[NB], acc2[NB / 2];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc1[t] = gf_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NB / 2; ++t) acc2[t] = gf_f4{0.f, 0.f, 0.f, 0.f};
+    if (kbeg < kend)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) load(u);
+    advance();
+    int par = 0;
+    for (long k0 = kbeg; k0 < kend; k0 += kGfK, par ^= 1) {
+        __syncthreads();
+        if (tid == 0) odd[par ^ 1] = 0;  // (read by every wave before this barrier, set after the next)
+        // (a register's next load leaves as soon as it is free; past the range: clamped addresses or
+        // the next range's, never consumed)
+        bool f = false;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            f |= store(k0, u);
+            load(u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        advance();
+        if (f) odd[par] = 1;
+        __syncthreads();
+        if (b2 < b1) continue;
+        if (odd[par]) {
+            // from memory, FP32 products
+            for (int q = 0; q < 16; ++q) {
+                const long kk = k0 + 4 * q + lg, k = min(kk, K - 1), kd = k / P;
+                const float *p = X + (k - kd * P) + kd * P * In;
+                auto value = [&](int blk) {
+                    const float v = p[min((long)(16 * blk + lm), In - 1) * P];
+                    return kk < K ? v : 0.0f;
+                };
+                const float v1 = value(b1), v2 = value(b2);
+#pragma unroll
+                for (int t = 0; t < NB; ++t)
+                    if (nb - 1 - t >= b1) {
+                        const float w = value(nb - 1 - t);
+                        acc1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1, w, acc1[t], 0, 0, 0);
+                        if (t < NB / 2 && t <= wave && b2 > b1)
+                            acc2[t < NB / 2 ? t : 0] =
+                                __builtin_amdgcn_mfma_f32_16x16x4f32(v2, w, acc2[t < NB / 2 ? t : 0], 0, 0, 0);
+                    }
+            }
+            continue;
+        }
+        gf_b8 a1[2][3], a2[2][3];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) a1[ks][k] = operand(b1, ks, k), a2[ks][k] = operand(b2, ks, k);
+        // the step's sums, smallest terms first (so two roundings at the size of the sum)
+        auto mul = [&](const gf_b8 (&a)[2][3], const gf_b8 (&b)[2][3]) {
+            gf_f4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][2], b[ks][0], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][0], b[ks][2], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][1], b[ks][1], s, 0, 0, 0);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][1], b[ks][0], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][0], b[ks][1], s, 0, 0, 0);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][0], b[ks][0], s, 0, 0, 0);
+            return s;
+        };
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+            if (nb - 1 - t >= b1) {
+                gf_b8 b[2][3];
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) b[ks][k] = operand(nb - 1 - t, ks, k);
+                // (the sums are added before the branch: hipcc left out the wait states that a read
+                // of a matrix result needs where it had moved the add behind one)
+                acc1[t] += mul(a1, b);
+                asm volatile("" : "+v"(acc1[t]));
+                if (t < NB / 2 && t <= wave && b2 > b1) {
+                    acc2[t < NB / 2 ? t : 0] += mul(a2, b);
+                    asm volatile("" : "+v"(acc2[t < NB / 2 ? t : 0]));
+                }
+            }
+    }
+    // register v of lane (lm, lg): row 4 lg + v, column lm of the pair's block
+    float *dst = part + (long)blockIdx.x * kGfN * kGfN;
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int c = 16 * (nb - 1 - t) + lm;
+            if (b2 >= b1 && nb - 1 - t >= b1) dst[(16 * b1 + 4 * lg + v) * kGfN + c] = acc1[t][v];
+            if (t < NB / 2 && t <= wave && b2 > b1) dst[(16 * b2 + 4 * lg + v) * kGfN + c] = acc2[t < NB / 2 ? t : 0][v];
+        }
+}
+
+// Partial Grams (upper triangle of each kGfN^2 block, row-major) in part, of nblk ranges of kper
+// columns.  Requires X 16-byte aligned, P % 4 == 0, or P = 1 and In % 4 == 0; In <= kGfN.
+void gram_f32_launch(const float *X, long P, long In, long Q, long kper, float *part, unsigned nblk, hipStream_t s) {
+    const int nb = (int)ceil_div(In, 16L);
+    if (P > 1) {
+        if (nb <= 2) k_gram_f32<true, 2><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else if (nb <= 4) k_gram_f32<true, 4><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else k_gram_f32<true, 8><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+    } else {
+        // (at least 64 rows: a 4 x 4 block for every thread)
+        if (nb <= 4) k_gram_f32<false, 4><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else k_gram_f32<false, 8><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+    }
+}
+
+}  // namespace tdx

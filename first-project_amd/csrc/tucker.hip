@@ -9,8 +9,8 @@
 //
 // The Gram never forms an unfolded copy (the reference materialises X2 with t2m and, for
 // order 4, X2 and X3 by identity-matrix GEMMs, src/tucker4_hosvd.cu:23-37): a workgroup
-// accumulates an In x In FP32 tile over a range of the (P, In, Q) view's fibres (gram_any.hip,
-// gram.hip), partial tiles are summed in FP64 in a fixed order.  The eigensolve is the FP64
+// accumulates an In x In FP32 tile over a range of the (P, In, Q) view's fibres (gram_f32.hip,
+// gram_any.hip, gram.hip), partial tiles are summed in FP64 in a fixed order.  The eigensolve is the FP64
 // tridiagonal solver in one workgroup (subspace iteration first where the top eigenvalues
 // stand clear of the rest, warm-started from the previous factor in HOOI); eigenvector signs
 // are fixed so that the entry of largest magnitude is positive (syevdx leaves the sign
@@ -152,7 +152,7 @@ static int unfold_gram(const void *X, int xtype, int order, const long *dims, in
     for (int m = mode + 1; m < order; ++m) Q *= dims[m];
     const long In = dims[mode];
     if (In > kGramMaxN) return record(TDX_ERR_UNSUPPORTED);
-    // the BF16 kernel for whole vectors (gram.hip), the LDS kernel otherwise
+    // the BF16 kernel for whole vectors (gram.hip), the LDS kernels otherwise
     int nb = 0;
     if (xtype == TDX_BF16)
         nb = gram_mfma_launch(X, P, In, Q, W.gram_part, W.gram_blocks < 512 ? W.gram_blocks : 512, s);
@@ -359,7 +359,7 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
     }
     // The final core, always from the FP32 tensor.  After an iteration on FP32 storage the last Y
     // holds all modes but d-1 contracted with the final factors, so one small TTM is left (a chain
-    // over X took 0.41 ms of the 4.62 ms of HOSVD and one iteration of 128^4, ranks 32); with an error
+    // over X took 0.36 ms of the 4.62 ms of HOSVD and one iteration of 128^4, ranks 32); with an error
     // history the last iteration has already made the core.
     if (iters == 0 || (bf16 && !relerr_hist)) st = core_from(X, order, dims, ranks, U, W, core, s);
     else if (!relerr_hist)
