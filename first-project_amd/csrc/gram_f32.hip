@@ -26,12 +26,6 @@
 // errors against 64 bits 7e-9 -> 5e-9 (64^4), 2.2e-8 -> 1.1e-8 (124 x 100 x 76), 3.7e-8 -> 1.6e-8
 // (64 x 48 x 40).  Not faster: eight waves a tile (128 registers spill), the pair counts at compile
 // time.
-// A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
-// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock.  Modes 0 .. 3 on
-// FP32 matrix instructions before: 128^4 420 / 396 / 393 / 395 -> 278 / 277 / 306 / 318 us (1.07 GB:
-// 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 21 / 22 / 22 / 21, 256 x 128 x 128 15 -> 12; errors
-// against 64 bits 7e-9 -> 8e-9 (64^4), 2.2e-8 -> 1.8e-8 (124 x 100 x 76), 3.7e-8 -> 2.6e-8 (64 x 48 x
-// 40).  Not faster: eight waves a tile (128 registers spill), the pair counts at compile time.
 #include "common.hpp"
 #include <algorithm>
 
@@ -176,6 +170,7 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
                                 __builtin_amdgcn_mfma_f32_16x16x4f32(v2, w, acc2[t < NB / 2 ? t : 0], 0, 0, 0);
                     }
             }
+            __builtin_amdgcn_s_sleep(1);  // (as below: the last results are in place before any branch)
             continue;
         }
         gf_b8 a1[2][3], a2[2][3];

@@ -171,6 +171,9 @@ __global__ __launch_bounds__(256, 2) void k_cp_model(FacArgs f, float *__restric
                             acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(aop[t][k], w, acc[t], 0, 0, 0);
                 }
             }
+            // (the wait states between a matrix result and its first read: hipcc counted one too few on
+            // the way past the skipped row blocks)
+            asm volatile("s_nop 9" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const long i = row0 + 16 * t + 4 * lg;
