@@ -1276,20 +1276,12 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     // is the default one, run on a private blocking stream (it orders after earlier
     // default-stream work by the legacy-stream rules) and join it before returning.
     hipStream_t s = stream();
-    hipStream_t owned = nullptr;
+    StreamLease owned;
     if (!s) {
-        TDX_HIP(hipStreamCreate(&owned));
-        s = owned;
+        const int st = owned.take();
+        if (st) return st;
+        s = owned.get();
     }
-    struct StreamGuard {
-        hipStream_t st;
-        ~StreamGuard() {
-            if (st) {
-                (void)hipStreamSynchronize(st);
-                (void)hipStreamDestroy(st);
-            }
-        }
-    } guard{owned};
     const int total = opt.max_sweeps + (opt.storage == TDX_F32 ? 0 : opt.refine_sweeps);
     if (opt.line_search < 0 || opt.line_search > 3) return record(TDX_ERR_ARG);
     if (opt.line_search == 1 && (!opt.mlp_params || opt.mlp_width <= 0 || opt.mlp_width > 128))
@@ -1449,6 +1441,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     int result = status ? TDX_WARN_SINGULAR : TDX_OK;
     if (opt.record_fit && count > 0 && !isfinite(last)) result = TDX_ERR_NONFINITE;
     give_plan(key, std::move(Pp));
+    owned.done();
     if (report) {
         report->sweeps_done = done_main + done_ref;
         report->status = result;

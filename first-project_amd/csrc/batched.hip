@@ -780,7 +780,7 @@ const char *tdx_cp_batched_variant_name(int v) {
 // tensor t at uoff[3t+m], I_m x R column-major).  init = 0 draws U(0,1) from Philox stream
 // (seed + t, m); 1 uses the caller's U.  variant < 0 picks the item design ("items").  fit_hist (host, may
 // be NULL) receives ntensors x sweeps relative errors; sweep_ms (host, may be NULL) the
-// device time of every sweep.  The per-sweep launches are captured once in a hipGraph.
+// device time of every sweep.
 int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *ranks, const long *xoff,
                        const long *uoff, long ntensors, int sweeps, int init, uint64_t seed, int variant,
                        double *fit_hist, float *sweep_ms) {
@@ -788,7 +788,6 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
     if (variant >= kNumVariants) return record(TDX_ERR_ARG);
     if (variant < 0) variant = kItemsVariant;
     std::vector<BDesc> h(ntensors);
-    std::vector<std::pair<long, int>> order(ntensors);
     for (long t = 0; t < ntensors; ++t) {
         BDesc &d = h[t];
         d.I = (int)dims[3 * t];
@@ -801,133 +800,134 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
         d.xoff = xoff[t];
         d.toff = 0;
         for (int m = 0; m < 3; ++m) d.uoff[m] = uoff[3 * t + m];
-        order[t] = {-(long)d.I * d.J * d.K * d.R, (int)t};  // largest work first
     }
-    std::sort(order.begin(), order.end());
-    std::vector<int> sched(ntensors);
-    for (long t = 0; t < ntensors; ++t) sched[t] = order[t].second;
+    const bool items = variant == kItemsVariant;
+    std::vector<int> sched;
+    if (!items) {
+        std::vector<std::pair<long, int>> order(ntensors);
+        for (long t = 0; t < ntensors; ++t)
+            order[t] = {-(long)h[t].I * h[t].J * h[t].K * h[t].R, (int)t};  // largest work first
+        std::sort(order.begin(), order.end());
+        sched.resize(ntensors);
+        for (long t = 0; t < ntensors; ++t) sched[t] = order[t].second;
+    }
 
     hipStream_t s = stream();
-    hipStream_t owned = nullptr;
+    StreamLease owned;
+    DeviceLease mem;  // (given back before the stream: its work has finished)
+    int st = TDX_OK;
     if (!s) {
-        TDX_HIP(hipStreamCreate(&owned));
-        s = owned;
+        st = owned.take();
+        if (st) return st;
+        s = owned.get();
     }
-    BDesc *d_desc = nullptr;
-    int *d_sched = nullptr, *d_int = nullptr;
-    double *d_nx = nullptr, *d_fit = nullptr;
-    struct Guard {
-        hipStream_t st;
-        void *p[11];
-        ~Guard() {
-            if (st) (void)hipStreamSynchronize(st);
-            for (void *q : p)
-                if (q) (void)hipFree(q);
-            if (st) (void)hipStreamDestroy(st);
-        }
-    } guard{owned, {nullptr}};
-    TDX_HIP(hipMalloc(&d_desc, sizeof(BDesc) * ntensors));
-    guard.p[0] = d_desc;
-    TDX_HIP(hipMalloc(&d_sched, sizeof(int) * ntensors));
-    guard.p[1] = d_sched;
-    TDX_HIP(hipMalloc(&d_int, sizeof(int) * 8));
-    guard.p[2] = d_int;
-    TDX_HIP(hipMalloc(&d_nx, sizeof(double) * ntensors));
-    guard.p[3] = d_nx;
     const int S = sweeps > 0 ? sweeps : 1;
-    TDX_HIP(hipMalloc(&d_fit, sizeof(double) * ntensors * S));
-    guard.p[4] = d_fit;
-    TDX_HIP(hipMemcpyAsync(d_desc, h.data(), sizeof(BDesc) * ntensors, hipMemcpyHostToDevice, s));
-    TDX_HIP(hipMemcpyAsync(d_sched, sched.data(), sizeof(int) * ntensors, hipMemcpyHostToDevice, s));
+    ItemPlan ip;
+    long mf = 0, tf = 0;
+    const bool split = !items && !kVariants[variant].fn;
+    if (items) items_plan(ip, h.data(), ntensors);
+    if (split) {
+        for (long t = 0; t < ntensors; ++t)  // M is laid out like the factors
+            for (int m = 0; m < 3; ++m) mf = std::max(mf, h[t].uoff[m] + (long)dims[3 * t + m] * h[t].R);
+        if (variant_uses_t(variant))
+            for (long t = 0; t < ntensors; ++t) {
+                h[t].toff = tf;
+                tf += (long)h[t].J * h[t].K * h[t].R;
+            }
+    }
+    Parts p;
+    const size_t o_desc = p.add(sizeof(BDesc) * ntensors), o_sched = p.add(sizeof(int) * sched.size());
+    const size_t o_int = p.add(sizeof(int) * 8), o_nx = p.add(sizeof(double) * ntensors);
+    const size_t o_fit = p.add(sizeof(double) * ntensors * S);
+    const size_t o_G = p.add(items || split ? sizeof(double) * ntensors * 3 * kBMaxR * kBMaxR : 0);
+    const size_t o_M = p.add(sizeof(float) * mf), o_T = p.add(sizeof(float) * (items ? ip.t_floats : tf));
+    const size_t o_id = p.add(sizeof(IDesc) * ip.desc.size()), o_it = p.add(sizeof(IItem) * ip.items.size());
+    const size_t o_part = p.add(sizeof(float) * ip.part_floats), o_np = p.add(sizeof(double) * ip.items.size());
+    st = mem.take(p.bytes);
+    if (st) return st;
+    char *base = mem.ptr();
+    BDesc *d_desc = (BDesc *)(base + o_desc);
+    int *d_sched = (int *)(base + o_sched), *d_int = (int *)(base + o_int);
+    double *d_nx = (double *)(base + o_nx), *d_fit = (double *)(base + o_fit);
+    if (!items || init == 0)
+        TDX_HIP(hipMemcpyAsync(d_desc, h.data(), sizeof(BDesc) * ntensors, hipMemcpyHostToDevice, s));
+    if (!items) TDX_HIP(hipMemcpyAsync(d_sched, sched.data(), sizeof(int) * ntensors, hipMemcpyHostToDevice, s));
     int *queue = d_int, *sweep_ctr = d_int + 1, *status = d_int + 2;
     k_batched_prologue<<<1, 1, 0, s>>>(sweep_ctr);
     k_batched_prologue<<<1, 1, 0, s>>>(status);
     if (init == 0) k_batched_init<<<1024, 256, 0, s>>>(U, d_desc, (int)ntensors, seed);
     TDX_LAUNCH_CHECK();
     BmBuffers bm;
-    ItemPlan ip;
     ItemBuffers ib{};
-    const bool items = variant == kItemsVariant;
     if (items) {
-        items_plan(ip, h.data(), ntensors);
-        void **dst[6] = {(void **)&ib.desc, (void **)&ib.items, (void **)&ib.part, (void **)&ib.T, (void **)&ib.G,
-                         (void **)&ib.npart};
-        const size_t bytes[6] = {sizeof(IDesc) * ntensors, sizeof(IItem) * ip.items.size(),
-                                 sizeof(float) * ip.part_floats, sizeof(float) * ip.t_floats,
-                                 sizeof(double) * ntensors * 3 * kBMaxR * kBMaxR, sizeof(double) * ip.items.size()};
-        for (int k = 0; k < 6; ++k) {
-            TDX_HIP(hipMalloc(dst[k], bytes[k]));
-            guard.p[5 + k] = *dst[k];
-        }
+        ib.desc = (IDesc *)(base + o_id);
+        ib.items = (IItem *)(base + o_it);
+        ib.part = (float *)(base + o_part);
+        ib.T = (float *)(base + o_T);
+        ib.G = (double *)(base + o_G);
+        ib.npart = (double *)(base + o_np);
         ib.ntensors = (int)ntensors;
         ib.nitems = (int)ip.items.size();
-        TDX_HIP(hipMemcpyAsync((void *)ib.desc, ip.desc.data(), bytes[0], hipMemcpyHostToDevice, s));
-        TDX_HIP(hipMemcpyAsync((void *)ib.items, ip.items.data(), bytes[1], hipMemcpyHostToDevice, s));
+        TDX_HIP(hipMemcpyAsync((void *)ib.desc, ip.desc.data(), sizeof(IDesc) * ntensors, hipMemcpyHostToDevice, s));
+        TDX_HIP(hipMemcpyAsync((void *)ib.items, ip.items.data(), sizeof(IItem) * ip.items.size(), hipMemcpyHostToDevice,
+                               s));
         k_batched_set<<<1, 1, 0, s>>>(sweep_ctr, -1);
-        const int st = items_prologue(ib, X, U, d_nx, s);
+        st = items_prologue(ib, X, U, d_nx, s);
         if (st) return st;
     } else {
         k_batched_norm2<<<1024, 256, 0, s>>>(X, d_desc, (int)ntensors, d_nx);
         TDX_LAUNCH_CHECK();
     }
-    if (!items && !kVariants[variant].fn) {
-        long mf = 0;  // M is laid out like the factors
-        for (long t = 0; t < ntensors; ++t)
-            for (int m = 0; m < 3; ++m) mf = std::max(mf, h[t].uoff[m] + (long)dims[3 * t + m] * h[t].R);
-        TDX_HIP(hipMalloc(&bm.M, sizeof(float) * mf));
-        guard.p[5] = bm.M;
-        TDX_HIP(hipMalloc(&bm.G, sizeof(double) * ntensors * 3 * kBMaxR * kBMaxR));
-        guard.p[6] = bm.G;
-        if (variant_uses_t(variant)) {
-            long tf = 0;
-            for (long t = 0; t < ntensors; ++t) {
-                h[t].toff = tf;
-                tf += (long)h[t].J * h[t].K * h[t].R;
-            }
-            TDX_HIP(hipMalloc(&bm.T, sizeof(float) * tf));
-            guard.p[7] = bm.T;
-            TDX_HIP(hipMemcpyAsync(d_desc, h.data(), sizeof(BDesc) * ntensors, hipMemcpyHostToDevice, s));
-        }
+    if (split) {
+        bm.M = (float *)(base + o_M);
+        bm.G = (double *)(base + o_G);
+        if (variant_uses_t(variant)) bm.T = (float *)(base + o_T);
         bm.queues = d_int + 3;
         k_bm_gram_init<<<1024, 256, 0, s>>>(U, d_desc, (int)ntensors, bm.G);
         TDX_LAUNCH_CHECK();
     }
-    // capture one sweep
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    TDX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int st = items ? items_sweep(ib, X, U, d_nx, d_fit, S, sweep_ctr, status, s)
-                   : launch_variant(variant, s, X, U, d_desc, d_sched, (int)ntensors, queue, d_nx, d_fit, S, sweep_ctr,
-                                    status, bm);
-    hipError_t e = hipStreamEndCapture(s, &g);
-    if (st) {
-        if (g) (void)hipGraphDestroy(g);
-        return st;
-    }
-    if (e != hipSuccess) return record_hip(e, "hipStreamEndCapture", __FILE__, __LINE__);
-    e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(g);
-        return record_hip(e, "hipGraphInstantiate", __FILE__, __LINE__);
+    // One sweep: six plain launches of the item design, which take the host less than they take the
+    // GPU (a captured graph cost 40 us before its first launch and as much for each later one, and
+    // while it was recorded no other thread could use the default stream); a graph of the others.
+    struct Graph {
+        hipGraph_t g = nullptr;
+        hipGraphExec_t e = nullptr;
+        ~Graph() {
+            if (e) (void)hipGraphExecDestroy(e);
+            if (g) (void)hipGraphDestroy(g);
+        }
+    } graph;
+    hipError_t e = hipSuccess;
+    if (!items) {
+        TDX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        st = launch_variant(variant, s, X, U, d_desc, d_sched, (int)ntensors, queue, d_nx, d_fit, S, sweep_ctr, status,
+                            bm);
+        e = hipStreamEndCapture(s, &graph.g);
+        if (st) return st;
+        if (e != hipSuccess) return record_hip(e, "hipStreamEndCapture", __FILE__, __LINE__);
+        e = hipGraphInstantiate(&graph.e, graph.g, nullptr, nullptr, 0);
+        if (e != hipSuccess) return record_hip(e, "hipGraphInstantiate", __FILE__, __LINE__);
     }
     std::vector<hipEvent_t> evs(sweeps + 1);
     for (auto &ev : evs) (void)hipEventCreate(&ev);
     (void)hipEventRecord(evs[0], s);
-    for (int it = 0; it < sweeps && e == hipSuccess; ++it) {
-        e = hipGraphLaunch(ge, s);
+    for (int it = 0; it < sweeps && e == hipSuccess && !st; ++it) {
+        if (items) st = items_sweep(ib, X, U, d_nx, d_fit, S, sweep_ctr, status, s);
+        else e = hipGraphLaunch(graph.e, s);
         if (e == hipSuccess) e = hipEventRecord(evs[it + 1], s);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e == hipSuccess && sweep_ms)
         for (int it = 0; it < sweeps; ++it) (void)hipEventElapsedTime(&sweep_ms[it], evs[it], evs[it + 1]);
     for (auto &ev : evs) (void)hipEventDestroy(ev);
-    (void)hipGraphExecDestroy(ge);
-    (void)hipGraphDestroy(g);
+    if (st) return st;
     if (e != hipSuccess) return record_hip(e, "batched sweeps", __FILE__, __LINE__);
     if (fit_hist && sweeps > 0)
         TDX_HIP(hipMemcpy(fit_hist, d_fit, sizeof(double) * ntensors * S, hipMemcpyDeviceToHost));
     int hs = 0;
     TDX_HIP(hipMemcpy(&hs, status, sizeof(int), hipMemcpyDeviceToHost));
+    mem.done();
+    owned.done();
     return record(hs ? TDX_WARN_SINGULAR : TDX_OK);
 }
 

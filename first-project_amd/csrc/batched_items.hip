@@ -462,10 +462,19 @@ void items_plan(ItemPlan &p, const BDesc *d, long n) {
         p.part_floats += (long)q.nit * q.pstep;
         p.t_floats += (long)q.J * q.K * q.Rq;
     }
-    std::stable_sort(p.items.begin(), p.items.end(), [&](const IItem &a, const IItem &b) {
-        const IDesc &x = p.desc[a.t], &y = p.desc[b.t];
-        return (long)(a.k1 - a.k0) * x.I * x.J > (long)(b.k1 - b.k0) * y.I * y.J;
-    });
+    // largest first, in 64 classes of size (a comparison sort of the 4-5 thousand items of 1024 tensors
+    // took 0.2 ms)
+    constexpr int kClasses = 64;
+    long most = 1;
+    auto size = [&](const IItem &a) { return (long)(a.k1 - a.k0) * p.desc[a.t].I * p.desc[a.t].J; };
+    for (const IItem &a : p.items) most = std::max(most, size(a));
+    auto cls = [&](const IItem &a) { return kClasses - 1 - (int)(size(a) * (kClasses - 1) / most); };
+    size_t at[kClasses + 1] = {0};
+    for (const IItem &a : p.items) ++at[cls(a) + 1];
+    for (int c = 0; c < kClasses; ++c) at[c + 1] += at[c];
+    std::vector<IItem> sorted(p.items.size());
+    for (const IItem &a : p.items) sorted[at[cls(a)]++] = a;
+    p.items.swap(sorted);
 }
 
 int items_prologue(const ItemBuffers &b, const float *X, const float *U, double *normx2, hipStream_t s) {

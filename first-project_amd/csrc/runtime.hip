@@ -59,6 +59,123 @@ void release_workspace() {
     }
 }
 
+static constexpr int kIdleBlocks = 4, kIdleStreams = 4;
+static constexpr size_t kIdleBytes = size_t(2) << 30;
+struct IdleBlock {
+    void *p;
+    size_t bytes;
+    int dev;
+};
+struct IdleStream {
+    hipStream_t s;
+    int dev;
+};
+static std::mutex g_lease_mutex;
+static IdleBlock g_idle[kIdleBlocks];
+static int g_nidle = 0;
+static IdleStream g_idle_streams[kIdleStreams];
+static int g_nidle_streams = 0;
+
+// frees the idle blocks and streams (of one device; -1: of every device)
+static void free_idle(int dev) {
+    std::lock_guard<std::mutex> lk(g_lease_mutex);
+    int n = 0;
+    for (int i = 0; i < g_nidle; ++i) {
+        if (dev >= 0 && g_idle[i].dev != dev) g_idle[n++] = g_idle[i];
+        else (void)hipFree(g_idle[i].p);
+    }
+    g_nidle = n;
+    n = 0;
+    for (int i = 0; i < g_nidle_streams; ++i) {
+        if (dev >= 0 && g_idle_streams[i].dev != dev) g_idle_streams[n++] = g_idle_streams[i];
+        else (void)hipStreamDestroy(g_idle_streams[i].s);
+    }
+    g_nidle_streams = n;
+}
+
+void release_leases() { free_idle(-1); }
+
+int DeviceLease::take(size_t bytes) {
+    TDX_HIP(hipGetDevice(&dev_));
+    {
+        std::lock_guard<std::mutex> lk(g_lease_mutex);
+        int best = -1;
+        for (int i = 0; i < g_nidle; ++i)
+            if (g_idle[i].dev == dev_ && g_idle[i].bytes >= bytes && (best < 0 || g_idle[i].bytes < g_idle[best].bytes))
+                best = i;
+        if (best >= 0) {
+            p_ = g_idle[best].p;
+            bytes_ = g_idle[best].bytes;
+            g_idle[best] = g_idle[--g_nidle];
+            return TDX_OK;
+        }
+    }
+    hipError_t e = hipMalloc(&p_, bytes < 256 ? 256 : bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        free_idle(dev_);
+        e = hipMalloc(&p_, bytes < 256 ? 256 : bytes);
+    }
+    if (e != hipSuccess) {
+        p_ = nullptr;
+        return record_hip(e, "hipMalloc", __FILE__, __LINE__);
+    }
+    bytes_ = bytes < 256 ? 256 : bytes;
+    return TDX_OK;
+}
+
+DeviceLease::~DeviceLease() {
+    if (!p_) return;
+    if (done_) {
+        std::lock_guard<std::mutex> lk(g_lease_mutex);
+        size_t held = bytes_;
+        int least = 0;
+        for (int i = 0; i < g_nidle; ++i) {
+            held += g_idle[i].bytes;
+            if (g_idle[i].bytes < g_idle[least].bytes) least = i;
+        }
+        if (g_nidle < kIdleBlocks && held <= kIdleBytes) {
+            g_idle[g_nidle++] = IdleBlock{p_, bytes_, dev_};
+            return;
+        }
+        // (a full set of idle blocks: the smallest goes)
+        if (g_nidle == kIdleBlocks && g_idle[least].bytes < bytes_ && held - g_idle[least].bytes <= kIdleBytes) {
+            void *old = g_idle[least].p;
+            g_idle[least] = IdleBlock{p_, bytes_, dev_};
+            p_ = old;
+        }
+    }
+    (void)hipFree(p_);
+}
+
+int StreamLease::take() {
+    TDX_HIP(hipGetDevice(&dev_));
+    {
+        std::lock_guard<std::mutex> lk(g_lease_mutex);
+        for (int i = 0; i < g_nidle_streams; ++i)
+            if (g_idle_streams[i].dev == dev_) {
+                s_ = g_idle_streams[i].s;
+                g_idle_streams[i] = g_idle_streams[--g_nidle_streams];
+                return TDX_OK;
+            }
+    }
+    TDX_HIP(hipStreamCreate(&s_));
+    return TDX_OK;
+}
+
+StreamLease::~StreamLease() {
+    if (!s_) return;
+    (void)hipStreamSynchronize(s_);
+    if (done_) {
+        std::lock_guard<std::mutex> lk(g_lease_mutex);
+        if (g_nidle_streams < kIdleStreams) {
+            g_idle_streams[g_nidle_streams++] = IdleStream{s_, dev_};
+            return;
+        }
+    }
+    (void)hipStreamDestroy(s_);
+}
+
 int device_cus() {
     static int cache[64] = {0};
     int dev = 0;
@@ -136,6 +253,7 @@ int tdx_copy_to_device(void *dst, const void *src, size_t bytes) {
 int tdx_release_workspace(void) {
     tdx::release_cp_plans();
     tdx::release_workspace();
+    tdx::release_leases();
     return tdx::record(TDX_OK);
 }
 

@@ -138,11 +138,8 @@ struct TuckerWs {
     double *Q = nullptr;
     float *y0 = nullptr, *y1 = nullptr, *y2 = nullptr;
     double *scal = nullptr;
-    ~TuckerWs() {
-        void *ps[] = {gram_part, G, Q, y0, y1, y2, scal};
-        for (void *p : ps)
-            if (p) (void)hipFree(p);
-    }
+    uint16_t *xb = nullptr;
+    DeviceLease mem;  // all of it
 };
 
 static int unfold_gram(const void *X, int xtype, int order, const long *dims, int mode, TuckerWs &W, double *G,
@@ -203,12 +200,8 @@ static int top_eigvecs(const EigJob *jobs, int njobs, int try_sub, hipStream_t s
     return TDX_OK;
 }
 
-static int ws_setup(TuckerWs &W, int order, const long *dims, const long *ranks) {
+static int ws_setup(TuckerWs &W, int order, const long *dims, const long *ranks, bool bf16) {
     W.gram_blocks = 1024;
-    TDX_HIP(hipMalloc(&W.gram_part, sizeof(float) * (size_t)W.gram_blocks * kGramMaxN * kGramMaxN));
-    TDX_HIP(hipMalloc(&W.G, sizeof(double) * 4 * kGramMaxN * kGramMaxN));
-    TDX_HIP(hipMalloc(&W.Q, sizeof(double) * 8 * kGramMaxN * kGramMaxN));
-    TDX_HIP(hipMalloc(&W.scal, sizeof(double) * 2048));
     // largest intermediate of a TTM chain: the first contraction of the biggest mode
     long N = 1;
     for (int m = 0; m < order; ++m) N *= dims[m];
@@ -217,9 +210,24 @@ static int ws_setup(TuckerWs &W, int order, const long *dims, const long *ranks)
         long sz = N / dims[m] * ranks[m];
         if (sz > maxsz) maxsz = sz;
     }
-    TDX_HIP(hipMalloc(&W.y0, sizeof(float) * maxsz));
-    TDX_HIP(hipMalloc(&W.y1, sizeof(float) * maxsz));
-    TDX_HIP(hipMalloc(&W.y2, sizeof(float) * maxsz));
+    Parts p;
+    const size_t gp = p.add(sizeof(float) * (size_t)W.gram_blocks * kGramMaxN * kGramMaxN);
+    const size_t g = p.add(sizeof(double) * 4 * kGramMaxN * kGramMaxN);
+    const size_t q = p.add(sizeof(double) * 8 * kGramMaxN * kGramMaxN);
+    const size_t sc = p.add(sizeof(double) * 2048);
+    const size_t y0 = p.add(sizeof(float) * maxsz), y1 = p.add(sizeof(float) * maxsz), y2 = p.add(sizeof(float) * maxsz);
+    const size_t xb = p.add(bf16 ? sizeof(uint16_t) * N : 0);
+    const int st = W.mem.take(p.bytes);
+    if (st) return st;
+    char *b = W.mem.ptr();
+    W.gram_part = (float *)(b + gp);
+    W.G = (double *)(b + g);
+    W.Q = (double *)(b + q);
+    W.scal = (double *)(b + sc);
+    W.y0 = (float *)(b + y0);
+    W.y1 = (float *)(b + y1);
+    W.y2 = (float *)(b + y2);
+    W.xb = (uint16_t *)(b + xb);
     return TDX_OK;
 }
 
@@ -262,25 +270,17 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
     }
     hipStream_t s = stream();
     TuckerWs W;
-    int st = ws_setup(W, order, dims, ranks);
+    int st = ws_setup(W, order, dims, ranks, bf16 != 0);
     if (st) return st;
     long N = 1;
     for (int m = 0; m < order; ++m) N *= dims[m];
     // BF16 storage: the Grams of X and the first TTM of every chain stream a BF16 copy
     const void *Xs = X;
     int xtype = TDX_F32;
-    uint16_t *Xb = nullptr;
-    struct FreeB {
-        uint16_t *&p;
-        ~FreeB() {
-            if (p) (void)hipFree(p);
-        }
-    } freeb{Xb};
     if (bf16) {
-        TDX_HIP(hipMalloc(&Xb, sizeof(uint16_t) * N));
-        st = tdx_quantize_bf16(X, Xb, N);
+        st = tdx_quantize_bf16(X, W.xb, N);
         if (st) return st;
-        Xs = Xb;
+        Xs = W.xb;
         xtype = TDX_BF16;
     }
     // HOSVD init (only the spans matter when HOOI iterations follow: every later product
@@ -366,6 +366,7 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
         st = ttm_generic(Y, order, ydims, order - 1, U[order - 1], dims[order - 1], 1, ranks[order - 1], core, s);
     if (st) return st;
     TDX_HIP(hipStreamSynchronize(s));
+    W.mem.done();
     return TDX_OK;
 }
 
@@ -381,9 +382,14 @@ int tdx_unfold_gram_ex(const void *X, int dtype, int order, const long *dims, in
     for (int m = 0; m < order; ++m) TDX_CHECK_ARG(dims[m] > 0);
     TuckerWs W;
     W.gram_blocks = 1024;
-    TDX_HIP(hipMalloc(&W.gram_part, sizeof(float) * (size_t)W.gram_blocks * kGramMaxN * kGramMaxN));
-    int st = unfold_gram(X, dtype, order, dims, mode, W, G, stream());
-    if (!st) TDX_HIP(hipStreamSynchronize(stream()));
+    int st = W.mem.take(sizeof(float) * (size_t)W.gram_blocks * kGramMaxN * kGramMaxN);
+    if (st) return st;
+    W.gram_part = (float *)W.mem.ptr();
+    st = unfold_gram(X, dtype, order, dims, mode, W, G, stream());
+    if (!st) {
+        TDX_HIP(hipStreamSynchronize(stream()));
+        W.mem.done();
+    }
     return record(st);
 }
 
