@@ -32,20 +32,9 @@ namespace tdx {
 static constexpr int kSolveRows = 16;  // rows per k_solve workgroup
 static constexpr int kGramRows = 64;   // rows per Gram-partial workgroup
 
-// gram_part != nullptr: first G_gmode (Gsum) = the ordered sum of the nblk Gram partials of
-// that mode (what k_gram_psum computes, same order), so a small-rank sweep, whose inverses
-// run in line, needs no separate Gram kernel between a solve and the next mode's inverse.
 template <int NS>
-__global__ __launch_bounds__(256) void k_vinv(const double *G0, const double *G1, const double *G2, const double *G3,
-                                              int order, int mode, int R, double *__restrict__ Vinv,
-                                              int *__restrict__ status, double *__restrict__ fb_ws,
-                                              const double *__restrict__ gram_part, int nblk, double *Gsum) {
-    const double *G[4] = {G0, G1, G2, G3};
-    if (gram_part) {
-        for (int e = threadIdx.x; e < R * R; e += blockDim.x) Gsum[e] = ordered_sum(gram_part + e, (long)R * R, nblk);
-        __syncthreads();
-    }
-    vinv_block<NS>(G, order, mode, R, Vinv, status, fb_ws);
+__global__ __launch_bounds__(256) void k_vinv(VinvJob j) {
+    vinv_job<NS>(j);
 }
 
 // M = sum of the split-K partials of the MTTKRP, FP64, in split order (deterministic);
@@ -958,18 +947,18 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
         return R > 16 && (dt || S.mp[n].rowtiles * (long)S.mp[n].nsplit <= device_cus());
     };
     // gmode >= 0: the inverse first sums mode gmode's Gram partials (gnblk blocks) into G_gmode
-    auto launch_vinv = [&](int n, hipStream_t vs, int gmode = -1, int gnblk = 0) {
-        const double *g2 = P.order > 2 ? P.G[2] : P.G[0], *g3 = P.order > 3 ? P.G[3] : P.G[0];
-        const double *gp = gmode >= 0 ? P.gram_part : nullptr;
-        double *gs = gmode >= 0 ? P.G[gmode] : nullptr;
-        if (R <= 16) k_vinv<4><<<1, 256, 0, vs>>>(P.G[0], P.G[1], g2, g3, P.order, n, R, P.Vinv[n], P.status,
-                                                P.vinv_ws, gp, gnblk, gs);
-        else if (R <= 32) k_vinv<8><<<1, 256, 0, vs>>>(P.G[0], P.G[1], g2, g3, P.order, n, R, P.Vinv[n], P.status,
-                                                     P.vinv_ws, gp, gnblk, gs);
-        else k_vinv<16><<<1, 256, 0, vs>>>(P.G[0], P.G[1], g2, g3, P.order, n, R, P.Vinv[n], P.status,
-                                         P.vinv_ws, gp, gnblk, gs);
+    auto vinv_of = [&](int n, int gmode = -1, int gnblk = 0) {
+        return VinvJob{{P.G[0], P.G[1], P.order > 2 ? P.G[2] : P.G[0], P.order > 3 ? P.G[3] : P.G[0]},
+                       P.order, n, R, P.Vinv[n], P.status, P.vinv_ws,
+                       gmode >= 0 ? P.gram_part : nullptr, gnblk, gmode >= 0 ? P.G[gmode] : nullptr};
     };
-    // R <= 16 (every inverse in line): mode n's Gram is summed by mode n + 1's inverse
+    auto launch_vinv = [&](int n, hipStream_t vs, int gmode = -1, int gnblk = 0) {
+        const VinvJob j = vinv_of(n, gmode, gnblk);
+        if (R <= 16) k_vinv<4><<<1, 256, 0, vs>>>(j);
+        else if (R <= 32) k_vinv<8><<<1, 256, 0, vs>>>(j);
+        else k_vinv<16><<<1, 256, 0, vs>>>(j);
+    };
+    // R <= 16 (every inverse in line or with the MTTKRP): mode n's Gram is summed by mode n + 1's inverse
     int pending_gram = -1, pending_nblk = 0;
     int prev_nblk = 0;  // Gram-partial blocks of the mode whose Gram a forked branch sums
     // forked[n]: the fork point of mode n's inverse was recorded after the previous mode's
@@ -983,7 +972,12 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
     for (int n = 0; n < P.order; ++n) {
         const bool dt = S.dt.on && n > 0;
         const bool beside = beside_of(n);
-        if (!forked[n] && !(fuse2 && n == 2)) {
+        VinvJob with{};  // the inverse that runs in the MTTKRP's own launch
+        const bool inside = !beside && !dt && mttkrp_takes_inverse(S.mp[n]);
+        if (inside) {
+            with = vinv_of(n, pending_gram, pending_nblk);
+            pending_gram = -1;
+        } else if (!forked[n] && !(fuse2 && n == 2)) {
             if (beside) {
                 TDX_HIP(hipEventRecord(P.ev_fork[n], s));
             } else {
@@ -1011,7 +1005,7 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
             nsplit = S.dt.nsplit2;
             rows_pad = S.dt.I2;
         } else {
-            st = mttkrp_launch(S.mp[n], S.X, panels, row_scale, P.partial, s, skip);
+            st = mttkrp_launch(S.mp[n], S.X, panels, row_scale, P.partial, s, skip, inside ? &with : nullptr);
         }
         if (st) return st;
         if (beside) {

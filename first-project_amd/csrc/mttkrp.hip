@@ -604,7 +604,8 @@ static void launch_fast(const MttkrpPlan &p, const KArgs &a, hipStream_t s) {
 }
 
 int mttkrp_launch(const MttkrpPlan &p, const void *X, const float *const *panels, const float *row_scale,
-                  float *partial, hipStream_t s, const int *skip) {
+                  float *partial, hipStream_t s, const int *skip, const VinvJob *inverse) {
+    if (inverse && !mttkrp_takes_inverse(p)) return record(TDX_ERR_UNSUPPORTED);
     KArgs a{};
     a.skip = skip;
     a.X = X;
@@ -632,7 +633,7 @@ int mttkrp_launch(const MttkrpPlan &p, const void *X, const float *const *panels
         if (m != p.mode && m != a.fmode) a.slow[a.nslow++] = m;
     const int stt = storage_type(p.dtype);
     if (p.dtype == TDX_FP8_E4M3 && p.mode == 0 && !row_scale) return record(TDX_ERR_ARG);
-    if (p.lds && p.dtype == TDX_F32) return mttkrp_f32_launch(p, X, panels, partial, s, skip);
+    if (p.lds && p.dtype == TDX_F32) return mttkrp_f32_launch(p, X, panels, partial, s, skip, inverse);
     if (p.lds) return mttkrp_lds_launch(p, X, panels, row_scale, partial, s, skip);
     if (p.split) return record(TDX_ERR_UNSUPPORTED);  // the split block exists in the LDS kernel only
     if (p.fast) {

@@ -42,8 +42,14 @@ int mttkrp_plan(MttkrpPlan &p, int order, const long *dims, int mode, int dtype,
 // Launches the split-K MTTKRP writing partial[split][row][Rp] (FP32).
 // panels[m] are factor panels (panels[mode] unused); for FP8 storage panels[0] must be
 // pre-scaled by the slice scales when mode != 0, and row_scale = scales when mode == 0.
+// inverse: a CP-ALS inverse to run in the same launch, where mttkrp_takes_inverse says so.
+struct VinvJob;
 int mttkrp_launch(const MttkrpPlan &p, const void *X, const float *const *panels,
-                  const float *row_scale, float *partial, hipStream_t s, const int *skip = nullptr);
+                  const float *row_scale, float *partial, hipStream_t s, const int *skip = nullptr,
+                  const VinvJob *inverse = nullptr);
+// FP32 kernel at rank <= 16: a third workgroup fits on a CU, so the inverse costs no MTTKRP workgroup
+// its place (at higher ranks a CU holds two, and the last one would wait for it)
+inline bool mttkrp_takes_inverse(const MttkrpPlan &p) { return p.lds && p.dtype == TDX_F32 && p.Rp == 16; }
 
 // the LDS-staged kernel (mttkrp_lds.hip; BF16 and FP8 storage)
 bool mttkrp_lds_covers(int order, int mode, long rank, long In, int dtype);
@@ -52,7 +58,7 @@ int mttkrp_lds_launch(const MttkrpPlan &p, const void *X, const float *const *pa
 
 // FP32 storage on the plan of the LDS-staged kernel (mttkrp_f32.hip)
 int mttkrp_f32_launch(const MttkrpPlan &p, const void *X, const float *const *panels, float *partial, hipStream_t s,
-                      const int *skip);
+                      const int *skip, const VinvJob *inverse);
 
 // the kernel for the remaining shapes and alignments (mttkrp_any.hip): completes a plan whose
 // order, extents, mode, storage and rank are set; partial rows are exactly the output rows

@@ -155,4 +155,28 @@ __device__ __forceinline__ void vinv_block(const double *const *G, int order, in
     }
 }
 
+// The inverse of a sweep's mode.  gram_part != nullptr: first G_gmode (Gsum) = the ordered sum of the
+// nblk Gram partials of that mode (what k_gram_psum computes, same order), so a small-rank sweep,
+// whose inverses run in line or with the MTTKRP, needs no separate Gram kernel between a solve and
+// the next mode's inverse.
+struct VinvJob {
+    const double *G[4];
+    int order, mode, R;
+    double *Vinv;
+    int *status;
+    double *fb_ws;
+    const double *gram_part;
+    int nblk;
+    double *Gsum;
+};
+template <int NS>
+__device__ __forceinline__ void vinv_job(const VinvJob &j) {
+    if (j.gram_part) {
+        for (int e = threadIdx.x; e < j.R * j.R; e += blockDim.x)
+            j.Gsum[e] = ordered_sum(j.gram_part + e, (long)j.R * j.R, j.nblk);
+        __syncthreads();
+    }
+    vinv_block<NS>(j.G, j.order, j.mode, j.R, j.Vinv, j.status, j.fb_ws);
+}
+
 }  // namespace tdx
