@@ -1097,10 +1097,14 @@ static int enqueue_ls(CpPlan &P, const Storage &S, hipStream_t s) {
     return TDX_OK;
 }
 
+// The captured sweep of a phase.  Its launches run on after the host has enqueued them, so it is
+// destroyed only when its stream has finished: a call keeps the graphs of all its phases to its end.
 struct SweepGraph {
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
+    hipStream_t s = nullptr;
     ~SweepGraph() {
+        if (ge) (void)hipStreamSynchronize(s);
         if (ge) (void)hipGraphExecDestroy(ge);
         if (g) (void)hipGraphDestroy(g);
     }
@@ -1117,20 +1121,21 @@ static int capture_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit, S
     }
     if (e != hipSuccess) return record_hip(e, "hipStreamEndCapture", __FILE__, __LINE__);
     G.g = g;
+    G.s = s;
     TDX_HIP(hipGraphInstantiate(&G.ge, g, nullptr, nullptr, 0));
     return TDX_OK;
 }
 
 // Runs `sweeps` sweeps on storage S; records per-sweep ms if sweep_ms != NULL, and the device
-// time from the event `origin` to the end of every sweep if elapsed_ms != NULL.
-static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bool fit, bool graph, float *sweep_ms,
+// time from the event `origin` to the end of every sweep if elapsed_ms != NULL.  G: the phase's graph
+// (none is captured for a null one); the sweeps may still run on return.
+static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bool fit, SweepGraph *G, float *sweep_ms,
                       double tol, double target, int *done, hipEvent_t origin = nullptr,
                       float *elapsed_ms = nullptr) {
     *done = 0;
     if (sweeps <= 0) return TDX_OK;
-    SweepGraph G;
-    if (graph) {
-        int st = capture_sweep(P, S, s, fit, G);
+    if (G) {
+        int st = capture_sweep(P, S, s, fit, *G);
         if (st) return st;
     }
     if (!origin) elapsed_ms = nullptr;
@@ -1146,8 +1151,8 @@ static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bo
     double prev = -1.0;
     int st = TDX_OK;
     for (int it = 0; it < sweeps; ++it) {
-        if (graph) {
-            hipError_t e = hipGraphLaunch(G.ge, s);
+        if (G) {
+            hipError_t e = hipGraphLaunch(G->ge, s);
             if (e != hipSuccess) { st = record_hip(e, "hipGraphLaunch", __FILE__, __LINE__); break; }
         } else {
             st = enqueue_sweep(P, S, s, fit);
@@ -1381,15 +1386,17 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     }
     float *elapsed = opt.trace ? opt.trace->elapsed_ms : nullptr;
     int done_open = 0, done_main = 0, done_ref = 0;
+    SweepGraph graphs[3];
+    auto graph_of = [&](int phase) { return opt.use_graph ? &graphs[phase] : nullptr; };
     st = refresh_factors(P, opening ? Sopen : Smain, s);
     (void)hipEventRecord(evg.e[1], s);
     if (!st && opening > 0) {
-        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, opt.use_graph != 0, sweep_ms, 0.0, 0.0, &done_open,
+        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, graph_of(0), sweep_ms, 0.0, 0.0, &done_open,
                         evg.e[0], elapsed);
         if (!st) st = refresh_factors(P, Smain, s);
     }
     if (!st)
-        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, opt.use_graph != 0,
+        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, graph_of(1),
                         sweep_ms ? sweep_ms + done_open : nullptr, opt.tol,
                         opt.storage == TDX_F32 ? opt.target_relerr : 0.0, &done_main, evg.e[0],
                         elapsed ? elapsed + done_open : nullptr);
@@ -1398,7 +1405,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
         // FP32 refinement: the mode-0 panel must be unscaled again (rebuilt by the first solve)
         st = refresh_factors(P, S32, s);
         if (!st)
-            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, opt.use_graph != 0,
+            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, graph_of(2),
                             sweep_ms ? sweep_ms + done_main : nullptr, 0.0, 0.0, &done_ref, evg.e[0],
                             elapsed ? elapsed + done_main : nullptr);
     }

@@ -890,13 +890,15 @@ int tdx_cp_als_batched(const float *X, float *U, const long *dims, const long *r
     // GPU (a captured graph cost 40 us before its first launch and as much for each later one, and
     // while it was recorded no other thread could use the default stream); a graph of the others.
     struct Graph {
+        hipStream_t s;
         hipGraph_t g = nullptr;
         hipGraphExec_t e = nullptr;
-        ~Graph() {
+        ~Graph() {  // (its launches have finished, also where a later step failed)
+            if (e) (void)hipStreamSynchronize(s);
             if (e) (void)hipGraphExecDestroy(e);
             if (g) (void)hipGraphDestroy(g);
         }
-    } graph;
+    } graph{s};
     hipError_t e = hipSuccess;
     if (!items) {
         TDX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));

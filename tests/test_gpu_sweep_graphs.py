@@ -1,0 +1,26 @@
+"""The captured sweeps of a call's phases (opening, main, refinement) stay alive while their launches
+run: short mixed calls one after the other, the same bits every time and without a graph."""
+import pytest
+import torch
+
+import tdx
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dims,R", [((120, 98, 87), 33), ((128, 64, 40), 16)])
+def test_repeated_mixed_calls(dims, R):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    X = torch.randn(dims[0] * dims[1] * dims[2], device="cuda", generator=g)
+    U0 = [torch.randn(R, d, device="cuda", generator=g) for d in dims]
+    first = None
+    for k in range(40):
+        o = tdx.default_cp_options()
+        o.init, o.max_sweeps, o.storage = 1, 5, tdx.TDX_BF16
+        o.opening_sweeps, o.opening_split, o.refine_sweeps, o.use_graph = 2, 1, 1, int(k > 0)
+        U = [u.clone() for u in U0]
+        st, rep, _, _ = tdx.cp_als_ex(X, dims, R, U, o)
+        assert st == tdx.TDX_OK and rep.sweeps_done == 6
+        first = first or U
+        assert all(torch.equal(a, b) for a, b in zip(U, first)), k
