@@ -650,7 +650,7 @@ struct CpPlan {
     double *hpart = nullptr;    // k_gram_psum_fit: per-block partials (R^2 / 256 doubles)
     int *fit_done = nullptr;    // k_gram_psum_fit: ticket (0 between launches)
     bool shared_pass = true;    // modes 1 and 2 from one pass over X where eligible
-    uint16_t *T = nullptr;      // shared-pass intermediate X x_0 A^T (BF16, I2 x I1 x Rp)
+    void *T = nullptr;          // shared-pass intermediate X x_0 A^T (dt: BF16; tw: FP32 and A's parts)
     size_t t_bytes = 0;
     int max_sweeps_hist = 0;
     hipStream_t side = nullptr;
@@ -725,6 +725,7 @@ struct Storage {
     const float *scales;  // FP8 slice scales
     MttkrpPlan mp[4];
     DtreePlan dt;         // order 3, BF16/FP8: modes 1 and 2 from one shared pass over X
+    TwPlan tw;            // order 3, FP32 and split BF16: the same with FP32 T
 };
 
 // sets the shape of a plan whose buffers are (or will be) large enough for it
@@ -804,19 +805,31 @@ static int plan_setup(CpPlan &P, int order, const long *dims, long R, float *con
     return TDX_OK;
 }
 
-static int ensure_partial(CpPlan &P, const Storage &S) {
+static int ensure_partial(CpPlan &P, Storage &S) {
     size_t need = 0;
     for (int m = 0; m < P.order; ++m)
         if (S.mp[m].partial_floats() > need) need = S.mp[m].partial_floats();
-    if (S.dt.on) {
-        if (S.dt.partial_floats() > need) need = S.dt.partial_floats();
-        if (S.dt.t_bytes() > P.t_bytes) {
-            if (P.T) TDX_HIP(hipFree(P.T));
+    const size_t tneed = S.dt.on ? S.dt.t_bytes() : S.tw.on ? S.tw.ws_bytes() : 0;
+    if (tneed > P.t_bytes) {
+        if (P.T && !S.tw.on) {
+            TDX_HIP(hipFree(P.T));
             P.T = nullptr;
-            TDX_HIP(hipMalloc(&P.T, S.dt.t_bytes()));
-            P.t_bytes = S.dt.t_bytes();
+            P.t_bytes = 0;
+        }
+        void *t = nullptr;
+        const hipError_t e = hipMalloc(&t, tneed);
+        if (e == hipErrorOutOfMemory && S.tw.on) {
+            (void)hipGetLastError();
+            S.tw.on = false;  // the separate passes need no T
+        } else {
+            TDX_HIP(e);
+            if (P.T) TDX_HIP(hipFree(P.T));
+            P.T = t;
+            P.t_bytes = tneed;
         }
     }
+    if (S.dt.on && S.dt.partial_floats() > need) need = S.dt.partial_floats();
+    if (S.tw.on && S.tw.partial_floats() > need) need = S.tw.partial_floats();
     if (need > P.partial_floats) {
         if (P.partial) TDX_HIP(hipFree(P.partial));
         P.partial = nullptr;
@@ -855,6 +868,7 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     }
     if (ok) *ok = true;
     int st = dtree_plan(S.dt, P.order, P.dims, dtype, P.R, P.shared_pass && !split);
+    if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && (split || dtype == TDX_F32));
     if (st) return st;
     return ensure_partial(P, S);
 }
@@ -941,7 +955,10 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
     // Order 3 with the shared pass, R > 16: mode 2's inverse runs inside the pass over T
     // (k_m2_vinv), after mode 1's Gram sum in line, so mode 2 has no inverse launch of its own.
     const bool fuse2 = S.dt.on && P.order == 3 && R > 16;
+    // The same with FP32 T (FP32 storage, split opening sweeps): the pass over X fills the registers of
+    // every CU, so mode 1's inverse runs in the launch ahead of it, mode 2's in the pass over T.
     auto beside_of = [&](int n) {
+        if (S.tw.on && n > 0) return false;
         if (fuse2 && n == 2) return false;
         const bool dt = S.dt.on && n > 0;
         return R > 16 && (dt || S.mp[n].rowtiles * (long)S.mp[n].nsplit <= device_cus());
@@ -972,8 +989,9 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
     for (int n = 0; n < P.order; ++n) {
         const bool dt = S.dt.on && n > 0;
         const bool beside = beside_of(n);
-        VinvJob with{};  // the inverse that runs in the MTTKRP's own launch
-        const bool inside = !beside && !dt && mttkrp_takes_inverse(S.mp[n]);
+        VinvJob with{};  // the inverse that runs in one of the MTTKRP's own launches
+        const bool tw = S.tw.on && n > 0;
+        const bool inside = tw || (!beside && !dt && mttkrp_takes_inverse(S.mp[n]));
         if (inside) {
             with = vinv_of(n, pending_gram, pending_nblk);
             pending_gram = -1;
@@ -993,17 +1011,25 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
         int nsplit = S.mp[n].nsplit;
         long rows_pad = S.mp[n].rows_pad;
         if (dt && n == 1) {
-            st = dtree_m1_launch(S.dt, S.X, P.panel[0], P.U[2], P.T, P.partial, s);
+            st = dtree_m1_launch(S.dt, S.X, P.panel[0], P.U[2], (uint16_t *)P.T, P.partial, s);
             nsplit = S.dt.nsplit1;
             rows_pad = S.dt.I1;
         } else if (dt && n == 2) {
             if (fuse2)
-                st = dtree_m2_vinv_launch(S.dt, P.T, P.panel[1], P.partial, P.G[0], P.G[1], R, P.Vinv[2],
+                st = dtree_m2_vinv_launch(S.dt, (const uint16_t *)P.T, P.panel[1], P.partial, P.G[0], P.G[1], R, P.Vinv[2],
                                           P.status, P.vinv_ws, s);
             else
-                st = dtree_m2_launch(S.dt, P.T, P.panel[1], P.partial, s);
+                st = dtree_m2_launch(S.dt, (const uint16_t *)P.T, P.panel[1], P.partial, s);
             nsplit = S.dt.nsplit2;
             rows_pad = S.dt.I2;
+        } else if (tw && n == 1) {
+            st = tw_m1_launch(S.tw, S.X, P.panel[0], P.panel[2], P.T, P.partial, with, s);
+            nsplit = S.tw.nsplit1;
+            rows_pad = S.tw.rows_pad1();
+        } else if (tw) {
+            st = tw_m2_launch(S.tw, P.T, P.panel[1], P.partial, with, s);
+            nsplit = S.tw.nsplit2;
+            rows_pad = S.tw.I2;
         } else {
             st = mttkrp_launch(S.mp[n], S.X, panels, row_scale, P.partial, s, skip, inside ? &with : nullptr);
         }

@@ -105,6 +105,33 @@ int dtree_m2_vinv_launch(const DtreePlan &d, const uint16_t *T, const float *pan
                          const double *G0, const double *G1, int R, double *Vinv, int *status, double *fb_ws,
                          hipStream_t s);
 
+// the same pass with FP32 T, for FP32 storage and BF16 storage with hi + lo coefficients
+// (dtree_wide.hip)
+struct TwPlan {
+    bool on = false;
+    int st = 0, Rp = 0, nfc = 0, chunk_ops = 0;  // st 0: FP32, 1: BF16; chunks of I0, 16-byte operands each
+    long I0 = 0, I1 = 0, I2 = 0;
+    int blocks_i1 = 0, nsplit1 = 0, i2per = 0;   // grid of the pass over X
+    int nsplit2 = 0, tper = 0, nb2 = 0;          // and of the pass over T
+    size_t lds = 0;
+    long rows_pad1() const { return blocks_i1 * 256L; }
+    size_t t_bytes() const { return sizeof(float) * (size_t)((I1 + 31) / 32 * 32) * I2 * Rp; }
+    // T, A's parts, its columns' scales and a flag
+    size_t ws_bytes() const { return t_bytes() + 16 * (size_t)nfc * chunk_ops + sizeof(float) * (Rp + 16); }
+    size_t partial_floats() const {
+        const size_t a = (size_t)nsplit1 * rows_pad1() * Rp, b = (size_t)nsplit2 * I2 * Rp;
+        return a > b ? a : b;
+    }
+};
+// fills p (p.on = false where the separate passes are used)
+int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled);
+// partial[split][i1][Rp] (nsplit1 splits, rows_pad1() rows), T in ws and the inverse
+int tw_m1_launch(const TwPlan &p, const void *X, const float *panelA, const float *panelC, void *ws, float *partial,
+                 const VinvJob &inverse, hipStream_t s);
+// partial[split][i2][Rp] (nsplit2 splits, I2 rows) from T and the mode-1 panel, and the inverse
+int tw_m2_launch(const TwPlan &p, const void *ws, const float *panelB, float *partial, const VinvJob &inverse,
+                 hipStream_t s);
+
 // packs the panels of every factor but `skip` (-1: all) in one launch; scale0 (or null): row i
 // of the mode-0 factor is multiplied by scale0[i]
 int pack_panels(int order, const long *dims, int skip, const float *const *U, long R, int Rp, const float *scale0,
