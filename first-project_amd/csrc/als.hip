@@ -273,27 +273,53 @@ __global__ __launch_bounds__(256) void k_gram_psum_fit(const double *__restrict_
     }
 }
 
+// Gram partial of 64 rows: a thread a 4 x 4 block of it, 256 / ceil(R / 4)^2 groups of threads sharing
+// the rows (1024 x 64: 13 us; 22 with an entry a thread, two LDS reads a multiply-add).
 __global__ __launch_bounds__(256) void k_gram_rows(const float *__restrict__ U, long I, int R,
                                                    double *__restrict__ gram_part) {
     __shared__ double Us[kGramRows * kMaxR];
+    static_assert(kGramRows * kMaxR >= 16 * 256, "the groups' sums fit");
     const long row0 = (long)blockIdx.x * kGramRows;
-    for (int e = threadIdx.x; e < kGramRows * R; e += 256) {
+    const int tid = threadIdx.x, nq = (R + 3) / 4, per = nq * nq, ng = 256 / per, RR = R * R;
+    for (int e = tid; e < kGramRows * 4 * nq; e += 256) {
         const int r = e % kGramRows, b = e / kGramRows;
         const long i = row0 + r;
-        Us[r * kMaxR + b] = (i < I) ? (double)U[i + (long)b * I] : 0.0;
+        Us[r * kMaxR + b] = (i < I && b < R) ? (double)U[i + (long)b * I] : 0.0;
     }
     __syncthreads();
-    const int RR = R * R;
-    double *gp = gram_part + (long)blockIdx.x * RR;
-    for (int e = threadIdx.x; e < RR; e += 256) {
-        const int a = e % R, b = e / R;
-        double s[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-        for (int r = 0; r < kGramRows; r += 4) {
+    const int g = tid / per, t = tid - g * per, a0 = 4 * (t % nq), c0 = 4 * (t / nq);
+    double s[4][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) s[q] += Us[(r + q) * kMaxR + a] * Us[(r + q) * kMaxR + b];
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[p][q] = 0.0;
+    if (g < ng)
+#pragma unroll 4
+        for (int r = g; r < kGramRows; r += ng) {
+            double ua[4], ub[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                ua[q] = Us[r * kMaxR + a0 + q];
+                ub[q] = Us[r * kMaxR + c0 + q];
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[p][q] = fma(ua[p], ub[q], s[p][q]);
         }
-        gp[e] = (s[0] + s[1]) + (s[2] + s[3]);
+    // the groups' sums through LDS, added in order
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) Us[(4 * q + p) * 256 + tid] = s[p][q];
+    __syncthreads();
+    double *gp = gram_part + (long)blockIdx.x * RR;
+    for (int e = tid; e < RR; e += 256) {
+        const int a = e % R, b = e / R, at = (4 * (b & 3) + (a & 3)) * 256 + (b >> 2) * nq + (a >> 2);
+        double v = Us[at];
+        for (int k = 1; k < ng; ++k) v += Us[at + k * per];
+        gp[e] = v;
     }
 }
 
@@ -873,13 +899,15 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     return ensure_partial(P, S);
 }
 
-// (re)packs panels and Grams from the current factors
-static int refresh_factors(CpPlan &P, const Storage &S, hipStream_t s) {
+// (re)packs the panels from the current factors and, before the first sweep, forms their Grams (a
+// sweep leaves every mode's Gram of the factor it has stored: after it they stand, 78 us a phase at
+// 1024^3 rank 64)
+static int refresh_factors(CpPlan &P, const Storage &S, hipStream_t s, bool grams) {
     // partials of a previous storage phase are never reused across a storage change
     if (P.ls_mode) k_set_int<<<1, 1, 0, s>>>(&P.ls->skip, 0);
     int st = pack_panels(P.order, P.dims, -1, P.U, P.R, P.Rp, S.dtype == TDX_FP8_E4M3 ? S.scales : nullptr, P.panel, s);
     if (st) return st;
-    for (int m = 0; m < P.order; ++m) {
+    for (int m = 0; m < P.order && grams; ++m) {
         st = gram_of(P.U[m], P.dims[m], (int)P.R, P.gram_part, P.G[m], s);
         if (st) return st;
     }
@@ -1414,12 +1442,12 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     int done_open = 0, done_main = 0, done_ref = 0;
     SweepGraph graphs[3];
     auto graph_of = [&](int phase) { return opt.use_graph ? &graphs[phase] : nullptr; };
-    st = refresh_factors(P, opening ? Sopen : Smain, s);
+    st = refresh_factors(P, opening ? Sopen : Smain, s, true);
     (void)hipEventRecord(evg.e[1], s);
     if (!st && opening > 0) {
         st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, graph_of(0), sweep_ms, 0.0, 0.0, &done_open,
                         evg.e[0], elapsed);
-        if (!st) st = refresh_factors(P, Smain, s);
+        if (!st) st = refresh_factors(P, Smain, s, false);
     }
     if (!st)
         st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, graph_of(1),
@@ -1429,7 +1457,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     done_main += done_open;
     if (!st && opt.storage != TDX_F32 && opt.refine_sweeps > 0) {
         // FP32 refinement: the mode-0 panel must be unscaled again (rebuilt by the first solve)
-        st = refresh_factors(P, S32, s);
+        st = refresh_factors(P, S32, s, false);
         if (!st)
             st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, graph_of(2),
                             sweep_ms ? sweep_ms + done_main : nullptr, 0.0, 0.0, &done_ref, evg.e[0],
