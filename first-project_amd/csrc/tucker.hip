@@ -283,8 +283,10 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
         Xs = W.xb;
         xtype = TDX_BF16;
     }
-    // HOSVD init (only the spans matter when HOOI iterations follow: every later product
-    // contracts U U^T, so the eigenvector rotation is left to the last iteration)
+    // HOSVD init.  Only the spans matter when HOOI iterations follow (every later product contracts
+    // U U^T), but from eigenvectors the last iteration's solves start with a nearly diagonal H and
+    // take fewer Jacobi sweeps, one after the other, where the HOSVD's run side by side (128^4, ranks
+    // 32, one iteration: 2.89 ms without this rotation, 2.70 with it)
     EigJob jobs[4];
     for (int m = 0; m < order; ++m) {
         double *G = W.G + (long)m * kGramMaxN * kGramMaxN;
@@ -293,7 +295,7 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
         jobs[m] = EigJob{G, (int)dims[m], (int)ranks[m], nullptr, U[m], nullptr, W.Q + 2L * m * kGramMaxN * kGramMaxN,
                          nullptr};
     }
-    st = top_eigvecs(jobs, order, 1, s, iters == 0);
+    st = top_eigvecs(jobs, order, 1, s);
     if (st) return st;
     // ||X||^2 serves the error history only: a pass over X that a call without one does not make
     if (relerr_hist) {
