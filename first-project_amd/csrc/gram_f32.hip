@@ -9,7 +9,8 @@
 // sums of a step enter the FP32 accumulators once, so the chains of roundings stay short.  Every
 // workgroup writes the FP32 partial of its range; the caller adds them in FP64.
 //   * G needs the block pairs bi <= bj of its 16 x 16 blocks only.  Wave w takes the block rows w
-//     and nb - 1 - w: nb + 1 pairs each, whose column operands it reads from LDS once.
+//     and nb - 1 - w: nb + 1 pairs each, whose column operands it reads from LDS once (34 operand blocks
+//     a step with 8 block rows; from 113 rows on the waves hold pairs that need 22).
 //   * LDS rows are 64 BF16 of a part (128 bytes); chunk c of 8 lies at c ^ (row / 2 ^ row / 16) mod
 //     8, so 16 rows of one chunk hit distinct banks, and so do the rows of a transposing store
 //     but for their parity.
@@ -20,9 +21,10 @@
 //     multiplied in FP32.
 //
 // A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
-// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock.  Modes 0 .. 3 on
-// FP32 matrix instructions before: 128^4 420 / 396 / 393 / 395 -> 275 / 272 / 299 / 307 us (1.07 GB:
-// 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 22 / 22 / 22 / 22, 256 x 128 x 128 15 / 13 -> 10 / 10;
+// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock; the LDS reads of
+// the operands take the most of a step.  Modes 0 .. 3 on FP32 matrix instructions before: 128^4 420 /
+// 396 / 393 / 395 -> 275 / 272 / 299 / 307 us, 252 / 244 / 249 / 250 with the pairs of 22 blocks (1.07
+// GB: 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 22 / 22 / 22 / 22, 256 x 128 x 128 15 / 13 -> 10 / 10;
 // errors against 64 bits 7e-9 -> 5e-9 (64^4), 2.2e-8 -> 1.1e-8 (124 x 100 x 76), 3.7e-8 -> 1.6e-8
 // (64 x 48 x 40).  Not faster: eight waves a tile (128 registers spill), the pair counts at compile
 // time.
@@ -40,8 +42,23 @@ static constexpr int kGfN = 128, kGfK = 64;
 constexpr int gf_wgs(int nb) { return nb > 4 ? 2 : 3; }
 int gram_f32_wgs(long In) { return gf_wgs((int)ceil_div(In, 16L)); }
 
+// FULL (all 8 row blocks): a wave's nine pairs form blocks of their own, 3 x 3 or a triangle and
+// what fits beside it, so that the waves read 22 operand blocks a step instead of 34
+struct GfWave {
+    int n, blk[6], a[9], b[9];  // row blocks, and the pairs as positions among them
+};
+constexpr GfWave kGfWaves[4] = {
+    {6, {0, 1, 2, 3, 4, 5}, {0, 0, 0, 1, 1, 1, 2, 2, 2}, {3, 4, 5, 3, 4, 5, 3, 4, 5}},
+    {5, {0, 1, 2, 6, 7, 7}, {0, 0, 1, 1, 2, 2, 3, 3, 4}, {3, 4, 3, 4, 3, 4, 3, 4, 4}},
+    {5, {3, 4, 5, 6, 7, 7}, {0, 0, 1, 1, 2, 2, 0, 1, 2}, {3, 4, 3, 4, 3, 4, 0, 1, 2}},
+    {6, {0, 1, 2, 3, 4, 5}, {0, 0, 0, 1, 1, 2, 3, 3, 4}, {0, 1, 2, 1, 2, 2, 4, 5, 5}},
+};
+template <int W> struct GfIs {
+    static constexpr int w = W;
+};
+
 // NB: row blocks, at least ceil(In / 16)
-template <bool PC, int NB>
+template <bool PC, int NB, bool FULL>
 __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__restrict__ X, long P, long In, long Q, long kper,
                                                      float *__restrict__ part) {
     constexpr int NR = 16 * NB;
@@ -123,6 +140,72 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
         const uint4 v = xs[(k * NR + 16 * b + lm) * 8 + ((4 * ks + lg) ^ ((lm >> 1) ^ (b & 7)))];
         return __builtin_bit_cast(gf_b8, v);
     };
+    // FULL: the wave's pairs
+    gf_f4 accf[9];
+    if constexpr (FULL)
+#pragma unroll
+        for (int p = 0; p < 9; ++p) accf[p] = gf_f4{0.f, 0.f, 0.f, 0.f};
+    auto full_step = [&](auto w) {
+        constexpr GfWave g = kGfWaves[decltype(w)::w];
+        gf_f4 s[9];
+        gf_b8 o[6][3];
+        // smallest terms first, as in mul below; the first half's leading parts are read again for it
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+            for (int j = 0; j < g.n; ++j)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) o[j][k] = operand(g.blk[j], ks, k);
+#pragma unroll
+            for (int p = 0; p < 9; ++p) {
+                const gf_b8(&a)[3] = o[g.a[p]], (&b)[3] = o[g.b[p]];
+                gf_f4 t = ks == 0 ? gf_f4{0.f, 0.f, 0.f, 0.f} : s[p];
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], t, 0, 0, 0);
+                s[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], t, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int ks = 1; ks >= 0; --ks) {
+            if (ks == 0)
+#pragma unroll
+                for (int j = 0; j < g.n; ++j) o[j][0] = operand(g.blk[j], 0, 0);
+#pragma unroll
+            for (int p = 0; p < 9; ++p)
+                s[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[g.a[p]][0], o[g.b[p]][0], s[p], 0, 0, 0);
+        }
+#pragma unroll
+        for (int p = 0; p < 9; ++p) {
+            accf[p] += s[p];
+            asm volatile("" : "+v"(accf[p]));  // (before the branch, as below)
+        }
+    };
+    // FP32 products of the tile at k0, from memory
+    auto full_odd = [&](auto w, long k0) {
+        constexpr GfWave g = kGfWaves[decltype(w)::w];
+        for (int q = 0; q < 16; ++q) {
+            const long kk = k0 + 4 * q + lg, k = min(kk, K - 1), kd = k / P;
+            const float *p = X + (k - kd * P) + kd * P * In;
+            float v[6];
+#pragma unroll
+            for (int j = 0; j < g.n; ++j) {
+                v[j] = p[min((long)(16 * g.blk[j] + lm), In - 1) * P];
+                v[j] = kk < K ? v[j] : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 9; ++j)
+                accf[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[g.a[j]], v[g.b[j]], accf[j], 0, 0, 0);
+        }
+        __builtin_amdgcn_s_sleep(1);  // (the last results are in place before any branch)
+    };
+    auto by_wave = [&](auto f) {
+        if (wave == 0) f(GfIs<0>());
+        else if (wave == 1) f(GfIs<1>());
+        else if (wave == 2) f(GfIs<2>());
+        else f(GfIs<3>());
+    };
     // acc1[t], acc2[t]: block rows b1, b2 with block column nb - 1 - t
     gf_f4 acc1[NB], acc2[NB / 2];
 #pragma unroll
@@ -150,6 +233,11 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
         if (f) odd[par] = 1;
         __syncthreads();
         if (b2 < b1) continue;
+        if constexpr (FULL) {
+            if (odd[par]) by_wave([&](auto w) { full_odd(w, k0); });
+            else by_wave(full_step);
+            continue;
+        }
         if (odd[par]) {
             // from memory, FP32 products
             for (int q = 0; q < 16; ++q) {
@@ -217,6 +305,17 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
     }
     // register v of lane (lm, lg): row 4 lg + v, column lm of the pair's block
     float *dst = part + (long)blockIdx.x * kGfN * kGfN;
+    if constexpr (FULL) {
+        by_wave([&](auto w) {
+            constexpr GfWave g = kGfWaves[decltype(w)::w];
+#pragma unroll
+            for (int p = 0; p < 9; ++p)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    dst[(16 * g.blk[g.a[p]] + 4 * lg + v) * kGfN + 16 * g.blk[g.b[p]] + lm] = accf[p][v];
+        });
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
@@ -232,13 +331,15 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
 void gram_f32_launch(const float *X, long P, long In, long Q, long kper, float *part, unsigned nblk, hipStream_t s) {
     const int nb = (int)ceil_div(In, 16L);
     if (P > 1) {
-        if (nb <= 2) k_gram_f32<true, 2><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
-        else if (nb <= 4) k_gram_f32<true, 4><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
-        else k_gram_f32<true, 8><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        if (nb <= 2) k_gram_f32<true, 2, false><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else if (nb <= 4) k_gram_f32<true, 4, false><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else if (nb < 8) k_gram_f32<true, 8, false><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else k_gram_f32<true, 8, true><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
     } else {
         // (at least 64 rows: a 4 x 4 block for every thread)
-        if (nb <= 4) k_gram_f32<false, 4><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
-        else k_gram_f32<false, 8><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        if (nb <= 4) k_gram_f32<false, 4, false><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else if (nb < 8) k_gram_f32<false, 8, false><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
+        else k_gram_f32<false, 8, true><<<nblk, 256, 0, s>>>(X, P, In, Q, kper, part);
     }
 }
 

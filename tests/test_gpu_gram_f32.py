@@ -71,3 +71,14 @@ def test_nonfinite_and_overflow(dims, mode, value):
         assert got[17, 17] == np.inf  # the square overflows FP32
         ref = (B @ B.T)[17, rest]
         assert np.all(np.abs(got[17, rest] - ref) <= (A.shape[1] + 2) * 2.0 ** -24 * ref)
+
+
+@pytest.mark.parametrize("dims,mode", [((116, 190), 0), ((8, 125, 33), 1), ((128, 65), 0), ((4, 113, 16), 1)])
+def test_all_eight_row_blocks(dims, mode):
+    """113 to 128 rows, whose waves hold pairs of their own: the edges, and both kinds of tile that are
+    multiplied in FP32."""
+    test_edges(dims, mode)
+    test_rows_of_different_magnitude(dims, mode)
+    if int(np.prod(dims)) // dims[mode] > 70:
+        for value in (np.inf, np.nan, 1e30):
+            test_nonfinite_and_overflow(dims, mode, value)
