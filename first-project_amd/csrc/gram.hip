@@ -1,20 +1,19 @@
-// gram.hip -- Gram of a mode-n unfolding of a BF16 tensor on MFMA, G = X(n) X(n)^T, In <= 128.
+// gram.hip -- Gram of a mode-n unfolding on MFMA, G = X(n) X(n)^T, In <= 128: BF16 tensors, and FP32
+// ones inside HOOI on BF16 storage, whose sums keep their order (other FP32 Grams: gram_f32.hip and
+// gram_any.hip; 128^4 takes 404-439 us here, 244-252 there).
 //
 // The unfolding is never formed (the reference builds it with tensor2matrix and, for order
 // 4, identity-matrix GEMMs, src/tucker4_hosvd.cu:23-37, then calls cublasSgemm).  X is read
 // as the (P, In, Q) view, column k of X(n) being the fibre (p, q).  One K step is KS
-// = 32 consecutive columns; every lane loads one 16-byte vector per 16-row block, and the same
+// consecutive columns; every lane loads one 16-byte vector per 16-row block, and the same
 // registers serve as the A operand (rows i) and the B operand (columns j) of the MFMA, since
 // B = A^T.  Only the 36 block pairs bi <= bj of the 8 x 8 block grid are multiplied.
 //
-//  case B (P > 1, P % 32 == 0): K is contiguous along p; a lane's 16 bytes are 8 consecutive p
-//    of one row, rows of block b are 16 b + 0..15.
-//  case A (P == 1): rows are contiguous and K (= q) is strided; a lane loads its 8 consecutive
-//    rows at 8 columns and transposes in registers, so row block t holds rows 8 m + t,
-//    m = lane % 16.
-// BF16 tensors only: FP32 ones, and BF16 ones without whole vectors, go through LDS (gram_f32.hip,
-// gram_any.hip; in FP32 this kernel's one wave per SIMD took 404-439 us for 128^4 where the first
-// takes 272-307, and 60 us for 32^3 128 where it takes 14).
+//  case B (P > 1, P % KS == 0): K is contiguous along p; a lane's 16 bytes are KS/4 (FP32:
+//    4, BF16: 8) consecutive p of one row, rows of block b are 16 b + 0..15.
+//  case A (P == 1): rows are contiguous and K (= q) is strided; a lane loads its 8 (BF16) or
+//    4 (FP32) consecutive rows at 8 (4) columns and transposes in registers, so row block t
+//    holds rows 8 m + t (BF16) or 64 h + 4 m + t (FP32, block 4 h + t), m = lane % 16.
 //
 // The 4 waves of a workgroup take contiguous quarters of its K range and are summed in LDS
 // in a fixed order; each workgroup writes one 128 x 128 FP32 partial, and the partials are
@@ -29,9 +28,21 @@ typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
 static constexpr int kGramTile = 128;
 static constexpr int kGramLd = kGramTile + 1;
 
+template <int ST> struct GramElem;
+template <> struct GramElem<0> { typedef float T; typedef float4 V; };
+template <> struct GramElem<1> { typedef uint16_t T; typedef uint4 V; };
+
+__device__ __forceinline__ float4 gmask(float4 v, bool ok) {
+    const uint32_t m = ok ? 0xffffffffu : 0u;
+    return float4{__uint_as_float(__float_as_uint(v.x) & m), __uint_as_float(__float_as_uint(v.y) & m),
+                  __uint_as_float(__float_as_uint(v.z) & m), __uint_as_float(__float_as_uint(v.w) & m)};
+}
 __device__ __forceinline__ uint4 gmask(uint4 v, bool ok) {
     const uint32_t m = ok ? 0xffffffffu : 0u;
     return uint4{v.x & m, v.y & m, v.z & m, v.w & m};
+}
+__device__ __forceinline__ float f4_get(const float4 &v, int i) {
+    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
 __device__ __forceinline__ uint32_t u4_at(const uint4 &v, int i) {
     return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
@@ -42,17 +53,18 @@ __device__ __forceinline__ uint32_t h16(const uint4 &v, int t) {
 }
 
 // row of the tile held by MFMA row m of row block b
-template <bool CA> __device__ __forceinline__ int gram_row(int b, int m) {
+template <int ST, bool CA> __device__ __forceinline__ int gram_row(int b, int m) {
     if constexpr (!CA) return 16 * b + m;
-    else return 8 * m + b;
+    else if constexpr (ST == 1) return 8 * m + b;
+    else return 64 * (b >> 2) + 4 * m + (b & 3);
 }
 
-template <bool CA>
+template <int ST, bool CA>
 __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__restrict__ Xv, long P, long In, long Q,
                                                      long steps, long kper, float *__restrict__ part) {
-    typedef uint16_t ET;
-    typedef uint4 VT;
-    constexpr int KS = 32;  // K columns per step
+    typedef typename GramElem<ST>::T ET;
+    typedef typename GramElem<ST>::V VT;
+    constexpr int KS = (ST == 1) ? 32 : 16;  // K columns per step
     constexpr int NPAIR = 36;
     __shared__ float red[kGramTile * kGramLd];
     const ET *__restrict__ X = reinterpret_cast<const ET *>(Xv);
@@ -88,7 +100,7 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
     } else {
 #pragma unroll
         for (int h = 0; h < 8; ++h) {
-            const long a0 = 8 * lm;
+            const long a0 = (ST == 1) ? 8 * lm : 64 * (h >> 2) + 4 * lm;
             rok[h] = a0 < In;
             roff[h] = rok[h] ? a0 : 0;
         }
@@ -100,13 +112,13 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
     auto issue = [&](Slot &sl) {
         sl.ok = 0;
         if constexpr (!CA) {
-            const ET *base = X + f_pc * KS + 8 * lg + f_q * P * In;
+            const ET *base = X + f_pc * KS + ((ST == 1) ? 8 : 4) * lg + f_q * P * In;
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
                 sl.v[b] = *reinterpret_cast<const VT *>(base + roff[b]);
                 sl.ok |= (uint32_t)rok[b] << b;
             }
-        } else {
+        } else if constexpr (ST == 1) {
             // 8 columns q0 + 8 lg + j, the lane's 8 rows each
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -115,6 +127,17 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
                 sl.v[j] = *reinterpret_cast<const VT *>(X + roff[0] + (in ? qq : 0) * In);
                 sl.ok |= (uint32_t)in << j;
             }
+        } else {
+            // loads [h][c]: rows 64 h + 4 lm .. +3 at column q0 + 4 lg + c
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const long qq = f_q * KS + 4 * lg + c;
+                    const bool in = rok[4 * h] && qq < Q;
+                    sl.v[4 * h + c] = *reinterpret_cast<const VT *>(X + roff[4 * h] + (in ? qq : 0) * In);
+                    sl.ok |= (uint32_t)in << (4 * h + c);
+                }
         }
         if (++issued < nst) {
             if constexpr (CA) {
@@ -126,30 +149,51 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
         }
     };
     auto compute = [&](const Slot &sl) {
-        gbf16x8 op[8];
-        if constexpr (!CA) {
+        if constexpr (ST == 1) {
+            gbf16x8 op[8];
+            if constexpr (!CA) {
 #pragma unroll
-            for (int b = 0; b < 8; ++b) op[b] = __builtin_bit_cast(gbf16x8, gmask(sl.v[b], (sl.ok >> b) & 1u));
+                for (int b = 0; b < 8; ++b) op[b] = __builtin_bit_cast(gbf16x8, gmask(sl.v[b], (sl.ok >> b) & 1u));
+            } else {
+                uint4 v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = gmask(sl.v[j], (sl.ok >> j) & 1u);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    uint4 o;
+                    o.x = h16(v[0], t) | (h16(v[1], t) << 16);
+                    o.y = h16(v[2], t) | (h16(v[3], t) << 16);
+                    o.z = h16(v[4], t) | (h16(v[5], t) << 16);
+                    o.w = h16(v[6], t) | (h16(v[7], t) << 16);
+                    op[t] = __builtin_bit_cast(gbf16x8, o);
+                }
+            }
+            int pi = 0;
+#pragma unroll
+            for (int bi = 0; bi < 8; ++bi)
+#pragma unroll
+                for (int bj = bi; bj < 8; ++bj, ++pi)
+                    acc[pi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[bi], op[bj], acc[pi], 0, 0, 0);
         } else {
-            uint4 v[8];
+            float4 v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = gmask(sl.v[j], (sl.ok >> j) & 1u);
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                uint4 o;
-                o.x = h16(v[0], t) | (h16(v[1], t) << 16);
-                o.y = h16(v[2], t) | (h16(v[3], t) << 16);
-                o.z = h16(v[4], t) | (h16(v[5], t) << 16);
-                o.w = h16(v[6], t) | (h16(v[7], t) << 16);
-                op[t] = __builtin_bit_cast(gbf16x8, o);
+            for (int c = 0; c < 4; ++c) {
+                float op[8];
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    if constexpr (!CA) op[b] = f4_get(v[b], c);               // block b, column 4 lg + c
+                    else op[b] = f4_get(v[4 * (b >> 2) + c], b & 3);           // block 4h+t, column 4 lg + c
+                }
+                int pi = 0;
+#pragma unroll
+                for (int bi = 0; bi < 8; ++bi)
+#pragma unroll
+                    for (int bj = bi; bj < 8; ++bj, ++pi)
+                        acc[pi] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[bi], op[bj], acc[pi], 0, 0, 0);
             }
         }
-        int pi = 0;
-#pragma unroll
-        for (int bi = 0; bi < 8; ++bi)
-#pragma unroll
-            for (int bj = bi; bj < 8; ++bj, ++pi)
-                acc[pi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[bi], op[bj], acc[pi], 0, 0, 0);
     };
 
     // PD register slots, PD - 1 steps in flight per wave (case A runs one workgroup per CU
@@ -179,7 +223,7 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
                 for (int bj = bi; bj < 8; ++bj, ++pi) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const int i = gram_row<CA>(bi, 4 * lg + v), j = gram_row<CA>(bj, lm);
+                        const int i = gram_row<ST, CA>(bi, 4 * lg + v), j = gram_row<ST, CA>(bj, lm);
                         const float x = acc[pi][v];
                         if (wv == 0) {
                             red[i * kGramLd + j] = x;
@@ -197,16 +241,18 @@ __global__ __launch_bounds__(256, CA ? 1 : 2) void k_gram_mfma(const void *__res
     for (int e = threadIdx.x; e < kGramTile * kGramTile; e += 256) dst[e] = red[(e >> 7) * kGramLd + (e & 127)];
 }
 
-// Partial Grams of the (P, In, Q) view of a BF16 tensor: returns the number of partials written
-// to part (each kGramTile^2 floats, row-major, rows/cols >= In zero), or 0 if the shape has no
-// whole vectors (the caller falls back), or -1 on a launch error.
-int gram_mfma_launch(const void *X, long P, long In, long Q, float *part, int max_parts, hipStream_t s) {
+// Partial Grams of the (P, In, Q) view: returns the number of partials written to part
+// (each kGramTile^2 floats, row-major, rows/cols >= In zero), or 0 if the shape is not
+// supported here (the caller falls back), or -1 on a launch error.
+int gram_mfma_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s) {
+    const int st = (xtype == TDX_BF16) ? 1 : 0;
+    if (xtype != TDX_BF16 && xtype != TDX_F32) return 0;
     if (In < 1 || In > kGramTile || ((uintptr_t)X & 15)) return 0;
-    const long KS = 32;
+    const long KS = st ? 32 : 16;
     const bool ca = (P == 1);
     long steps;
     if (ca) {
-        if (In % 8) return 0;
+        if (In % (st ? 8 : 4)) return 0;
         steps = ceil_div(Q, KS);
     } else {
         if (P % KS) return 0;
@@ -218,8 +264,13 @@ int gram_mfma_launch(const void *X, long P, long In, long Q, float *part, int ma
     const long kper = ceil_div(steps, nblk);
     nblk = ceil_div(steps, kper);
     const dim3 g((unsigned)nblk), b(256);
-    if (ca) k_gram_mfma<true><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
-    else k_gram_mfma<false><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
+    if (st) {
+        if (ca) k_gram_mfma<1, true><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
+        else k_gram_mfma<1, false><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
+    } else {
+        if (ca) k_gram_mfma<0, true><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
+        else k_gram_mfma<0, false><<<g, b, 0, s>>>(X, P, In, Q, steps, kper, part);
+    }
     if (hipGetLastError() != hipSuccess) return -1;
     return (int)nblk;
 }

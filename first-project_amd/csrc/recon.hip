@@ -370,8 +370,8 @@ __global__ void k_ratio(const double *__restrict__ part, int nparts, double *__r
 //   Y[p + a*P + q*P*Ra] = sum_{i < In} U[a*lda + i*ldi] * X[p + i*P + q*P*In]
 // (reference ttm, src/ttm.cu:21,29,37, with lda = 1, ldi = d; transposed factor with
 //  lda = In, ldi = 1; Tucker expansion core -> tensor with lda = 1, ldi = I).
-int ttm_mfma_launch(const void *X, long P, long In, long Q, const float *U, long lda, long ldi, long Ra, float *Y,
-                    hipStream_t s);
+int ttm_mfma_launch(const void *X, int xtype, long P, long In, long Q, const float *U, long lda, long ldi, long Ra,
+                    float *Y, hipStream_t s);
 // X is FP32 (xtype TDX_F32) or BF16 bit patterns (TDX_BF16)
 int ttm_any_launch(const void *X, int xtype, long P, long In, long Q, const float *U, long lda, long ldi, long Ra,
                    float *Y, hipStream_t s);
@@ -382,10 +382,55 @@ int ttm_generic_t(const void *X, int xtype, int order, const long *dims, int mod
     for (int m = 0; m < mode; ++m) P *= dims[m];
     for (int m = mode + 1; m < order; ++m) Q *= dims[m];
     // BF16: the register kernel for the shapes it covers (ttm.hip); the general one otherwise
-    const int mf = xtype != TDX_BF16 ? 0 : ttm_mfma_launch(X, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
+    const int mf = xtype != TDX_BF16 ? 0 : ttm_mfma_launch(X, xtype, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
     if (mf < 0) return record(TDX_ERR_HIP);
     if (mf > 0) return TDX_OK;
     return ttm_any_launch(X, xtype, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
+}
+
+__device__ __forceinline__ float ld_elem(const float *p, long i) { return p[i]; }
+__device__ __forceinline__ float ld_elem(const uint16_t *p, long i) { return __uint_as_float((uint32_t)p[i] << 16); }
+// the factor entry as it enters the product: unchanged for FP32 storage, rounded to BF16
+// (nearest-even) for BF16 storage, as on the MFMA path
+__device__ __forceinline__ float coef(float u, const float *) { return u; }
+__device__ __forceinline__ float coef(float u, const uint16_t *) {
+    return __uint_as_float(f32_to_bf16_bits(u) << 16);
+}
+
+// one output a thread (of the shapes that ttm.hip does not cover, in HOOI on BF16 storage)
+template <typename T>
+__global__ __launch_bounds__(256) void k_ttm_generic(const T *__restrict__ X, long P, long In, long Q,
+                                                     const float *__restrict__ U, long lda, long ldi, long Ra,
+                                                     float *__restrict__ Y) {
+    const long n = P * Ra * Q;
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
+        const long p = e % P;
+        const long a = (e / P) % Ra;
+        const long q = e / (P * Ra);
+        const T *x = X + p + q * P * In;
+        const float *u = U + a * lda;
+        float acc = 0.0f;
+        for (long i = 0; i < In; ++i) acc = fmaf(coef(u[i * ldi], x), ld_elem(x, i * P), acc);
+        Y[e] = acc;
+    }
+}
+
+// the product of HOOI on BF16 storage, whose summation order stays as it is (tucker.hip, unfold_gram)
+int ttm_bf16_hooi(const void *X, int xtype, int order, const long *dims, int mode, const float *U, long lda, long ldi,
+                  long Ra, float *Y, hipStream_t s) {
+    long P = 1, Q = 1;
+    for (int m = 0; m < mode; ++m) P *= dims[m];
+    for (int m = mode + 1; m < order; ++m) Q *= dims[m];
+    const int mf = ttm_mfma_launch(X, xtype, P, dims[mode], Q, U, lda, ldi, Ra, Y, s);
+    if (mf < 0) return record(TDX_ERR_HIP);
+    if (mf > 0) return TDX_OK;
+    const int g = (int)std::max(1L, std::min(ceil_div(P * Ra * Q, 256L), 65536L));
+    if (xtype == TDX_BF16)
+        k_ttm_generic<uint16_t><<<g, 256, 0, s>>>((const uint16_t *)X, P, dims[mode], Q, U, lda, ldi, Ra, Y);
+    else
+        k_ttm_generic<float><<<g, 256, 0, s>>>((const float *)X, P, dims[mode], Q, U, lda, ldi, Ra, Y);
+    TDX_LAUNCH_CHECK();
+    return TDX_OK;
 }
 
 int ttm_generic(const float *X, int order, const long *dims, int mode, const float *U, long lda, long ldi, long Ra,

@@ -19,18 +19,90 @@
 #include "eig.hpp"
 #include "eig_sub.hpp"
 #include "linalg.hpp"
+#include <algorithm>
 #include <vector>
 
 namespace tdx {
 
 int ttm_generic(const float *X, int order, const long *dims, int mode, const float *U, long lda, long ldi, long Ra,
                 float *Y, hipStream_t s);
-int gram_mfma_launch(const void *X, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
+int gram_mfma_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
 int gram_any_launch(const void *X, int xtype, long P, long In, long Q, float *part, int max_parts, hipStream_t s);
 int ttm_generic_t(const void *X, int xtype, int order, const long *dims, int mode, const float *U, long lda, long ldi,
                   long Ra, float *Y, hipStream_t s);
+int ttm_bf16_hooi(const void *X, int xtype, int order, const long *dims, int mode, const float *U, long lda, long ldi,
+                  long Ra, float *Y, hipStream_t s);
 
 static constexpr int kGramMaxN = 128;
+static constexpr int kGramChunk = 64;  // fibres a step of k_gram_partial
+
+// Partial Grams of the (P, In, Q) view, FP32 FMAs over a range of fibres k = p + P q in order: HOOI on
+// BF16 storage only (see bf16_hooi in unfold_gram; k_gram_any sums in another order).  A workgroup
+// takes a 32 x 32 block bi <= bj (blockIdx.y) of the tile, a thread 2 x 2 entries; 64 fibres of the two
+// row blocks are staged a step, the next 64 in flight.  The order of an entry's sum is that of a
+// workgroup owning the whole tile (8 x 8 entries a
+// thread, 500-730 us a mode of 125 x 101 x 77; HOOI of 60 x 97 x 65 3.16 ms with it, 1.43 this way).
+__device__ __forceinline__ float ldx(const float *p, long i) { return p[i]; }
+__device__ __forceinline__ float ldx(const uint16_t *p, long i) { return __uint_as_float((uint32_t)p[i] << 16); }
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_gram_partial(const T *__restrict__ X, long P, long In, long Q,
+                                                      long kper, float *__restrict__ part) {
+    __shared__ float xs[64][kGramChunk + 1];  // rows: 32 of block bi, 32 of block bj
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+    int bi = 0, bj = blockIdx.y;
+    for (const int nb = (int)((In + 31) / 32); bj >= nb - bi; ++bi) bj -= nb - bi;
+    bj += bi;
+    const long K = P * Q;
+    const long k0 = blockIdx.x * kper, k1 = min(k0 + kper, K);
+    float acc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+    // element u of a thread: row and fibre of the step, lanes along what is contiguous
+    constexpr int NL = 64 * kGramChunk / 256;
+    float v[NL];
+    auto at = [&](int u, int &r, int &kk) {
+        const int e = tid + 256 * u;
+        if (P == 1) r = e % 64, kk = e / 64;
+        else kk = e % kGramChunk, r = e / kGramChunk;
+    };
+    auto load = [&](long kb) {
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            int r, kk;
+            at(u, r, kk);
+            const long a = r < 32 ? 32 * bi + r : 32 * bj + r - 32, k = kb + kk;
+            const bool on = k < k1 && a < In;
+            const long kc = on ? k : k0, q = kc / P;
+            v[u] = ldx(X, (kc - q * P) + (on ? a : 0) * P + q * P * In);
+            if (!on) v[u] = 0.0f;
+        }
+    };
+    load(k0);
+    for (long kb = k0; kb < k1; kb += kGramChunk) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            int r, kk;
+            at(u, r, kk);
+            xs[r][kk] = v[u];
+        }
+        __syncthreads();
+        load(kb + kGramChunk);
+#pragma unroll 8
+        for (int kk = 0; kk < kGramChunk; ++kk) {
+            const float a0 = xs[2 * ty][kk], a1 = xs[2 * ty + 1][kk];
+            const float b0 = xs[32 + 2 * tx][kk], b1 = xs[32 + 2 * tx + 1][kk];
+            acc[0][0] = fmaf(a0, b0, acc[0][0]);
+            acc[0][1] = fmaf(a0, b1, acc[0][1]);
+            acc[1][0] = fmaf(a1, b0, acc[1][0]);
+            acc[1][1] = fmaf(a1, b1, acc[1][1]);
+        }
+    }
+    float *dst = part + (long)blockIdx.x * kGramMaxN * kGramMaxN + (32L * bi + 2 * ty) * kGramMaxN + 32 * bj + 2 * tx;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) dst[i * kGramMaxN + j] = acc[i][j];
+}
 
 // G = the sum of the nblk FP32 partial Grams (pitch kGramMaxN), in FP64: a workgroup takes 64
 // consecutive entries (a, b) of the upper triangle (b fastest: contiguous reads) and its four
@@ -142,8 +214,12 @@ struct TuckerWs {
     DeviceLease mem;  // all of it
 };
 
+// bf16_hooi: HOOI iterations on BF16 storage round the factors to BF16, so an entry next to the middle
+// of two BF16 values turns the last bits of a sum into differences of 1e-4 in the results.  Their Grams
+// and products keep the summation order (and so the bits) they have always had: the register kernels
+// of gram.hip and ttm.hip and the per-entry ones.
 static int unfold_gram(const void *X, int xtype, int order, const long *dims, int mode, TuckerWs &W, double *G,
-                       hipStream_t s) {
+                       hipStream_t s, bool bf16_hooi = false) {
     long P = 1, Q = 1;
     for (int m = 0; m < mode; ++m) P *= dims[m];
     for (int m = mode + 1; m < order; ++m) Q *= dims[m];
@@ -151,8 +227,20 @@ static int unfold_gram(const void *X, int xtype, int order, const long *dims, in
     if (In > kGramMaxN) return record(TDX_ERR_UNSUPPORTED);
     // the BF16 kernel for whole vectors (gram.hip), the LDS kernels otherwise
     int nb = 0;
-    if (xtype == TDX_BF16)
-        nb = gram_mfma_launch(X, P, In, Q, W.gram_part, W.gram_blocks < 512 ? W.gram_blocks : 512, s);
+    if (xtype == TDX_BF16 || bf16_hooi)
+        nb = gram_mfma_launch(X, xtype, P, In, Q, W.gram_part, W.gram_blocks < 512 ? W.gram_blocks : 512, s);
+    if (nb == 0 && bf16_hooi) {
+        const long K = P * Q, want = std::max(1L, std::min((long)W.gram_blocks, ceil_div(K, 2048L)));
+        const long kper = ceil_div(ceil_div(K, want), 32L) * 32;
+        nb = (int)ceil_div(K, kper);
+        const int n32 = (int)ceil_div(In, 32L);
+        const dim3 g((unsigned)nb, (unsigned)(n32 * (n32 + 1) / 2));
+        if (xtype == TDX_BF16)
+            k_gram_partial<uint16_t><<<g, 256, 0, s>>>((const uint16_t *)X, P, In, Q, kper, W.gram_part);
+        else
+            k_gram_partial<float><<<g, 256, 0, s>>>((const float *)X, P, In, Q, kper, W.gram_part);
+        TDX_LAUNCH_CHECK();
+    }
     if (nb == 0) nb = gram_any_launch(X, xtype, P, In, Q, W.gram_part, W.gram_blocks, s);
     if (nb < 0) return record(TDX_ERR_HIP);
     k_gram_sum<<<(int)ceil_div(In * In, 64L), 256, 0, s>>>(W.gram_part, nb, In, G);
@@ -234,12 +322,14 @@ static int ws_setup(TuckerWs &W, int order, const long *dims, const long *ranks,
 // Y = X x_{m in modes} U_m^T applied in the listed order, results alternating between the
 // buffers a and b (X itself when nmodes == 0); cur: the dims of X in, of the result out
 static int ttm_seq(const void *X, int xtype, int order, long *cur, const long *ranks, float *const *U,
-                   const int *modes, int nmodes, float *a, float *b, const float **out, hipStream_t s) {
+                   const int *modes, int nmodes, float *a, float *b, const float **out, hipStream_t s,
+                   bool bf16_hooi = false) {
     const void *src = X;
     for (int t = 0; t < nmodes; ++t) {
         const int m = modes[t];
         float *dst = (t & 1) ? b : a;
-        int st = ttm_generic_t(src, t == 0 ? xtype : TDX_F32, order, cur, m, U[m], cur[m], 1, ranks[m], dst, s);
+        auto *ttm = bf16_hooi ? ttm_bf16_hooi : ttm_generic_t;
+        int st = ttm(src, t == 0 ? xtype : TDX_F32, order, cur, m, U[m], cur[m], 1, ranks[m], dst, s);
         if (st) return st;
         cur[m] = ranks[m];
         src = dst;
@@ -286,16 +376,18 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
     // HOSVD init.  Only the spans matter when HOOI iterations follow (every later product contracts
     // U U^T), but from eigenvectors the last iteration's solves start with a nearly diagonal H and
     // take fewer Jacobi sweeps, one after the other, where the HOSVD's run side by side (128^4, ranks
-    // 32, one iteration: 2.89 ms without this rotation, 2.70 with it)
+    // 32, one iteration: 2.89 ms without this rotation, 2.70 with it).  Not with BF16 storage, whose
+    // products round U's entries and so depend on the basis.
+    const bool bf16_hooi = bf16 && iters > 0;  // (see unfold_gram)
     EigJob jobs[4];
     for (int m = 0; m < order; ++m) {
         double *G = W.G + (long)m * kGramMaxN * kGramMaxN;
-        st = unfold_gram(Xs, xtype, order, dims, m, W, G, s);
+        st = unfold_gram(Xs, xtype, order, dims, m, W, G, s, bf16_hooi);
         if (st) return st;
         jobs[m] = EigJob{G, (int)dims[m], (int)ranks[m], nullptr, U[m], nullptr, W.Q + 2L * m * kGramMaxN * kGramMaxN,
                          nullptr};
     }
-    st = top_eigvecs(jobs, order, 1, s);
+    st = top_eigvecs(jobs, order, 1, s, !bf16_hooi);
     if (st) return st;
     // ||X||^2 serves the error history only: a pass over X that a call without one does not make
     if (relerr_hist) {
@@ -322,7 +414,7 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
             long tdims[4];
             for (int m = 0; m < order; ++m) tdims[m] = dims[m];
             const float *T = nullptr;
-            st = ttm_seq(Xs, xtype, order, tdims, ranks, U, tm, nt, W.y0, W.y1, &T, s);
+            st = ttm_seq(Xs, xtype, order, tdims, ranks, U, tm, nt, W.y0, W.y1, &T, s, bf16_hooi);
             if (st) return st;
             float *fa = (T == W.y0) ? W.y1 : W.y0;
             for (int n = n0; n < n1; ++n) {
@@ -330,8 +422,8 @@ static int tucker_run(const float *X, int order, const long *dims, const long *r
                 for (int m = n1 - 1; m >= n0; --m)
                     if (m != n) sm[ns++] = m;
                 for (int m = 0; m < order; ++m) ydims[m] = tdims[m];
-                st = ttm_seq(T, TDX_F32, order, ydims, ranks, U, sm, ns, W.y2, fa, &Y, s);
-                if (!st) st = unfold_gram(Y, TDX_F32, order, ydims, n, W, W.G, s);
+                st = ttm_seq(T, TDX_F32, order, ydims, ranks, U, sm, ns, W.y2, fa, &Y, s, bf16_hooi);
+                if (!st) st = unfold_gram(Y, TDX_F32, order, ydims, n, W, W.G, s, bf16_hooi);
                 // warm start: the factor of the previous iteration spans nearly the same subspace;
                 // eigenvectors (ascending, sign convention) only in the last iteration
                 const EigJob job{W.G, (int)dims[n], (int)ranks[n], U[n], U[n], nullptr, W.Q, nullptr};
