@@ -751,7 +751,7 @@ struct Storage {
     const float *scales;  // FP8 slice scales
     MttkrpPlan mp[4];
     DtreePlan dt;         // order 3, BF16/FP8: modes 1 and 2 from one shared pass over X
-    TwPlan tw;            // order 3, FP32 and split BF16, and BF16 outside dt's shapes: the same with FP32 T
+    TwPlan tw;            // order 3, FP32 and split BF16: the same with FP32 T
 };
 
 // sets the shape of a plan whose buffers are (or will be) large enough for it
@@ -894,7 +894,7 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     }
     if (ok) *ok = true;
     int st = dtree_plan(S.dt, P.order, P.dims, dtype, P.R, P.shared_pass && !split);
-    if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && !S.dt.on, split);
+    if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && (split || dtype == TDX_F32));
     if (st) return st;
     return ensure_partial(P, S);
 }
@@ -983,7 +983,7 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
     // Order 3 with the shared pass, R > 16: mode 2's inverse runs inside the pass over T
     // (k_m2_vinv), after mode 1's Gram sum in line, so mode 2 has no inverse launch of its own.
     const bool fuse2 = S.dt.on && P.order == 3 && R > 16;
-    // The same with FP32 T (FP32 storage, split opening sweeps, BF16 outside the first one's shapes): the pass over X fills the registers of
+    // The same with FP32 T (FP32 storage, split opening sweeps): the pass over X fills the registers of
     // every CU, so mode 1's inverse runs in the launch ahead of it, mode 2's in the pass over T.
     auto beside_of = [&](int n) {
         if (S.tw.on && n > 0) return false;

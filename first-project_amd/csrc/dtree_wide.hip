@@ -1,7 +1,6 @@
 // dtree_wide.hip -- the shared pass of an order-3 CP-ALS sweep for the tensors whose products are not
-// rounded to one BF16 part: FP32 storage (three parts of X and of A) and BF16 storage with hi + lo
-// coefficients (the opening sweeps', and any BF16 sweep's whose shape dtree.hip does not cover; A is
-// not rounded to 8 bits then).  As in dtree.hip
+// rounded to one BF16 part: FP32 storage (three parts of X and of A) and the opening sweeps' BF16
+// storage with hi + lo coefficients.  As in dtree.hip
 //   T[i2][i1][r] = sum_{i0} X[i0, i1, i2] A[i0][r],  M1[i1][r] = sum_{i2} T C,  M2[i2][r] = sum_{i1} T B
 // with one pass over X (k_tw_m1) and one over T (k_tw_m2), but T stays FP32.
 //
@@ -435,7 +434,7 @@ static int tw_by_nb(const TwPlan &p, const TwArgs *a, hipStream_t s) {
     }
 }
 
-int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled, bool split) {
+int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled) {
     p = TwPlan();
     if (!enabled || order != 3 || R < 1 || R > 64 || ((uintptr_t)X & 15) != 0) return TDX_OK;
     if (dtype != TDX_F32 && dtype != TDX_BF16) return TDX_OK;
@@ -449,11 +448,9 @@ int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const voi
     // one, FP32: 1024 x 1024 x 256 rank 64 880 -> 631 us, 256 x 512 x 512 rank 64 382 -> 317, 128 x 512
     // x 1024 rank 64 (es I0 = 8 Rp) 397 -> 352, 64 x 1024 x 1024 rank 64 (4 Rp) 413 -> 415.  Below
     // 2^25 elements a pass is as short as the launches: 512 x 256 x 256 rank 16 130 -> 117, 256^3 rank
-    // 16 89 -> 91.  BF16 sweeps whose coefficients are not split hide the inverses beside their separate
-    // passes, so there the pass saved has to cost more than the two: 1000^3 rank 64 1409 -> 1152, 720^3
-    // rank 16 542 -> 428, but 904 x 520 x 264 rank 48 266 -> 270, 512 x 500 x 400 rank 40 193 -> 200.
+    // 16 89 -> 91.
     const long es = f32 ? 4 : 2, N = p.I0 * p.I1 * p.I2;
-    if (es * p.I0 < 8L * p.Rp || N < (f32 || split ? 1L << 25 : 1L << 28)) return TDX_OK;
+    if (es * p.I0 < 8L * p.Rp || N < (1L << 25)) return TDX_OK;
     const int ksn = f32 ? 2 : 4, np = f32 ? 3 : 2;
     p.nfc = (int)ceil_div(p.I0, 32L * ksn);
     p.chunk_ops = ksn * np * (p.Rp / 16) * 64;

@@ -105,8 +105,8 @@ int dtree_m2_vinv_launch(const DtreePlan &d, const uint16_t *T, const float *pan
                          const double *G0, const double *G1, int R, double *Vinv, int *status, double *fb_ws,
                          hipStream_t s);
 
-// the same pass with FP32 T, for FP32 storage and BF16 storage with hi + lo coefficients, split sweeps
-// or not (dtree_wide.hip)
+// the same pass with FP32 T, for FP32 storage and BF16 storage with hi + lo coefficients
+// (dtree_wide.hip)
 struct TwPlan {
     bool on = false;
     int st = 0, Rp = 0, nfc = 0, chunk_ops = 0;  // st 0: FP32, 1: BF16; chunks of I0, 16-byte operands each
@@ -124,7 +124,7 @@ struct TwPlan {
     }
 };
 // fills p (p.on = false where the separate passes are used)
-int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled, bool split);
+int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled);
 // partial[split][i1][Rp] (nsplit1 splits, rows_pad1() rows), T in ws and the inverse
 int tw_m1_launch(const TwPlan &p, const void *X, const float *panelA, const float *panelC, void *ws, float *partial,
                  const VinvJob &inverse, hipStream_t s);

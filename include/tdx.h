@@ -219,9 +219,8 @@ typedef struct {
                                 pass over X that also writes T = X x_0 A^T (I2 I1 Rp floats), then
                                 a pass over T (default 1; no counterpart in the reference, which
                                 runs one MTTKRP per mode); 0: one fused MTTKRP per mode.  The same,
-                                with FP32 T, for FP32 storage and split opening sweeps (from 2^25
-                                elements) and for BF16 shapes that the first one does not take
-                                (from 2^28; A is then not rounded to BF16) */
+                                with FP32 T, for FP32 storage and split opening sweeps of tensors
+                                where a pass over X costs more than T (2^25 elements and more) */
     int opening_sweeps;      /* BF16/FP8 storage: the first opening_sweeps of the max_sweeps main
                                 sweeps read the FP32 tensor (default 0).  The early sweeps decide
                                 which components ALS resolves; rounding the Khatri-Rao operand to
