@@ -894,7 +894,16 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     }
     if (ok) *ok = true;
     int st = dtree_plan(S.dt, P.order, P.dims, dtype, P.R, P.shared_pass && !split);
-    if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && (split || dtype == TDX_F32));
+    // Split opening sweeps whose successors round A to BF16 (dt) turn the last bits into differences of
+    // up to 5e-5 at 2^26 elements, 6e-6 at 2^30: from there on only
+    long least = 1L << 25;
+    if (!st && split) {
+        DtreePlan next;
+        st = dtree_plan(next, P.order, P.dims, dtype, P.R, P.shared_pass);
+        if (next.on) least = 1L << 30;
+    }
+    if (!st)
+        st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && (split || dtype == TDX_F32), least);
     if (st) return st;
     return ensure_partial(P, S);
 }
@@ -1441,16 +1450,22 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     float *elapsed = opt.trace ? opt.trace->elapsed_ms : nullptr;
     int done_open = 0, done_main = 0, done_ref = 0;
     SweepGraph graphs[3];
-    auto graph_of = [&](int phase) { return opt.use_graph ? &graphs[phase] : nullptr; };
+    // A phase of a few sweeps is launched plainly: recording and instantiating its graph takes the host
+    // longer than enqueuing it.  (Also, a process that made many short calls of three such phases, 120 x
+    // 98 x 87 rank 33, has ended in an abort on the host, cause not found: no such phase is captured.)
+    constexpr int kGraphSweeps = 8;
+    auto graph_of = [&](int phase, int sweeps) {
+        return opt.use_graph && sweeps >= kGraphSweeps ? &graphs[phase] : nullptr;
+    };
     st = refresh_factors(P, opening ? Sopen : Smain, s, true);
     (void)hipEventRecord(evg.e[1], s);
     if (!st && opening > 0) {
-        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, graph_of(0), sweep_ms, 0.0, 0.0, &done_open,
+        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, graph_of(0, opening), sweep_ms, 0.0, 0.0, &done_open,
                         evg.e[0], elapsed);
         if (!st) st = refresh_factors(P, Smain, s, false);
     }
     if (!st)
-        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, graph_of(1),
+        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, graph_of(1, opt.max_sweeps - opening),
                         sweep_ms ? sweep_ms + done_open : nullptr, opt.tol,
                         opt.storage == TDX_F32 ? opt.target_relerr : 0.0, &done_main, evg.e[0],
                         elapsed ? elapsed + done_open : nullptr);
@@ -1459,7 +1474,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
         // FP32 refinement: the mode-0 panel must be unscaled again (rebuilt by the first solve)
         st = refresh_factors(P, S32, s, false);
         if (!st)
-            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, graph_of(2),
+            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, graph_of(2, opt.refine_sweeps),
                             sweep_ms ? sweep_ms + done_main : nullptr, 0.0, 0.0, &done_ref, evg.e[0],
                             elapsed ? elapsed + done_main : nullptr);
     }

@@ -208,7 +208,7 @@ typedef struct {
                                 (mlp_params), 2 alpha = (sweep+1)^(1/3) (cpd_lsb.m:30),
                                 3 no step, record the relative error at every grid alpha.
                                 FP32 storage only: with BF16 / FP8 storage TDX_ERR_UNSUPPORTED */
-    int use_graph;           /* capture each sweep in a hipGraph (default 1) */
+    int use_graph;           /* capture each sweep in a hipGraph (default 1; phases of 8 sweeps or more) */
     const float *mlp_params; /* device MLP parameters, nin = TDX_LS_FEATURES, nout = 1 */
     int mlp_width;
     int ngrid;               /* line_search == 3: number of grid points (<= 8) */
@@ -220,7 +220,8 @@ typedef struct {
                                 a pass over T (default 1; no counterpart in the reference, which
                                 runs one MTTKRP per mode); 0: one fused MTTKRP per mode.  The same,
                                 with FP32 T, for FP32 storage and split opening sweeps of tensors
-                                where a pass over X costs more than T (2^25 elements and more) */
+                                where a pass over X costs more than T (2^25 elements and more;
+                                opening sweeps before BF16 sweeps with a shared pass: 2^30) */
     int opening_sweeps;      /* BF16/FP8 storage: the first opening_sweeps of the max_sweeps main
                                 sweeps read the FP32 tensor (default 0).  The early sweeps decide
                                 which components ALS resolves; rounding the Khatri-Rao operand to
