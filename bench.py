@@ -189,32 +189,29 @@ def extras(args, log):
     os.makedirs(os.path.dirname(cache), exist_ok=True)
     best, times = tdx.cp_batched_autotune(X, U, b, trial_sweeps=2, cache_path=cache)
     st, fit, ms = tdx.cp_als_batched(X, U, b, 30, init=0, seed=1, variant=best)
-    # per-tensor loop baseline on a sample: the single-tensor driver per tensor, eager launches
-    # and with a graph per call.  A first untimed call on the largest tensor leaves a plan
-    # whose buffers hold every tensor of the batch, so the timed calls allocate nothing.
+    # per-tensor loop baseline on a sample: the single-tensor driver per tensor.  A first untimed
+    # call on the largest tensor leaves a plan whose buffers hold every tensor of the batch, so the
+    # timed calls allocate nothing.
     loop_n = 64
     idx = np.linspace(0, b.n - 1, loop_n).astype(int)
-    loop = {}
-    for use_graph in (0, 1):
-        dmax, rmax = int(b.shapes.max()), int(b.ranks.max())  # 96^3, rank 16: holds every tensor
+    dmax, rmax = int(b.shapes.max()), int(b.ranks.max())  # 96^3, rank 16: holds every tensor
+    oo = tdx.default_cp_options()
+    oo.max_sweeps, oo.record_fit = 30, 1
+    tdx.cp_als_ex(X[:dmax ** 3], (dmax,) * 3, rmax, [torch.empty(dmax * rmax, device="cuda") for _ in range(3)], oo)
+    tot = 0.0
+    for t in idx:
+        dims = tuple(int(v) for v in b.shapes[t])
+        R = int(b.ranks[t])
+        Ut = [torch.empty(d * R, device="cuda") for d in dims]
+        xt = X[int(b.xoff[t]):int(b.xoff[t]) + int(np.prod(dims))]
         oo = tdx.default_cp_options()
-        oo.max_sweeps, oo.record_fit, oo.use_graph = 30, 1, use_graph
-        tdx.cp_als_ex(X[:dmax ** 3], (dmax,) * 3, rmax, [torch.empty(dmax * rmax, device="cuda") for _ in range(3)],
-                      oo)
-        tot = 0.0
-        for t in idx:
-            dims = tuple(int(v) for v in b.shapes[t])
-            R = int(b.ranks[t])
-            Ut = [torch.empty(d * R, device="cuda") for d in dims]
-            xt = X[int(b.xoff[t]):int(b.xoff[t]) + int(np.prod(dims))]
-            oo = tdx.default_cp_options()
-            oo.max_sweeps, oo.record_fit, oo.use_graph = 30, 1, use_graph
-            torch.cuda.synchronize()
-            t0 = time.perf_counter()
-            tdx.cp_als_ex(xt, dims, R, Ut, oo)
-            torch.cuda.synchronize()
-            tot += time.perf_counter() - t0
-        loop["graph" if use_graph else "eager"] = round(tot * b.n / loop_n, 3)
+        oo.max_sweeps, oo.record_fit = 30, 1
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        tdx.cp_als_ex(xt, dims, R, Ut, oo)
+        torch.cuda.synchronize()
+        tot += time.perf_counter() - t0
+    loop = {"eager": round(tot * b.n / loop_n, 3)}
     # bytes per sweep: three MTTKRPs stream X three times; the variants whose mode 2 reads
     # T = X x_0 A^T (J K R floats per tensor) stream X twice and write and read T once
     bytes_sweep = 3 * 4 * b.x_floats
@@ -385,7 +382,7 @@ def main():
         o = tdx.default_cp_options()
         o.max_sweeps, o.refine_sweeps, o.storage, o.opening_sweeps = sweeps, refine, storage, opening
         o.opening_split = split
-        o.init, o.record_fit, o.use_graph = 1, 1, 1
+        o.init, o.record_fit = 1, 1
         st, rep, fit, ms = tdx.cp_als_ex(X, dims, R, U, o, want_ms=True, want_elapsed=True)
         return rep, np.asarray(fit), np.asarray(ms, np.float64), U
 

@@ -16,7 +16,7 @@
 // fit and Gram partials) and k_gram_psum (Gram of the new factor; at R <= 16 summed by the
 // next mode's k_vinv instead); after the last mode k_gram_psum_fit (its Gram and the
 // sweep's fit in one kernel).
-// A sweep is captured once into a hipGraph and replayed.
+// Every sweep is launched plainly, without a captured graph (run_sweeps).
 #include "mttkrp.hpp"
 #include "linalg.hpp"
 #include "vinv.hpp"
@@ -1018,10 +1018,7 @@ static int enqueue_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit) {
     // forked[n]: the fork point of mode n's inverse was recorded after the previous mode's
     // solve (its branch also sums that mode's Gram).  A side branch is enqueued after the main
     // kernel it runs beside, with the fork event recorded before that kernel: the dependencies
-    // are the same, and a captured graph then has the main kernel as the first successor of
-    // the fork point, which keeps the chain MTTKRP -> solve -> MTTKRP on one hardware queue
-    // (with the side branch first, each of those edges crossed queues: ~9-15 us each instead
-    // of ~5 at 1024^3, R 64).
+    // are the same, and the main kernel is not held up by the side stream's launches.
     bool forked[4] = {false, false, false, false};
     for (int n = 0; n < P.order; ++n) {
         const bool dt = S.dt.on && n > 0;
@@ -1160,47 +1157,17 @@ static int enqueue_ls(CpPlan &P, const Storage &S, hipStream_t s) {
     return TDX_OK;
 }
 
-// The captured sweep of a phase.  Its launches run on after the host has enqueued them, so it is
-// destroyed only when its stream has finished: a call keeps the graphs of all its phases to its end.
-struct SweepGraph {
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    hipStream_t s = nullptr;
-    ~SweepGraph() {
-        if (ge) (void)hipStreamSynchronize(s);
-        if (ge) (void)hipGraphExecDestroy(ge);
-        if (g) (void)hipGraphDestroy(g);
-    }
-};
-
-static int capture_sweep(CpPlan &P, const Storage &S, hipStream_t s, bool fit, SweepGraph &G) {
-    TDX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int st = enqueue_sweep(P, S, s, fit);
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(s, &g);
-    if (st) {
-        if (g) (void)hipGraphDestroy(g);
-        return st;
-    }
-    if (e != hipSuccess) return record_hip(e, "hipStreamEndCapture", __FILE__, __LINE__);
-    G.g = g;
-    G.s = s;
-    TDX_HIP(hipGraphInstantiate(&G.ge, g, nullptr, nullptr, 0));
-    return TDX_OK;
-}
-
 // Runs `sweeps` sweeps on storage S; records per-sweep ms if sweep_ms != NULL, and the device
-// time from the event `origin` to the end of every sweep if elapsed_ms != NULL.  G: the phase's graph
-// (none is captured for a null one); the sweeps may still run on return.
-static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bool fit, SweepGraph *G, float *sweep_ms,
+// time from the event `origin` to the end of every sweep if elapsed_ms != NULL; the sweeps may still
+// run on return.  Nothing is captured: processes that made many mixed calls, whose phases were each
+// captured, instantiated and destroyed, have ended on the host (a segmentation fault, an abort) for a
+// reason that is not known; the library's own host code is clean on that case under an address
+// sanitizer, on a HIP runtime that checks every handle.
+static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bool fit, float *sweep_ms,
                       double tol, double target, int *done, hipEvent_t origin = nullptr,
                       float *elapsed_ms = nullptr) {
     *done = 0;
     if (sweeps <= 0) return TDX_OK;
-    if (G) {
-        int st = capture_sweep(P, S, s, fit, *G);
-        if (st) return st;
-    }
     if (!origin) elapsed_ms = nullptr;
     std::vector<hipEvent_t> evs;
     if (sweep_ms || elapsed_ms) {
@@ -1214,13 +1181,8 @@ static int run_sweeps(CpPlan &P, const Storage &S, hipStream_t s, int sweeps, bo
     double prev = -1.0;
     int st = TDX_OK;
     for (int it = 0; it < sweeps; ++it) {
-        if (G) {
-            hipError_t e = hipGraphLaunch(G->ge, s);
-            if (e != hipSuccess) { st = record_hip(e, "hipGraphLaunch", __FILE__, __LINE__); break; }
-        } else {
-            st = enqueue_sweep(P, S, s, fit);
-            if (st) break;
-        }
+        st = enqueue_sweep(P, S, s, fit);
+        if (st) break;
         if (!evs.empty()) {
             hipError_t e = hipEventRecord(evs[it + 1], s);
             if (e != hipSuccess) { st = record_hip(e, "hipEventRecord", __FILE__, __LINE__); break; }
@@ -1334,9 +1296,9 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
         if (dims[m] <= 0 || !factors[m]) return record(TDX_ERR_ARG);
         N *= dims[m];
     }
-    // Graph capture is not allowed on the legacy default stream: when the library stream
-    // is the default one, run on a private blocking stream (it orders after earlier
-    // default-stream work by the legacy-stream rules) and join it before returning.
+    // When the library stream is the legacy default one, run on a private blocking stream (it
+    // orders after earlier default-stream work by the legacy-stream rules) and join it before
+    // returning, so that calls of several threads do not queue behind each other.
     hipStream_t s = stream();
     StreamLease owned;
     if (!s) {
@@ -1449,23 +1411,15 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     }
     float *elapsed = opt.trace ? opt.trace->elapsed_ms : nullptr;
     int done_open = 0, done_main = 0, done_ref = 0;
-    SweepGraph graphs[3];
-    // A phase of a few sweeps is launched plainly: recording and instantiating its graph takes the host
-    // longer than enqueuing it.  (Also, a process that made many short calls of three such phases, 120 x
-    // 98 x 87 rank 33, has ended in an abort on the host, cause not found: no such phase is captured.)
-    constexpr int kGraphSweeps = 8;
-    auto graph_of = [&](int phase, int sweeps) {
-        return opt.use_graph && sweeps >= kGraphSweeps ? &graphs[phase] : nullptr;
-    };
     st = refresh_factors(P, opening ? Sopen : Smain, s, true);
     (void)hipEventRecord(evg.e[1], s);
     if (!st && opening > 0) {
-        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, graph_of(0, opening), sweep_ms, 0.0, 0.0, &done_open,
+        st = run_sweeps(P, Sopen, s, opening, opt.record_fit != 0, sweep_ms, 0.0, 0.0, &done_open,
                         evg.e[0], elapsed);
         if (!st) st = refresh_factors(P, Smain, s, false);
     }
     if (!st)
-        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0, graph_of(1, opt.max_sweeps - opening),
+        st = run_sweeps(P, Smain, s, opt.max_sweeps - opening, opt.record_fit != 0,
                         sweep_ms ? sweep_ms + done_open : nullptr, opt.tol,
                         opt.storage == TDX_F32 ? opt.target_relerr : 0.0, &done_main, evg.e[0],
                         elapsed ? elapsed + done_open : nullptr);
@@ -1474,7 +1428,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
         // FP32 refinement: the mode-0 panel must be unscaled again (rebuilt by the first solve)
         st = refresh_factors(P, S32, s, false);
         if (!st)
-            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0, graph_of(2, opt.refine_sweeps),
+            st = run_sweeps(P, S32, s, opt.refine_sweeps, opt.record_fit != 0,
                             sweep_ms ? sweep_ms + done_main : nullptr, 0.0, 0.0, &done_ref, evg.e[0],
                             elapsed ? elapsed + done_main : nullptr);
     }

@@ -67,7 +67,7 @@ def init_factors(seed, dims, R):
 
 def run(X, dims, R, U, mode, sweeps, params=None, target=0.0, grid=None):
     o = tdx.default_cp_options()
-    o.max_sweeps, o.init, o.record_fit, o.use_graph = sweeps, 1, 1, 1
+    o.max_sweeps, o.init, o.record_fit = sweeps, 1, 1
     o.line_search = mode
     o.target_relerr = target
     if mode == tdx.LS_LEARNED:

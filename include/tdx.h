@@ -208,7 +208,9 @@ typedef struct {
                                 (mlp_params), 2 alpha = (sweep+1)^(1/3) (cpd_lsb.m:30),
                                 3 no step, record the relative error at every grid alpha.
                                 FP32 storage only: with BF16 / FP8 storage TDX_ERR_UNSUPPORTED */
-    int use_graph;           /* capture each sweep in a hipGraph (default 1; phases of 8 sweeps or more) */
+    int use_graph;           /* accepted, without effect: sweeps are launched one by one (processes that
+                                made many calls with captured sweeps have ended on the host, for a
+                                reason that is not known) */
     const float *mlp_params; /* device MLP parameters, nin = TDX_LS_FEATURES, nout = 1 */
     int mlp_width;
     int ngrid;               /* line_search == 3: number of grid points (<= 8) */
@@ -288,7 +290,7 @@ int tdx_cp_tensorcore(const float *X, float *A, float *B, float *C, long a, long
  * m of tensor t at uoff[3t+m], I_m x R column-major).  By default the batch is cut into work items
  * of equal size (runs of slices of a tensor); the older variants (a persistent kernel per sweep, or
  * one MTTKRP and one solve kernel per mode over a queue of whole tensors) are kept for the
- * autotuner.  A sweep is captured in a hipGraph.  init = 0 draws
+ * autotuner, and capture a sweep in a hipGraph.  init = 0 draws
  * U(0,1) from Philox stream (seed + t, m), 1 uses the caller's U.  variant: kernel variant
  * (see tdx_cp_batched_autotune), < 0 for the default.  fit_hist (host, ntensors x sweeps,
  * may be NULL) receives the fast-fit relative errors; sweep_ms (host, may be NULL) the device
