@@ -874,10 +874,11 @@ static int ensure_partial(CpPlan &P, Storage &S) {
     return TDX_OK;
 }
 
-// split: BF16 storage streamed with the hi + lo Khatri-Rao block (no shared pass); *ok = false
-// (and nothing set up) when some mode's plan is not the LDS kernel that implements it
-static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const float *scales, bool split = false,
-                         bool *ok = nullptr) {
+// split: BF16 storage streamed with the hi + lo Khatri-Rao block (no shared pass with BF16 T); *ok =
+// false (and nothing set up) when some mode's plan is not the LDS kernel that implements it.  wide: the
+// shared pass with FP32 T may be used
+static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const float *scales, bool wide,
+                         bool split = false, bool *ok = nullptr) {
     S.X = X;
     S.dtype = dtype;
     S.scales = scales;
@@ -894,16 +895,7 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     }
     if (ok) *ok = true;
     int st = dtree_plan(S.dt, P.order, P.dims, dtype, P.R, P.shared_pass && !split);
-    // Split opening sweeps whose successors round A to BF16 (dt) turn the last bits into differences of
-    // up to 5e-5 at 2^26 elements, 6e-6 at 2^30: from there on only
-    long least = 1L << 25;
-    if (!st && split) {
-        DtreePlan next;
-        st = dtree_plan(next, P.order, P.dims, dtype, P.R, P.shared_pass);
-        if (next.on) least = 1L << 30;
-    }
-    if (!st)
-        st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && (split || dtype == TDX_F32), least);
+    if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && wide);
     if (st) return st;
     return ensure_partial(P, S);
 }
@@ -1390,22 +1382,28 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     st = norm2(X, TDX_F32, nullptr, dims[0], N, P.scratch, P.normx2, s, (uint16_t *)Xb, amax, &amax_done);
     if (st) return st;
     Storage S32;
-    st = storage_setup(P, S32, X, TDX_F32, nullptr);
+    st = storage_setup(P, S32, X, TDX_F32, nullptr, true);
     if (st) return st;
     Storage Smain = S32;
     if (opt.storage == TDX_BF16) {
-        st = storage_setup(P, Smain, Xq, TDX_BF16, nullptr);
+        st = storage_setup(P, Smain, Xq, TDX_BF16, nullptr, false);
     } else if (opt.storage == TDX_FP8_E4M3) {
         if (!amax_done) st = slice_amax(X, amax, dims[0], N / dims[0], s);
         if (!st) st = fp8_from_amax(X, amax, (uint8_t *)Xq, scales, dims[0], N / dims[0], s);
-        if (!st) st = storage_setup(P, Smain, Xq, TDX_FP8_E4M3, scales);
+        if (!st) st = storage_setup(P, Smain, Xq, TDX_FP8_E4M3, scales, false);
     }
     if (st) return record(st);
     Storage Sopen = S32;
     if (split_open) {
         Storage Ss;
         bool ok = false;
-        st = storage_setup(P, Ss, Xb, TDX_BF16, nullptr, true, &ok);
+        // Sweeps with BF16 T that follow round the whole of A to BF16: an entry of A next to the middle of
+        // two BF16 values turns the last bits of an opening sweep into a change of 2^-9 of it in every
+        // slab.  Their opening sweeps therefore keep the separate passes' order of summation at any size
+        // (with FP32 T the results were up to 5e-5 away from those at 2^26 elements; where the sweeps
+        // that follow round one Khatri-Rao entry at a time, 9e-6).
+        const bool rounds_a = Smain.dt.on && opening < opt.max_sweeps;
+        st = storage_setup(P, Ss, Xb, TDX_BF16, nullptr, !rounds_a, true, &ok);
         if (st) return record(st);
         if (ok) Sopen = Ss;
     }

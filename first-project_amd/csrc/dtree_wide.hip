@@ -434,7 +434,7 @@ static int tw_by_nb(const TwPlan &p, const TwArgs *a, hipStream_t s) {
     }
 }
 
-int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled, long least) {
+int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled) {
     p = TwPlan();
     if (!enabled || order != 3 || R < 1 || R > 64 || ((uintptr_t)X & 15) != 0) return TDX_OK;
     if (dtype != TDX_F32 && dtype != TDX_BF16) return TDX_OK;
@@ -450,7 +450,7 @@ int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const voi
     // 2^25 elements a pass is as short as the launches: 512 x 256 x 256 rank 16 130 -> 117, 256^3 rank
     // 16 89 -> 91.
     const long es = f32 ? 4 : 2, N = p.I0 * p.I1 * p.I2;
-    if (es * p.I0 < 8L * p.Rp || N < least) return TDX_OK;
+    if (es * p.I0 < 8L * p.Rp || N < (1L << 25)) return TDX_OK;
     const int ksn = f32 ? 2 : 4, np = f32 ? 3 : 2;
     p.nfc = (int)ceil_div(p.I0, 32L * ksn);
     p.chunk_ops = ksn * np * (p.Rp / 16) * 64;

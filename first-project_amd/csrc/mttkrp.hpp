@@ -123,8 +123,8 @@ struct TwPlan {
         return a > b ? a : b;
     }
 };
-// fills p (p.on = false where the separate passes are used: below `least` elements, among others)
-int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled, long least);
+// fills p (p.on = false where the separate passes are used)
+int tw_plan(TwPlan &p, int order, const long *dims, int dtype, long R, const void *X, bool enabled);
 // partial[split][i1][Rp] (nsplit1 splits, rows_pad1() rows), T in ws and the inverse
 int tw_m1_launch(const TwPlan &p, const void *X, const float *panelA, const float *panelC, void *ws, float *partial,
                  const VinvJob &inverse, hipStream_t s);

@@ -222,8 +222,9 @@ typedef struct {
                                 a pass over T (default 1; no counterpart in the reference, which
                                 runs one MTTKRP per mode); 0: one fused MTTKRP per mode.  The same,
                                 with FP32 T, for FP32 storage and split opening sweeps of tensors
-                                where a pass over X costs more than T (2^25 elements and more;
-                                opening sweeps before BF16 sweeps with a shared pass: 2^30) */
+                                where a pass over X costs more than T (2^25 elements and more);
+                                not for opening sweeps before BF16 / FP8 sweeps that take the
+                                shared pass, whose results they would move by rounding */
     int opening_sweeps;      /* BF16/FP8 storage: the first opening_sweeps of the max_sweeps main
                                 sweeps read the FP32 tensor (default 0).  The early sweeps decide
                                 which components ALS resolves; rounding the Khatri-Rao operand to

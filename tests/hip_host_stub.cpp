@@ -18,6 +18,7 @@ struct State {
     std::map<char *, size_t> mem;
     std::set<void *> streams, events, graphs, execs;
     std::map<std::string, long> calls;
+    std::map<const void *, std::string> kernels;
     size_t used = 0, limit = ~size_t(0), most = 0;
     std::string faults;
 };
@@ -65,12 +66,21 @@ size_t stub_most() {  // the largest use since the last call of this
     return v;
 }
 long stub_calls(const char *name) { return st().calls[name]; }
+long stub_launches(const char *kernel) {  // launches of the kernels whose mangled name holds `kernel`
+    long n = 0;
+    for (auto &c : st().calls)
+        if (c.first.compare(0, 2, "_Z") == 0 && c.first.find(kernel) != std::string::npos) n += c.second;
+    return n;
+}
 const char *stub_faults() { return st().faults.c_str(); }
 
 // ---- registration and launches
 void **__hipRegisterFatBinary(const void *) { return new void *; }
 void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, dim3 *, dim3 *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *,
+                           int *) {
+    st().kernels[f] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {
     t_grid = g, t_block = b, t_lds = lds, t_stream = s;
@@ -80,9 +90,10 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
     *g = t_grid, *b = t_block, *lds = t_lds, *s = t_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3 g, dim3 b, void **, size_t lds, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t lds, hipStream_t s) {
     Call c("hipLaunchKernel");
     c.stream(s);
+    ++st().calls[st().kernels[f]];
     c.need(g.x && g.y && g.z && b.x && b.x * b.y * b.z <= 1024 && lds <= 160 * 1024, "launch shape");
     return hipSuccess;
 }

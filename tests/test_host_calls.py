@@ -27,6 +27,7 @@ def lib(tmp_path_factory):
     lib.stub_limit.argtypes = [ctypes.c_size_t]
     lib.stub_used.restype = lib.stub_most.restype = ctypes.c_size_t
     lib.stub_calls.argtypes, lib.stub_calls.restype = [ctypes.c_char_p], L_
+    lib.stub_launches.argtypes, lib.stub_launches.restype = [ctypes.c_char_p], L_
     lib.stub_faults.restype = ctypes.c_char_p
     lib.hipMalloc.argtypes, lib.hipFree.argtypes = [ctypes.POINTER(P_), ctypes.c_size_t], [P_]
     return lib
@@ -79,3 +80,19 @@ def test_sweeps_are_launched_plainly(lib, memory, dims, R):
                           use_graph=1)
         assert (st, done) == (tdx.TDX_OK, 29)
     assert lib.stub_calls(b"hipStreamBeginCapture") == lib.stub_calls(b"hipGraphInstantiate") == 0
+
+
+@pytest.mark.parametrize("dims,R,storage,sweeps,wide", [
+    # BF16 or FP8 sweeps with the shared pass follow: the separate passes, whatever the size
+    ((1024, 1024, 1024), 64, tdx.TDX_BF16, 3, False), ((512, 512, 256), 64, tdx.TDX_BF16, 3, False),
+    ((4096, 128, 64), 16, tdx.TDX_FP8_E4M3, 3, False),  # (FP8 sweeps of that extent take it, BF16 ones do not)
+    # none follows, or such as do not round A
+    ((512, 512, 256), 64, tdx.TDX_BF16, 2, True), ((4096, 128, 64), 16, tdx.TDX_BF16, 3, True),
+    ((520, 400, 330), 64, tdx.TDX_BF16, 3, True)])
+def test_opening_sweeps_shared_pass(lib, memory, dims, R, storage, sweeps, wide):
+    X, U = buffers(memory, dims, R)
+    before = lib.stub_launches(b"k_tw_m1"), lib.stub_launches(b"k_ttm_m1")
+    st, done = cp_als(lib, X, dims, R, U, storage, sweeps, opening_sweeps=2, opening_split=1)
+    assert (st, done) == (tdx.TDX_OK, sweeps)
+    assert lib.stub_launches(b"k_tw_m1") - before[0] == (2 if wide else 0)
+    assert wide or lib.stub_launches(b"k_ttm_m1") - before[1] == 1
