@@ -781,28 +781,28 @@ static int plan_setup(CpPlan &P, int order, const long *dims, long R, float *con
     P.cap_R = R;
     for (int m = 0; m < order; ++m) {
         P.cap_panel[m] = std::max(panel_floats(dims[m], P.Rp), dims[m] * R);
-        TDX_HIP(hipMalloc(&P.panel[m], sizeof(float) * P.cap_panel[m]));
-        TDX_HIP(hipMalloc(&P.G[m], sizeof(double) * R * R));
-        TDX_HIP(hipMalloc(&P.Vinv[m], sizeof(double) * R * R));
+        TDX_TRY(device_malloc(&P.panel[m], sizeof(float) * P.cap_panel[m]));
+        TDX_TRY(device_malloc(&P.G[m], sizeof(double) * R * R));
+        TDX_TRY(device_malloc(&P.Vinv[m], sizeof(double) * R * R));
         long nb = ceil_div(dims[m], kSolveRows);
         if (nb > nblk_max) nblk_max = nb;
     }
     P.cap_nblk = nblk_max;
-    TDX_HIP(hipMalloc(&P.ip_part, sizeof(double) * nblk_max));
-    TDX_HIP(hipMalloc(&P.gram_part, sizeof(double) * nblk_max * R * R));
+    TDX_TRY(device_malloc(&P.ip_part, sizeof(double) * nblk_max));
+    TDX_TRY(device_malloc(&P.gram_part, sizeof(double) * nblk_max * R * R));
     P.max_sweeps_hist = max_hist < 1 ? 1 : max_hist;
-    TDX_HIP(hipMalloc(&P.fit_hist, sizeof(double) * P.max_sweeps_hist));
-    TDX_HIP(hipMalloc(&P.counter, sizeof(int)));
-    TDX_HIP(hipMalloc(&P.status, sizeof(int)));
-    TDX_HIP(hipMalloc(&P.normx2, sizeof(double)));
-    TDX_HIP(hipMalloc(&P.scratch, sizeof(double) * 4096));
-    TDX_HIP(hipMalloc(&P.vinv_ws, sizeof(double) * 2 * R * R));
-    TDX_HIP(hipMalloc(&P.hpart, sizeof(double) * ceil_div(R * R, 256L)));
-    TDX_HIP(hipMalloc(&P.fit_done, sizeof(int)));
+    TDX_TRY(device_malloc(&P.fit_hist, sizeof(double) * P.max_sweeps_hist));
+    TDX_TRY(device_malloc(&P.counter, sizeof(int)));
+    TDX_TRY(device_malloc(&P.status, sizeof(int)));
+    TDX_TRY(device_malloc(&P.normx2, sizeof(double)));
+    TDX_TRY(device_malloc(&P.scratch, sizeof(double) * 4096));
+    TDX_TRY(device_malloc(&P.vinv_ws, sizeof(double) * 2 * R * R));
+    TDX_TRY(device_malloc(&P.hpart, sizeof(double) * ceil_div(R * R, 256L)));
+    TDX_TRY(device_malloc(&P.fit_done, sizeof(int)));
     TDX_HIP(hipMemset(P.fit_done, 0, sizeof(int)));
     if (P.ls_mode) {
         auto alloc = [&](void **p, size_t bytes) -> int {
-            TDX_HIP(hipMalloc(p, bytes));
+            TDX_TRY(device_malloc(p, bytes));
             P.owned.push_back(*p);
             return TDX_OK;
         };
@@ -859,7 +859,7 @@ static int ensure_partial(CpPlan &P, Storage &S) {
     if (need > P.partial_floats) {
         if (P.partial) TDX_HIP(hipFree(P.partial));
         P.partial = nullptr;
-        TDX_HIP(hipMalloc(&P.partial, sizeof(float) * need));
+        TDX_TRY(device_malloc(&P.partial, sizeof(float) * need));
         P.partial_floats = need;
     }
     size_t mneed = 0;
@@ -868,7 +868,7 @@ static int ensure_partial(CpPlan &P, Storage &S) {
     if (mneed > P.msum_doubles) {
         if (P.msum) TDX_HIP(hipFree(P.msum));
         P.msum = nullptr;
-        TDX_HIP(hipMalloc(&P.msum, sizeof(double) * mneed));
+        TDX_TRY(device_malloc(&P.msum, sizeof(double) * mneed));
         P.msum_doubles = mneed;
     }
     return TDX_OK;

@@ -992,7 +992,7 @@ int tdx_cp_batched_autotune(const float *X, const float *U, const long *dims, co
         }
     }
     float *Uw = nullptr;
-    TDX_HIP(hipMalloc(&Uw, sizeof(float) * u_floats));
+    TDX_TRY(device_malloc(&Uw, sizeof(float) * u_floats));
     float best_ms = 1e30f;
     int bv = 1, rc = TDX_OK;
     std::vector<float> ms(trial_sweeps);

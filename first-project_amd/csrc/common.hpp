@@ -20,6 +20,12 @@ int device_cus();
         if (e_ != hipSuccess) return tdx::record_hip(e_, #call, __FILE__, __LINE__); \
     } while (0)
 
+#define TDX_TRY(call)                  \
+    do {                               \
+        const int st_ = (call);        \
+        if (st_ != TDX_OK) return st_; \
+    } while (0)
+
 #define TDX_CHECK_ARG(cond)                          \
     do {                                             \
         if (!(cond)) return tdx::record(TDX_ERR_ARG); \
@@ -53,7 +59,7 @@ void release_workspace();
 // from several threads and on several streams do not meet.  done() says that all work on it has
 // finished: the destructor then keeps it for a later call, up to 4 idle blocks of 2 GiB together and 4
 // idle streams; without it (a call that failed) or past those bounds it is freed.
-// tdx_release_workspace frees what is idle, and so does an allocation that finds no memory.
+// tdx_release_workspace frees what is idle, and so does a device_malloc that finds no memory.
 class DeviceLease {
   public:
     DeviceLease() = default;
@@ -87,6 +93,13 @@ class StreamLease {
     bool done_ = false;
 };
 void release_leases();
+// hipMalloc for everything the library allocates: where memory has run out, again after the idle
+// leases and the cached CP-ALS plans, which no call is using, have been freed
+int device_malloc(void **p, size_t bytes);
+template <typename T>
+int device_malloc(T **p, size_t bytes) {
+    return device_malloc((void **)p, bytes);
+}
 // consecutive parts of one block, 256-byte aligned
 struct Parts {
     size_t bytes = 0;

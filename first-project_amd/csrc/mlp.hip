@@ -118,10 +118,10 @@ struct MlpWs {
     int alloc(long batch, const MlpShape &s) {
         long bw = batch * s.width, bo = batch * s.nout;
         float **ps[] = {&z1, &h1, &z2, &h2, &d2, &d1};
-        for (float **p : ps) TDX_HIP(hipMalloc(p, sizeof(float) * bw));
-        TDX_HIP(hipMalloc(&y, sizeof(float) * bo));
-        TDX_HIP(hipMalloc(&dy, sizeof(float) * bo));
-        TDX_HIP(hipMalloc(&sq, sizeof(float) * bo));
+        for (float **p : ps) TDX_TRY(device_malloc(p, sizeof(float) * bw));
+        TDX_TRY(device_malloc(&y, sizeof(float) * bo));
+        TDX_TRY(device_malloc(&dy, sizeof(float) * bo));
+        TDX_TRY(device_malloc(&sq, sizeof(float) * bo));
         return TDX_OK;
     }
 };
@@ -238,13 +238,13 @@ int tdx_mlp_train(float *params, const float *X, const float *T, long nsamples, 
         }
     } fr{{(void **)&G, (void **)&m, (void **)&v, (void **)&xb, (void **)&tb, (void **)&loss, (void **)&idx}};
     const long n = s.count();
-    TDX_HIP(hipMalloc(&G, sizeof(float) * n));
-    TDX_HIP(hipMalloc(&m, sizeof(float) * n));
-    TDX_HIP(hipMalloc(&v, sizeof(float) * n));
-    TDX_HIP(hipMalloc(&xb, sizeof(float) * batch * nin));
-    TDX_HIP(hipMalloc(&tb, sizeof(float) * batch * nout));
-    TDX_HIP(hipMalloc(&loss, sizeof(float)));
-    TDX_HIP(hipMalloc(&idx, sizeof(int) * nsamples));
+    TDX_TRY(device_malloc(&G, sizeof(float) * n));
+    TDX_TRY(device_malloc(&m, sizeof(float) * n));
+    TDX_TRY(device_malloc(&v, sizeof(float) * n));
+    TDX_TRY(device_malloc(&xb, sizeof(float) * batch * nin));
+    TDX_TRY(device_malloc(&tb, sizeof(float) * batch * nout));
+    TDX_TRY(device_malloc(&loss, sizeof(float)));
+    TDX_TRY(device_malloc(&idx, sizeof(int) * nsamples));
     k_zero<<<grid1(n), 256, 0, st>>>(m, n);
     k_zero<<<grid1(n), 256, 0, st>>>(v, n);
     std::vector<int> perm(nsamples);

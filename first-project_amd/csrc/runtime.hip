@@ -42,7 +42,7 @@ int workspace(int slot, size_t bytes, void **ptr) {
             s.bytes = 0;
         }
         size_t want = bytes < 256 ? 256 : bytes;
-        TDX_HIP(hipMalloc(&s.ptr, want));
+        TDX_TRY(device_malloc(&s.ptr, want));
         s.bytes = want;
     }
     *ptr = s.ptr;
@@ -95,6 +95,23 @@ static void free_idle(int dev) {
 
 void release_leases() { free_idle(-1); }
 
+int device_malloc(void **p, size_t bytes) {
+    *p = nullptr;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int dev = 0;
+        TDX_HIP(hipGetDevice(&dev));
+        free_idle(dev);
+        release_cp_plans();
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) return TDX_OK;
+    (void)hipGetLastError();  // (handled: not for the next call's launch check)
+    *p = nullptr;
+    return record_hip(e, "hipMalloc", __FILE__, __LINE__);
+}
+
 int DeviceLease::take(size_t bytes) {
     TDX_HIP(hipGetDevice(&dev_));
     {
@@ -110,16 +127,7 @@ int DeviceLease::take(size_t bytes) {
             return TDX_OK;
         }
     }
-    hipError_t e = hipMalloc(&p_, bytes < 256 ? 256 : bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        free_idle(dev_);
-        e = hipMalloc(&p_, bytes < 256 ? 256 : bytes);
-    }
-    if (e != hipSuccess) {
-        p_ = nullptr;
-        return record_hip(e, "hipMalloc", __FILE__, __LINE__);
-    }
+    TDX_TRY(device_malloc(&p_, bytes < 256 ? 256 : bytes));
     bytes_ = bytes < 256 ? 256 : bytes;
     return TDX_OK;
 }

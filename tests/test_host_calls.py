@@ -96,3 +96,34 @@ def test_opening_sweeps_shared_pass(lib, memory, dims, R, storage, sweeps, wide)
     assert (st, done) == (tdx.TDX_OK, sweeps)
     assert lib.stub_launches(b"k_tw_m1") - before[0] == (2 if wide else 0)
     assert wide or lib.stub_launches(b"k_ttm_m1") - before[1] == 1
+
+
+def test_idle_memory_is_freed_for_every_allocation(lib, memory):
+    """A Tucker call leaves its memory idle, CP-ALS calls their plans; a CP-ALS call of another shape, a
+    workspace and a training run then find theirs."""
+    dims = (128, 128, 128, 128)
+    X = memory(128 ** 4)
+    U = [memory(128 * 64) for _ in range(4)]
+    core = memory(32 ** 4)
+
+    def fill():
+        lib.stub_limit(2 ** 63)
+        assert lib.tdx_tucker_hooi(X, 4, tdx.dims_arr(dims), tdx.dims_arr((32,) * 4), 1, 0, core, (P_ * 4)(*U), None) == 0
+        for d in ((128,) * 4, (256, 256, 256), (64, 64, 64)):
+            assert cp_als(lib, X, d, 16, U)[0] == tdx.TDX_OK
+        kept = lib.stub_used()
+        lib.stub_limit(kept)
+        return kept
+
+    calls = {
+        "plan": lambda: cp_als(lib, X, (2048, 64, 64), 64, [memory_u] * 3)[0],
+        "workspace": lambda: lib.tdx_mttkrp_ex(X, tdx.TDX_F32, None, 3, tdx.dims_arr((512, 512, 512)), (P_ * 4)(
+            memory_u, memory_u, memory_u), 64, 0, memory_u),
+        "training": lambda: lib.tdx_mlp_train(memory_u, memory_u, memory_u, 4096, 8, 64, 1, 1, 4096, 1e-3, 0,
+                                              (ctypes.c_float * 4)()),
+    }
+    memory_u = memory(1 << 20)
+    for name, call in calls.items():
+        lib.tdx_release_workspace()
+        fill()
+        assert call() == tdx.TDX_OK, name
