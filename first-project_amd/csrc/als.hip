@@ -676,8 +676,7 @@ struct CpPlan {
     double *hpart = nullptr;    // k_gram_psum_fit: per-block partials (R^2 / 256 doubles)
     int *fit_done = nullptr;    // k_gram_psum_fit: ticket (0 between launches)
     bool shared_pass = true;    // modes 1 and 2 from one pass over X where eligible
-    void *T = nullptr;          // shared-pass intermediate X x_0 A^T (dt: BF16; tw: FP32 and A's parts)
-    size_t t_bytes = 0;
+    void *T = nullptr;          // shared-pass intermediate X x_0 A^T (dt: BF16; tw: FP32 and A's parts), leased
     int max_sweeps_hist = 0;
     hipStream_t side = nullptr;
     hipEvent_t ev_fork[4], ev_join[4];
@@ -725,14 +724,13 @@ struct CpPlan {
             if (Vinv[m]) (void)hipFree(Vinv[m]);
             panel[m] = nullptr; G[m] = nullptr; Vinv[m] = nullptr;
         }
-        void *ps[] = {partial, msum, ip_part, gram_part, fit_hist, counter, status, normx2, scratch, vinv_ws, T,
+        void *ps[] = {partial, msum, ip_part, gram_part, fit_hist, counter, status, normx2, scratch, vinv_ws,
                       hpart, fit_done};
         for (void *p : ps)
             if (p) (void)hipFree(p);
         partial = nullptr; msum = nullptr; ip_part = nullptr; gram_part = nullptr; fit_hist = nullptr;
-        counter = nullptr; status = nullptr; normx2 = nullptr; scratch = nullptr; vinv_ws = nullptr; T = nullptr;
+        counter = nullptr; status = nullptr; normx2 = nullptr; scratch = nullptr; vinv_ws = nullptr;
         hpart = nullptr; fit_done = nullptr;
-        t_bytes = 0;
         if (events) {
             for (int m = 0; m < 4; ++m) {
                 (void)hipEventDestroy(ev_fork[m]);
@@ -831,51 +829,49 @@ static int plan_setup(CpPlan &P, int order, const long *dims, long R, float *con
     return TDX_OK;
 }
 
-static int ensure_partial(CpPlan &P, Storage &S) {
-    size_t need = 0;
-    for (int m = 0; m < P.order; ++m)
-        if (S.mp[m].partial_floats() > need) need = S.mp[m].partial_floats();
-    const size_t tneed = S.dt.on ? S.dt.t_bytes() : S.tw.on ? S.tw.ws_bytes() : 0;
-    if (tneed > P.t_bytes) {
-        if (P.T && !S.tw.on) {
-            TDX_HIP(hipFree(P.T));
-            P.T = nullptr;
-            P.t_bytes = 0;
-        }
-        void *t = nullptr;
-        const hipError_t e = hipMalloc(&t, tneed);
-        if (e == hipErrorOutOfMemory && S.tw.on) {
-            (void)hipGetLastError();
-            S.tw.on = false;  // the separate passes need no T
-        } else {
-            TDX_HIP(e);
-            if (P.T) TDX_HIP(hipFree(P.T));
-            P.T = t;
-            P.t_bytes = tneed;
-        }
-    }
-    if (S.dt.on && S.dt.partial_floats() > need) need = S.dt.partial_floats();
-    if (S.tw.on && S.tw.partial_floats() > need) need = S.tw.partial_floats();
-    if (need > P.partial_floats) {
-        if (P.partial) TDX_HIP(hipFree(P.partial));
-        P.partial = nullptr;
-        TDX_TRY(device_malloc(&P.partial, sizeof(float) * need));
-        P.partial_floats = need;
-    }
-    size_t mneed = 0;
-    for (int m = 0; m < P.order; ++m)
-        if ((size_t)S.mp[m].rows_pad * P.Rp > mneed) mneed = (size_t)S.mp[m].rows_pad * P.Rp;
-    if (mneed > P.msum_doubles) {
-        if (P.msum) TDX_HIP(hipFree(P.msum));
-        P.msum = nullptr;
-        TDX_TRY(device_malloc(&P.msum, sizeof(double) * mneed));
-        P.msum_doubles = mneed;
-    }
+template <typename T>
+static int grow(T *&p, size_t &have, size_t need) {
+    if (need <= have) return TDX_OK;
+    if (p) TDX_HIP(hipFree(p));
+    p = nullptr;
+    have = 0;
+    TDX_TRY(device_malloc(&p, sizeof(T) * need));
+    have = need;
     return TDX_OK;
 }
 
+// the memory of the phases that run: partials, their sums and T
+static int phase_memory(CpPlan &P, Storage *const *S, int n, DeviceLease &T) {
+    bool wide = false;
+    for (int k = 0; k < n; ++k) wide |= S[k]->tw.on;
+    for (;;) {
+        size_t partial = 0, msum = 0, t = 0;
+        for (int k = 0; k < n; ++k) {
+            const Storage &q = *S[k];
+            for (int m = 0; m < P.order; ++m) {
+                partial = std::max(partial, q.mp[m].partial_floats());
+                msum = std::max(msum, (size_t)q.mp[m].rows_pad * P.Rp);
+            }
+            if (q.dt.on) partial = std::max(partial, q.dt.partial_floats());
+            if (q.tw.on) partial = std::max(partial, q.tw.partial_floats());
+            t = std::max(t, q.dt.on ? q.dt.t_bytes() : q.tw.on ? q.tw.ws_bytes() : 0);
+        }
+        int st = grow(P.partial, P.partial_floats, partial);
+        if (!st) st = grow(P.msum, P.msum_doubles, msum);
+        if (!st && t > 0) st = T.take(t);
+        P.T = T.ptr();
+        if (st != TDX_ERR_ALLOC || !wide) return st;
+        // the separate passes need no FP32 T, and had to fit before there was one
+        for (int k = 0; k < n; ++k) S[k]->tw.on = false;
+        wide = false;
+        TDX_HIP(hipFree(P.partial));
+        P.partial = nullptr;
+        P.partial_floats = 0;
+    }
+}
+
 // split: BF16 storage streamed with the hi + lo Khatri-Rao block (no shared pass with BF16 T); *ok =
-// false (and nothing set up) when some mode's plan is not the LDS kernel that implements it.  wide: the
+// false (and nothing planned) when some mode's plan is not the LDS kernel that implements it.  wide: the
 // shared pass with FP32 T may be used
 static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const float *scales, bool wide,
                          bool split = false, bool *ok = nullptr) {
@@ -896,8 +892,7 @@ static int storage_setup(CpPlan &P, Storage &S, const void *X, int dtype, const 
     if (ok) *ok = true;
     int st = dtree_plan(S.dt, P.order, P.dims, dtype, P.R, P.shared_pass && !split);
     if (!st) st = tw_plan(S.tw, P.order, P.dims, dtype, P.R, X, P.shared_pass && wide);
-    if (st) return st;
-    return ensure_partial(P, S);
+    return st;
 }
 
 // (re)packs the panels from the current factors and, before the first sweep, forms their Grams (a
@@ -1293,6 +1288,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     // returning, so that calls of several threads do not queue behind each other.
     hipStream_t s = stream();
     StreamLease owned;
+    DeviceLease tmem;  // (given back before the stream: its work has finished)
     if (!s) {
         const int st = owned.take();
         if (st) return st;
@@ -1357,6 +1353,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     // BF16 / FP8 storage: the first `opening` of the max_sweeps main sweeps read the FP32 tensor,
     // or (opening_split) a BF16 copy with the split Khatri-Rao block
     const int opening = (opt.storage == TDX_F32) ? 0 : std::min(opt.opening_sweeps, opt.max_sweeps);
+    const bool refine = opt.storage != TDX_F32 && opt.refine_sweeps > 0, main_runs = opt.max_sweeps > opening;
     const bool split_open = opening > 0 && opt.opening_split && opt.storage != TDX_F32;
     void *Xq = nullptr, *Xb = nullptr;  // main-phase copy; BF16 copy (= Xq for BF16 storage)
     float *scales = nullptr;
@@ -1394,19 +1391,26 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     }
     if (st) return record(st);
     Storage Sopen = S32;
+    bool ok = false;  // the split opening sweeps have their kernel
     if (split_open) {
         Storage Ss;
-        bool ok = false;
         // Sweeps with BF16 T that follow round the whole of A to BF16: an entry of A next to the middle of
         // two BF16 values turns the last bits of an opening sweep into a change of 2^-9 of it in every
         // slab.  Their opening sweeps therefore keep the separate passes' order of summation at any size
         // (with FP32 T the results were up to 5e-5 away from those at 2^26 elements; where the sweeps
         // that follow round one Khatri-Rao entry at a time, 9e-6).
-        const bool rounds_a = Smain.dt.on && opening < opt.max_sweeps;
+        const bool rounds_a = Smain.dt.on && main_runs;
         st = storage_setup(P, Ss, Xb, TDX_BF16, nullptr, !rounds_a, true, &ok);
         if (st) return record(st);
         if (ok) Sopen = Ss;
     }
+    Storage *phases[3];
+    int nphase = 0;
+    if (opening > 0) phases[nphase++] = &Sopen;
+    if (main_runs) phases[nphase++] = &Smain;
+    if (refine) phases[nphase++] = &S32;
+    st = phase_memory(P, phases, nphase, tmem);
+    if (st) return record(st);
     float *elapsed = opt.trace ? opt.trace->elapsed_ms : nullptr;
     int done_open = 0, done_main = 0, done_ref = 0;
     st = refresh_factors(P, opening ? Sopen : Smain, s, true);
@@ -1422,7 +1426,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
                         opt.storage == TDX_F32 ? opt.target_relerr : 0.0, &done_main, evg.e[0],
                         elapsed ? elapsed + done_open : nullptr);
     done_main += done_open;
-    if (!st && opt.storage != TDX_F32 && opt.refine_sweeps > 0) {
+    if (!st && refine) {
         // FP32 refinement: the mode-0 panel must be unscaled again (rebuilt by the first solve)
         st = refresh_factors(P, S32, s, false);
         if (!st)
@@ -1464,6 +1468,7 @@ int tdx_cp_als_ex(const float *X, int order, const long *dims, long rank, float 
     if (opt.record_fit && count > 0 && !isfinite(last)) result = TDX_ERR_NONFINITE;
     give_plan(key, std::move(Pp));
     owned.done();
+    tmem.done();
     if (report) {
         report->sweeps_done = done_main + done_ref;
         report->status = result;

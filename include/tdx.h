@@ -224,7 +224,9 @@ typedef struct {
                                 with FP32 T, for FP32 storage and split opening sweeps of tensors
                                 where a pass over X costs more than T (2^25 elements and more);
                                 not for opening sweeps before BF16 / FP8 sweeps that take the
-                                shared pass, whose results they would move by rounding */
+                                shared pass, whose results they would move by rounding.  Where the
+                                device has no memory for FP32 T, the fused MTTKRPs run (the results
+                                then differ by rounding) */
     int opening_sweeps;      /* BF16/FP8 storage: the first opening_sweeps of the max_sweeps main
                                 sweeps read the FP32 tensor (default 0).  The early sweeps decide
                                 which components ALS resolves; rounding the Khatri-Rao operand to

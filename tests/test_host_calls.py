@@ -98,6 +98,58 @@ def test_opening_sweeps_shared_pass(lib, memory, dims, R, storage, sweeps, wide)
     assert wide or lib.stub_launches(b"k_ttm_m1") - before[1] == 1
 
 
+def least_limit(lib, call):
+    """the least memory under which call() succeeds with nothing kept from earlier calls"""
+    low, high = lib.stub_used(), 1 << 40
+    while high - low > 1 << 16:
+        mid = (low + high) // 2
+        lib.tdx_release_workspace()
+        lib.stub_limit(mid)
+        st, _ = call()
+        assert st in (tdx.TDX_OK, tdx.TDX_ERR_ALLOC)
+        low, high = (low, mid) if st == tdx.TDX_OK else (mid, high)
+    lib.tdx_release_workspace()
+    return high
+
+
+@pytest.mark.parametrize("storage,options", [
+    (tdx.TDX_F32, {}), (tdx.TDX_BF16, dict(opening_sweeps=1, opening_split=1, refine_sweeps=1)),
+    (tdx.TDX_FP8_E4M3, dict(opening_sweeps=1, opening_split=1, refine_sweeps=1))])
+def test_fp32_t_never_costs_a_call_its_memory(lib, memory, storage, options):
+    """What fits with separate passes fits with the shared pass asked for: T of the FP32 sweeps is given up."""
+    dims, R = (8208, 64, 64), 64  # (T takes less than the partials that are allocated with it)
+    X, U = buffers(memory, dims, R)
+    limit = least_limit(lib, lambda: cp_als(lib, X, dims, R, U, storage, shared_pass=0, **options))
+    lib.stub_limit(limit)
+    before = lib.stub_launches(b"k_tw_m1")
+    assert cp_als(lib, X, dims, R, U, storage, **options)[0] == tdx.TDX_OK
+    assert lib.stub_launches(b"k_tw_m1") == before
+    lib.stub_limit(limit + (1 << 30))
+    assert cp_als(lib, X, dims, R, U, storage, **options)[0] == tdx.TDX_OK
+    assert lib.stub_launches(b"k_tw_m1") > before
+
+
+def test_no_fp32_t_without_fp32_sweeps(lib, memory):
+    dims, R = (1024, 1024, 256), 64
+    X, U = buffers(memory, dims, R)
+    most = []
+    for shared in (0, 1):
+        lib.tdx_release_workspace()
+        lib.stub_most()
+        assert cp_als(lib, X, dims, R, U, tdx.TDX_BF16, shared_pass=shared)[0] == tdx.TDX_OK
+        most.append(lib.stub_most())
+    assert most[1] - most[0] <= 2 * dims[1] * dims[2] * R + (16 << 20)  # T in BF16, and partials
+
+
+def test_memory_kept_after_a_large_call(lib, memory):
+    dims, R = (1024, 4096, 4096), 64
+    X, U = buffers(memory, dims, R)
+    before, launches = lib.stub_used(), lib.stub_launches(b"k_tw_m1")
+    assert cp_als(lib, X, dims, R, U)[0] == tdx.TDX_OK
+    assert lib.stub_launches(b"k_tw_m1") > launches  # (with 4 GiB of T)
+    assert lib.stub_used() - before <= 2 << 30
+
+
 def test_idle_memory_is_freed_for_every_allocation(lib, memory):
     """A Tucker call leaves its memory idle, CP-ALS calls their plans; a CP-ALS call of another shape, a
     workspace and a training run then find theirs."""
