@@ -142,6 +142,19 @@ __device__ __forceinline__ uint2 ld_stream(const uint2 *p) {
     return uint2{t.x, t.y};
 }
 
+// ---- FP32 values as three BF16 parts (mttkrp_f32.hip, dtree_wide.hip, gram_f32.hip) -------------
+// A value below 2^-100, unless it is zero, would lose bits of its last part.  small_key orders the
+// magnitudes as unsigned integers with zero past every value, so the least key of a tile says whether
+// it holds such an entry.
+constexpr uint32_t kSmallKey = 2u * 0x0d800000u - 1u;  // of 2^-100
+__device__ __forceinline__ uint32_t small_key(float v) { return 2u * __float_as_uint(v) - 1u; }
+// Such a tile is multiplied twice, half 0 with the entries from 2^-64 up, half 1 with the others times
+// 2^64 (exact; NaN stays in half 0).
+__device__ __forceinline__ float magnitude_half(float v, int half) {
+    const bool small = fabsf(v) < 0x1p-64f;
+    return half ? (small ? v * 0x1p64f : 0.0f) : (small ? 0.0f : v);
+}
+
 // ---- device helpers ------------------------------------------------------------
 __device__ __forceinline__ uint32_t f2u(float x) { return __float_as_uint(x); }
 __device__ __forceinline__ float u2f(uint32_t u) { return __uint_as_float(u); }

@@ -10,8 +10,8 @@
 // once a sweep (k_tw_parts) in operand order and staged chunk by chunk in two buffers, 24 KB for the
 // 128 KB of X that share them, one barrier a chunk.  A tile goes from 16-byte loads of whole lines
 // through the wave's part of LDS (rows of 272 bytes) into operand order while the next one is in
-// flight, as in mttkrp_f32.hip, whose exact three-part FP32 products and whose FP32 way for tiles with
-// infinities or values near the ends of the range are used here too.  The 64-term sums enter the FP32
+// flight, as in mttkrp_f32.hip, whose exact three-part FP32 products, whose FP32 way for tiles with
+// infinities or values near the largest and whose halves for small entries are used here too.  The 64-term sums enter the FP32
 // tile of T once; a finished tile is stored as the lanes hold it (1 KB a store) and, times C, added to
 // the mode-1 partial.
 // Bound by power and HBM as the MTTKRP kernels it replaces.  1024^3 rank 64: FP32 955 us (4.8 TB/s of X
@@ -190,12 +190,25 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
             for (int u = 0; u < 8; ++u)
                 if (!in) xv[u] = uint4{0u, 0u, 0u, 0u};
         }
-        float big = 0.0f;  // largest magnitude (NaN left out)
+        bool fp32 = false, halves = false;  // (as in mttkrp_f32.hip)
         if constexpr (ST == 0) {
+            float big = 0.0f, least = __uint_as_float(0x7f800000u);  // magnitudes (NaN left out)
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(big) : "v"(xv[u].x), "v"(xv[u].y));
                 asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(big) : "v"(xv[u].z), "v"(xv[u].w));
+                asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(xv[u].x), "v"(xv[u].y));
+                asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(xv[u].z), "v"(xv[u].w));
+            }
+            fp32 = pinf || __any(big > 0x1p119f);
+            halves = __any(least < 0x1p-100f);
+            if (halves) {
+                uint32_t key = ~0u;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    key = min(key, min(min(small_key(__uint_as_float(xv[u].x)), small_key(__uint_as_float(xv[u].y))),
+                                       min(small_key(__uint_as_float(xv[u].z)), small_key(__uint_as_float(xv[u].w)))));
+                halves = __any(key < kSmallKey);
             }
         }
         // (a wave's LDS operations complete in order: no barrier between its stores and loads)
@@ -207,7 +220,7 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
         load();
         __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs
         if constexpr (ST == 0) {
-            if (pinf || __any(big > 0x1p119f || (big < 0x1p-100f && big > 0.0f))) {
+            if (fp32) {
                 // FP32 products
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
@@ -232,32 +245,61 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
                 }
                 return;
             }
+            auto split_row = [&](int rb, int ks, uint4 (&x)[3], auto value) {
+                const float *p = xs + (16 * rb + lm) * kTwLd + 32 * ks + 8 * lg;
+                tw_f4 u = *reinterpret_cast<const tw_f4 *>(p), v = *reinterpret_cast<const tw_f4 *>(p + 4);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) u[c] = value(u[c]), v[c] = value(v[c]);
+                tw_split<3>(u, v, x);
+            };
+            // s + the products, smallest terms first
+            auto products = [&](const uint4 (&x)[3], const uint4 (&p)[3], tw_f4 s) {
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[2]), tw_op(p[0]), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[0]), tw_op(p[2]), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[1]), tw_op(p[1]), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[1]), tw_op(p[0]), s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[0]), tw_op(p[1]), s, 0, 0, 0);
+                return __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[0]), tw_op(p[0]), s, 0, 0, 0);
+            };
+            if (halves) {
+#pragma unroll 1
+                for (int h = 0; h < 4; ++h) {
+                    const int ks = h & 1, half = h >> 1;
+                    uint4 x[2][3];
+#pragma unroll
+                    for (int rb = 0; rb < 2; ++rb)
+                        split_row(rb, ks, x[rb], [&](float v) { return magnitude_half(v, half); });
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        uint4 p[3];
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) p[k] = pb[((ks * 3 + k) * NB + nb) * 64 + lane];
+#pragma unroll
+                        for (int rb = 0; rb < 2; ++rb) {
+                            const tw_f4 s = products(x[rb], p, tw_f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) ac[rb][nb][v] = fmaf(s[v], half ? 0x1p-64f : 1.0f, ac[rb][nb][v]);
+                            asm volatile("" : "+v"(ac[rb][nb]));
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                return;
+            }
             tw_f4 t[2][NB];
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 uint4 x[2][3];
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb) {
-                    const float *p = xs + (16 * rb + lm) * kTwLd + 32 * ks + 8 * lg;
-                    tw_split<3>(*reinterpret_cast<const tw_f4 *>(p), *reinterpret_cast<const tw_f4 *>(p + 4), x[rb]);
-                }
+                for (int rb = 0; rb < 2; ++rb) split_row(rb, ks, x[rb], [](float v) { return v; });
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     uint4 p[3];
 #pragma unroll
                     for (int k = 0; k < 3; ++k) p[k] = pb[((ks * 3 + k) * NB + nb) * 64 + lane];
-                    // smallest terms first
 #pragma unroll
-                    for (int rb = 0; rb < 2; ++rb) {
-                        tw_f4 s = ks == 0 ? tw_f4{0.f, 0.f, 0.f, 0.f} : t[rb][nb];
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][2]), tw_op(p[0]), s, 0, 0, 0);
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][0]), tw_op(p[2]), s, 0, 0, 0);
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][1]), tw_op(p[1]), s, 0, 0, 0);
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][1]), tw_op(p[0]), s, 0, 0, 0);
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][0]), tw_op(p[1]), s, 0, 0, 0);
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tw_op(x[rb][0]), tw_op(p[0]), s, 0, 0, 0);
-                        t[rb][nb] = s;
-                    }
+                    for (int rb = 0; rb < 2; ++rb)
+                        t[rb][nb] = products(x[rb], p, ks == 0 ? tw_f4{0.f, 0.f, 0.f, 0.f} : t[rb][nb]);
                 }
             }
 #pragma unroll

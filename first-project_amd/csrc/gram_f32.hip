@@ -16,9 +16,9 @@
 //     but for their parity.
 //   * Loads along the contiguous index: along p, or, for P = 1, 4 rows of 4 columns transposed in
 //     registers.  The next step's are in flight meanwhile.
-//   * A tile with an entry above 2^60 (its products may overflow, an infinity has no parts) or a
-//     loaded vector below 2^-100 throughout (whose last part would lose bits) is read again and
-//     multiplied in FP32.
+//   * A tile with an entry above 2^60 (its products may overflow, an infinity has no parts) or below
+//     2^-100 but not zero (its last part would lose bits) is read again and multiplied in FP32 (every
+//     tile of 128^3 x 32: 94 / 90 / 96 -> 264 / 249 / 250 us for modes 0 .. 2).
 //
 // A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
 // fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock; the LDS reads of
@@ -102,9 +102,11 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
             q += wrap;
         }
     };
-    // four consecutive columns of a row: their parts to LDS; true where FP32 products are needed
+    // four consecutive columns of a row: their parts to LDS
+    float m = 0.0f;       // largest magnitude of the step (NaN left out: it stays NaN in its parts)
+    uint32_t key = ~0u;   // and least small_key
     auto put = [&](int row, int kq, float4 x) {
-        float m = 0.0f;  // largest magnitude (NaN left out: it stays NaN in its parts)
+        key = min(key, min(min(small_key(x.x), small_key(x.y)), min(small_key(x.z), small_key(x.w))));
         asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x.x), "v"(x.y));
         asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x.z), "v"(x.w));
         uint2 *d = reinterpret_cast<uint2 *>(xs + row * 8 + ((kq >> 1) ^ (((row >> 1) ^ (row >> 4)) & 7))) + (kq & 1);
@@ -117,11 +119,10 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
             x.x -= __uint_as_float(w.x << 16), x.y -= __uint_as_float(w.x & 0xffff0000u);
             x.z -= __uint_as_float(w.y << 16), x.w -= __uint_as_float(w.y & 0xffff0000u);
         }
-        return m > 0x1p60f || (m < 0x1p-100f && m > 0.0f);
     };
     auto store = [&](long k0, int u) {
         if constexpr (PC) {
-            return put((tid >> 4) + 16 * u, kq, k0 + 4 * kq < K ? xq[u] : float4{0.f, 0.f, 0.f, 0.f});
+            put((tid >> 4) + 16 * u, kq, k0 + 4 * kq < K ? xq[u] : float4{0.f, 0.f, 0.f, 0.f});
         } else {
             float v[4][4];
 #pragma unroll
@@ -130,10 +131,8 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
                 const float4 w = xq[4 * u + c];
                 v[0][c] = on ? w.x : 0.f, v[1][c] = on ? w.y : 0.f, v[2][c] = on ? w.z : 0.f, v[3][c] = on ? w.w : 0.f;
             }
-            bool f = false;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) f |= put(4 * rq + t, kq + KQ * u, float4{v[t][0], v[t][1], v[t][2], v[t][3]});
-            return f;
+            for (int t = 0; t < 4; ++t) put(4 * rq + t, kq + KQ * u, float4{v[t][0], v[t][1], v[t][2], v[t][3]});
         }
     };
     auto operand = [&](int b, int ks, int k) {
@@ -182,21 +181,43 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
             asm volatile("" : "+v"(accf[p]));  // (before the branch, as below)
         }
     };
-    // FP32 products of the tile at k0, from memory
+    // FP32 products of the tile at k0, from memory: four consecutive columns of a row a lane
+    auto odd_run = [&](long k0) {  // of the tile's first column (in scalar registers)
+        const long kd = PC ? k0 / P : 0;
+        return (long)__builtin_amdgcn_readfirstlane((int)(kd >> 32)) << 32 |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)kd);
+    };
+    auto odd_values = [&](long k0, long kd, int q, int blk) {
+        int lo = lane;
+        uint32_t pd = (uint32_t)P;
+        asm volatile("" : "+v"(lo), "+s"(pd));  // (hoisted out of the loop over steps the rows' offsets spill)
+        const long k = k0 + 16 * q + 4 * (lo >> 4), row = min((long)(16 * blk + (lo & 15)), In - 1);
+        gf_f4 v;  // (every load unconditional)
+        if constexpr (PC) {
+            const long t = k - kd * P;
+            const long d = P > 64 ? (long)(t >= P) : (long)((uint32_t)t / pd);
+            v = *reinterpret_cast<const gf_f4 *>(X + (k < K ? (t - d * P) + (kd + d) * P * In : 0) + row * P);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = X[min(k + c, K - 1) * In + row];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = k + c < K ? v[c] : 0.0f;
+        return v;
+    };
     auto full_odd = [&](auto w, long k0) {
         constexpr GfWave g = kGfWaves[decltype(w)::w];
-        for (int q = 0; q < 16; ++q) {
-            const long kk = k0 + 4 * q + lg, k = min(kk, K - 1), kd = k / P;
-            const float *p = X + (k - kd * P) + kd * P * In;
-            float v[6];
+        const long kd = odd_run(k0);
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+            gf_f4 v[6];
 #pragma unroll
-            for (int j = 0; j < g.n; ++j) {
-                v[j] = p[min((long)(16 * g.blk[j] + lm), In - 1) * P];
-                v[j] = kk < K ? v[j] : 0.0f;
-            }
+            for (int j = 0; j < g.n; ++j) v[j] = odd_values(k0, kd, q, g.blk[j]);
 #pragma unroll
-            for (int j = 0; j < 9; ++j)
-                accf[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[g.a[j]], v[g.b[j]], accf[j], 0, 0, 0);
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int j = 0; j < 9; ++j)
+                    accf[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[g.a[j]][c], v[g.b[j]][c], accf[j], 0, 0, 0);
         }
         __builtin_amdgcn_s_sleep(1);  // (the last results are in place before any branch)
     };
@@ -222,15 +243,15 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
         if (tid == 0) odd[par ^ 1] = 0;  // (read by every wave before this barrier, set after the next)
         // (a register's next load leaves as soon as it is free; past the range: clamped addresses or
         // the next range's, never consumed)
-        bool f = false;
+        m = 0.0f, key = ~0u;
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
-            f |= store(k0, u);
+            store(k0, u);
             load(u);
             __builtin_amdgcn_sched_barrier(0);
         }
         advance();
-        if (f) odd[par] = 1;
+        if (m > 0x1p60f || key < kSmallKey) odd[par] = 1;  // FP32 products are needed
         __syncthreads();
         if (b2 < b1) continue;
         if constexpr (FULL) {
@@ -239,23 +260,21 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
             continue;
         }
         if (odd[par]) {
-            // from memory, FP32 products
-            for (int q = 0; q < 16; ++q) {
-                const long kk = k0 + 4 * q + lg, k = min(kk, K - 1), kd = k / P;
-                const float *p = X + (k - kd * P) + kd * P * In;
-                auto value = [&](int blk) {
-                    const float v = p[min((long)(16 * blk + lm), In - 1) * P];
-                    return kk < K ? v : 0.0f;
-                };
-                const float v1 = value(b1), v2 = value(b2);
+            const long kd = odd_run(k0);
+#pragma unroll 1
+            for (int q = 0; q < 4; ++q) {
+                const gf_f4 v1 = odd_values(k0, kd, q, b1), v2 = odd_values(k0, kd, q, b2);
 #pragma unroll
                 for (int t = 0; t < NB; ++t)
                     if (nb - 1 - t >= b1) {
-                        const float w = value(nb - 1 - t);
-                        acc1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1, w, acc1[t], 0, 0, 0);
-                        if (t < NB / 2 && t <= wave && b2 > b1)
-                            acc2[t < NB / 2 ? t : 0] =
-                                __builtin_amdgcn_mfma_f32_16x16x4f32(v2, w, acc2[t < NB / 2 ? t : 0], 0, 0, 0);
+                        const gf_f4 w = odd_values(k0, kd, q, nb - 1 - t);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            acc1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1[c], w[c], acc1[t], 0, 0, 0);
+                            if (t < NB / 2 && t <= wave && b2 > b1)
+                                acc2[t < NB / 2 ? t : 0] =
+                                    __builtin_amdgcn_mfma_f32_16x16x4f32(v2[c], w[c], acc2[t < NB / 2 ? t : 0], 0, 0, 0);
+                        }
                     }
             }
             __builtin_amdgcn_s_sleep(1);  // (as below: the last results are in place before any branch)

@@ -17,10 +17,15 @@
 // are cut in registers as the operands are read (5.5 vector operations an element, once).
 //   * A panel column is scaled by a power of two to a largest entry in [1, 2) (undone in w), so
 //     that factors of uneven magnitude neither overflow nor lose bits in the 64-term sums.
-//   * An infinity has no such parts (inf - inf), sums of values near the largest would overflow
-//     before w scales them, and values below 2^-110 would lose bits of their last part: a tile with
-//     entries above 2^119, or a lane's entries all below 2^-100, and a chunk whose panel holds an
-//     infinity are multiplied in FP32 (v_mfma_f32_16x16x4_f32) by w p instead.  NaN stays NaN.
+//   * An infinity has no such parts (inf - inf), and sums of values near the largest would overflow
+//     before w scales them: a tile with entries above 2^119 and a chunk whose panel holds an infinity
+//     are multiplied in FP32 (v_mfma_f32_16x16x4_f32) by w p instead.  NaN stays NaN.
+//   * An entry below 2^-110 would lose bits of its last part, down to 11 of 24 at 2^-120: a tile with
+//     any entry below 2^-100 but zero is multiplied in two halves of its magnitudes (magnitude_half).
+//     The least magnitude is found with the largest; only tiles where it is below 2^-100 are looked
+//     over for what is not zero.  (Panel entries keep 2^-134 of their column's largest in the chunk.)
+//     No difference without such entries; with one entry in five such, 512^3 rank 16 92 / 98 / 107 ->
+//     163 / 192 / 185 us, rank 64 132 / 164 / 174 -> 283 / 303 / 282.
 // Errors against 64 bits, FP32 products with one long chain of sums before: 2.3e-6 -> 3.1e-7
 // (1024^3 rank 64), 8.5e-7 -> 1.5e-7 (512^3 rank 33), 4.4e-7 -> 1.1e-7 (128^3 rank 16).
 // Bound by power (1.6-1.9 GHz while the tensor streams) and HBM.  Modes 0 / 1 / 2, FP32 matrix
@@ -67,6 +72,9 @@ struct MfArgs {
 // the three parts of 8 consecutive values, packed as BF16 operands
 struct MfParts {
     uint4 p[3];
+};
+struct MfRows {
+    MfParts r[2];
 };
 __device__ __forceinline__ MfParts mf_split(const mf_f4 &a, const mf_f4 &b) {
     float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
@@ -226,11 +234,23 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                     for (int u = 0; u < 8; ++u)
                         if (!((ok >> u) & 1u)) b.x[u] = float4{0.f, 0.f, 0.f, 0.f};
                 }
-                float big = 0.0f;  // largest magnitude (NaN left out)
+                float big = 0.0f, least = __uint_as_float(0x7f800000u);  // magnitudes (NaN left out)
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(big) : "v"(b.x[u].x), "v"(b.x[u].y));
                     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(big) : "v"(b.x[u].z), "v"(b.x[u].w));
+                    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(b.x[u].x), "v"(b.x[u].y));
+                    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(b.x[u].z), "v"(b.x[u].w));
+                }
+                const bool fp32 = pinf || __any(big > 0x1p119f);
+                bool halves = __any(least < 0x1p-100f);
+                if (halves) {
+                    uint32_t key = ~0u;
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        key = min(key, min(min(small_key(b.x[u].x), small_key(b.x[u].y)),
+                                           min(small_key(b.x[u].z), small_key(b.x[u].w))));
+                    halves = __any(key < kSmallKey);
                 }
                 // (a wave's LDS operations complete in order: no barrier between its stores and loads)
                 __builtin_amdgcn_wave_barrier();
@@ -253,7 +273,7 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                 __builtin_amdgcn_wave_barrier();
                 load(b);
                 __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs
-                if (pinf || __any(big > 0x1p119f || (big < 0x1p-100f && big > 0.0f))) {
+                if (fp32) {
                     // FP32 products with w times the unscaled panel
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
@@ -274,32 +294,64 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                         }
                     return;
                 }
-                mf_f4 t[2][NB];
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    MfParts x[2];
+                auto split_rows = [&](int ks, auto value) {
+                    MfRows x;
 #pragma unroll
                     for (int rb = 0; rb < 2; ++rb) {
                         const float *xp = xs + (16 * rb + lm) * kMfLd + 32 * ks + 8 * lg;
-                        x[rb] = mf_split(*reinterpret_cast<const mf_f4 *>(xp), *reinterpret_cast<const mf_f4 *>(xp + 4));
+                        mf_f4 u = *reinterpret_cast<const mf_f4 *>(xp), v = *reinterpret_cast<const mf_f4 *>(xp + 4);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) u[c] = value(u[c]), v[c] = value(v[c]);
+                        x.r[rb] = mf_split(u, v);
                     }
+                    return x;
+                };
+                // s + the products of row block rb, smallest terms first
+                auto products = [&](const MfParts &x, const uint4 (&p)[3], mf_f4 s) {
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[2]), mf_op(p[0]), s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[0]), mf_op(p[2]), s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[1]), mf_op(p[1]), s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[1]), mf_op(p[0]), s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[0]), mf_op(p[1]), s, 0, 0, 0);
+                    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[0]), mf_op(p[0]), s, 0, 0, 0);
+                };
+                if (halves) {
+                    // (a k-step of a half at a time: arranged as below, registers spill)
+#pragma unroll 1
+                    for (int h = 0; h < 4; ++h) {
+                        const int ks = h & 1, half = h >> 1;
+                        const MfRows x = split_rows(ks, [&](float v) { return magnitude_half(v, half); });
+                        // (2^-64 is taken out of both factors, so that neither underflows)
+                        const float down = half ? 0x1p-32f : 1.0f;
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) {
+                            uint4 p[3];
+#pragma unroll
+                            for (int k = 0; k < 3; ++k) p[k] = bs[((ks * 3 + k) * NB + nb) * 64 + lane];
+                            const float ws = w[nb] * sc[nb] * down;
+#pragma unroll
+                            for (int rb = 0; rb < 2; ++rb) {
+                                const mf_f4 s = products(x.r[rb], p, mf_f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                                for (int v = 0; v < 4; ++v) acc[rb][nb][v] = fmaf(s[v] * down, ws, acc[rb][nb][v]);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                    return;
+                }
+                mf_f4 t[2][NB];
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    const MfRows x = split_rows(ks, [](float v) { return v; });
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
                         uint4 p[3];
 #pragma unroll
                         for (int k = 0; k < 3; ++k) p[k] = bs[((ks * 3 + k) * NB + nb) * 64 + lane];
-                        // smallest terms first
 #pragma unroll
-                        for (int rb = 0; rb < 2; ++rb) {
-                            mf_f4 s = ks == 0 ? mf_f4{0.f, 0.f, 0.f, 0.f} : t[rb][nb];
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[2]), mf_op(p[0]), s, 0, 0, 0);
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[0]), mf_op(p[2]), s, 0, 0, 0);
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[1]), mf_op(p[1]), s, 0, 0, 0);
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[1]), mf_op(p[0]), s, 0, 0, 0);
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[0]), mf_op(p[1]), s, 0, 0, 0);
-                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x[rb].p[0]), mf_op(p[0]), s, 0, 0, 0);
-                            t[rb][nb] = s;
-                        }
+                        for (int rb = 0; rb < 2; ++rb)
+                            t[rb][nb] = products(x.r[rb], p, ks == 0 ? mf_f4{0.f, 0.f, 0.f, 0.f} : t[rb][nb]);
                     }
                 }
 #pragma unroll
