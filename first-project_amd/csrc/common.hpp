@@ -143,6 +143,16 @@ __device__ __forceinline__ uint2 ld_stream(const uint2 *p) {
 }
 
 // ---- FP32 values as three BF16 parts (mttkrp_f32.hip, dtree_wide.hip, gram_f32.hip) -------------
+// Two values rounded to nearest even, in one register: a conversion instruction that the compiler knows
+// (inside an asm statement it is placed without regard to matrix instructions that still read or write
+// its register), opaque so that the halves taken out of it are not converted once more each.
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), b2));
+    asm("" : "+v"(w));
+    return w;
+}
 // A value below 2^-100, unless it is zero, would lose bits of its last part.  small_key orders the
 // magnitudes as unsigned integers with zero past every value, so the least key of a tile says whether
 // it holds such an entry.

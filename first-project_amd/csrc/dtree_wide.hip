@@ -57,8 +57,7 @@ __device__ __forceinline__ void tw_split(const tw_f4 &a, const tw_f4 &b, uint4 (
         uint32_t w[4];
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-            // round to nearest even (as a vector cast the compiler converted a pair twice)
-            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w[h]) : "v"(v[2 * h]), "v"(v[2 * h + 1]));
+            w[h] = bf16_pair(v[2 * h], v[2 * h + 1]);
             v[2 * h] -= __uint_as_float(w[h] << 16);
             v[2 * h + 1] -= __uint_as_float(w[h] & 0xffff0000u);
         }

@@ -112,9 +112,7 @@ __global__ __launch_bounds__(256, gf_wgs(NB)) void k_gram_f32(const float *__res
         uint2 *d = reinterpret_cast<uint2 *>(xs + row * 8 + ((kq >> 1) ^ (((row >> 1) ^ (row >> 4)) & 7))) + (kq & 1);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            uint2 w;
-            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w.x) : "v"(x.x), "v"(x.y));
-            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w.y) : "v"(x.z), "v"(x.w));
+            const uint2 w = {bf16_pair(x.x, x.y), bf16_pair(x.z, x.w)};
             d[k * NR * 16] = w;
             x.x -= __uint_as_float(w.x << 16), x.y -= __uint_as_float(w.x & 0xffff0000u);
             x.z -= __uint_as_float(w.y << 16), x.w -= __uint_as_float(w.y & 0xffff0000u);
