@@ -183,12 +183,6 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
 
     // one tile: through LDS into operand order, the next one's loads, the products
     auto step = [&](tw_f4 (&ac)[2][NB], const uint4 *pb, int fc) {
-        const bool in = fc * (32 * KSN) + EV * (lane & 15) < I0;
-        if ((fc + 1) * (32 * KSN) > I0) {
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (!in) xv[u] = uint4{0u, 0u, 0u, 0u};
-        }
         bool fp32 = false, halves = false;  // (as in mttkrp_f32.hip)
         if constexpr (ST == 0) {
             float big = 0.0f, least = __uint_as_float(0x7f800000u);  // magnitudes (NaN left out)
@@ -199,9 +193,8 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
                 asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(xv[u].x), "v"(xv[u].y));
                 asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(xv[u].z), "v"(xv[u].w));
             }
-            fp32 = pinf || __any(big > 0x1p119f);
-            halves = __any(least < 0x1p-100f);
-            if (halves) {
+            if (pinf || __any(big > 0x1p119f || least < 0x1p-100f)) {
+                fp32 = pinf || __any(big > 0x1p119f);
                 uint32_t key = ~0u;
 #pragma unroll
                 for (int u = 0; u < 8; ++u)
@@ -209,6 +202,12 @@ __global__ __launch_bounds__(64 * kTwWaves, 1) void k_tw_m1(TwArgs a) {
                                        min(small_key(__uint_as_float(xv[u].z)), small_key(__uint_as_float(xv[u].w)))));
                 halves = __any(key < kSmallKey);
             }
+        }
+        const bool in = fc * (32 * KSN) + EV * (lane & 15) < I0;
+        if ((fc + 1) * (32 * KSN) > I0) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (!in) xv[u] = uint4{0u, 0u, 0u, 0u};
         }
         // (a wave's LDS operations complete in order: no barrier between its stores and loads)
         __builtin_amdgcn_wave_barrier();

@@ -24,8 +24,9 @@
 //     any entry below 2^-100 but zero is multiplied in two halves of its magnitudes (magnitude_half).
 //     The least magnitude is found with the largest; only tiles where it is below 2^-100 are looked
 //     over for what is not zero.  (Panel entries keep 2^-134 of their column's largest in the chunk.)
-//     No difference without such entries; with one entry in five such, 512^3 rank 16 92 / 98 / 107 ->
-//     163 / 192 / 185 us, rank 64 132 / 164 / 174 -> 283 / 303 / 282.
+//     Without such entries 0.2 us of a launch of 7 (64 x 48 x 40) and nothing at 1024^3; with one entry
+//     in five such, 512^3 rank 16 92 / 98 / 107 -> 160 / 183 / 183 us, rank 64 129 / 157 / 172 -> 273 /
+//     298 / 273.
 // Errors against 64 bits, FP32 products with one long chain of sums before: 2.3e-6 -> 3.1e-7
 // (1024^3 rank 64), 8.5e-7 -> 1.5e-7 (512^3 rank 33), 4.4e-7 -> 1.1e-7 (128^3 rank 16).
 // Bound by power (1.6-1.9 GHz while the tensor streams) and HBM.  Modes 0 / 1 / 2, FP32 matrix
@@ -228,11 +229,7 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                 float w[NB];
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) w[nb] = (a.nslow > 1) ? b.wa[nb] * b.wb[nb] : b.wa[nb];
-                if (!full) {
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        if (!((ok >> u) & 1u)) b.x[u] = float4{0.f, 0.f, 0.f, 0.f};
-                }
+                // (before the entries past the extent become zero: they are entries of the tensor still)
                 float big = 0.0f, least = __uint_as_float(0x7f800000u);  // magnitudes (NaN left out)
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
@@ -241,15 +238,20 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                     asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(b.x[u].x), "v"(b.x[u].y));
                     asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(b.x[u].z), "v"(b.x[u].w));
                 }
-                const bool fp32 = pinf || __any(big > 0x1p119f);
-                bool halves = __any(least < 0x1p-100f);
-                if (halves) {
+                bool fp32 = false, halves = false;
+                if (__builtin_expect(pinf || __any(big > 0x1p119f || least < 0x1p-100f), 0)) {
+                    fp32 = pinf || __any(big > 0x1p119f);
                     uint32_t key = ~0u;
 #pragma unroll
                     for (int u = 0; u < 8; ++u)
                         key = min(key, min(min(small_key(b.x[u].x), small_key(b.x[u].y)),
                                            min(small_key(b.x[u].z), small_key(b.x[u].w))));
                     halves = __any(key < kSmallKey);
+                }
+                if (!full) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (!((ok >> u) & 1u)) b.x[u] = float4{0.f, 0.f, 0.f, 0.f};
                 }
                 // (a wave's LDS operations complete in order: no barrier between its stores and loads)
                 __builtin_amdgcn_wave_barrier();
@@ -272,7 +274,7 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                 __builtin_amdgcn_wave_barrier();
                 load(b);
                 __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs
-                if (fp32) {
+                if (__builtin_expect(fp32, 0)) {
                     // FP32 products with w times the unscaled panel
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
@@ -314,7 +316,7 @@ __device__ __forceinline__ void mf_block(const MfArgs &a, const int block) {
                     s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[0]), mf_op(p[1]), s, 0, 0, 0);
                     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf_op(x.p[0]), mf_op(p[0]), s, 0, 0, 0);
                 };
-                if (halves) {
+                if (__builtin_expect(halves, 0)) {
                     // (a k-step of a half at a time: arranged as below, registers spill)
 #pragma unroll 1
                     for (int h = 0; h < 4; ++h) {
