@@ -21,8 +21,7 @@
 //     tile of 128^3 x 32: 94 / 90 / 96 -> 264 / 249 / 250 us for modes 0 .. 2).
 //
 // A step is a chain (wait, cut, barrier, operand reads, products) and two workgroups of 128 rows
-// fill a CU: the matrix pipe is busy 38 % of 128^4 and 2.1 GHz are left of the clock; the LDS reads of
-// the operands take the most of a step.  Modes 0 .. 3 on FP32 matrix instructions before: 128^4 420 /
+// fill a CU: at 128^4 the matrix pipe is busy 44 % and LDS 24 % of the time, at 2.05 GHz.  Modes 0 .. 3 on FP32 matrix instructions before: 128^4 420 /
 // 396 / 393 / 395 -> 275 / 272 / 299 / 307 us, 252 / 244 / 249 / 250 with the pairs of 22 blocks (1.07
 // GB: 165 us at 6.5 TB/s), 64^4 32 / 25 / 25 / 25 -> 22 / 22 / 22 / 22, 256 x 128 x 128 15 / 13 -> 10 / 10;
 // errors against 64 bits 7e-9 -> 5e-9 (64^4), 2.2e-8 -> 1.1e-8 (124 x 100 x 76), 3.7e-8 -> 1.6e-8

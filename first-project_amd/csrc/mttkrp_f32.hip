@@ -29,7 +29,7 @@
 //     298 / 273.
 // Errors against 64 bits, FP32 products with one long chain of sums before: 2.3e-6 -> 3.1e-7
 // (1024^3 rank 64), 8.5e-7 -> 1.5e-7 (512^3 rank 33), 4.4e-7 -> 1.1e-7 (128^3 rank 16).
-// Bound by power (1.6-1.9 GHz while the tensor streams) and HBM.  Modes 0 / 1 / 2, FP32 matrix
+// Bound by power (1.65-1.7 GHz while the tensor streams; matrix pipe 46 %, LDS 27 %) and HBM.  Modes 0 / 1 / 2, FP32 matrix
 // instructions before: 1024^3 rank 64 1352 / 1223 / 1212 -> 1104 / 980 / 1009 us (0.66 ms is the
 // stream's time at 6.5 TB/s), rank 32 806 / 790 / 790 -> 717 / 694 / 753, rank 16 664 / 669 / 655
 // -> 621 / 658 / 669; 256^3 rank 20 20-21 -> 17-19; 640 x 72 x 1024 rank 40 89 / 89 / 55 -> 68 / 59
